@@ -10,6 +10,9 @@ BatchLauncher *make_batch_launcher_fp32() { return new BatchLauncherT<float, tru
 void step_buffers_fp32(const lb3d_params &p, const DevBufs &b, hipStream_t s)
 {
     LauncherT<float, true> L(p);
+    const Plan q = default_plan(p);
+    L.xg = q.xg;
+    if (q.fused && L.fused(b, q.tx, q.ty, q.lz, q.stage, s)) return;
     L.moments(b, s);
     L.dipole(b, s);
     L.collide(b, s);

@@ -10,6 +10,9 @@ BatchLauncher *make_batch_launcher_fp64() { return new BatchLauncherT<double, fa
 void step_buffers_fp64(const lb3d_params &p, const DevBufs &b, hipStream_t s)
 {
     LauncherT<double, false> L(p);
+    const Plan q = default_plan(p);
+    L.xg = q.xg;
+    if (q.fused && L.fused(b, q.tx, q.ty, q.lz, q.stage, s)) return;
     L.moments(b, s);
     L.dipole(b, s);
     L.collide(b, s);

@@ -62,17 +62,17 @@ const char *const KNAMES[] = {"le_neighbours", "le_faces_pc", "moments",
                               "le_faces_aux",  "dipole",      "collide", "fused"};
 enum { K_LEN = 0, K_LE6, K_MOM, K_LE8, K_DIP, K_COL, K_FUS, K_COUNT };
 
-// How a timestep is executed: the two-pass sequence (moments, [dipole],
-// collide) or, for binary lattices, the one-pass z-march kernel with a tile
-// shape (tx, ty) and a z-chunk lz.
 const char *const STAGE_NAMES[3] = {"regs", "lds", "reload"};
 
-struct Plan {
-    bool fused = false;
-    int tx = 64, ty = 4, lz = 0;
-    int stage = 1;      // plane k's populations: 0 registers, 1 LDS, 2 pulled again
-    uint32_t xg = 1;    // tiles per XCD chunk (xcd_tile): 1 plain order, 0 one run per XCD
-};
+// Tile shapes that lb3d_gpu_set_plan takes.
+static bool listed_shape(int ncomp, int tx, int ty)
+{
+    if (ncomp == 2 && tx == 16) return false;  // 16 x 16 is a shape of the ternary kernel only
+    for (auto &sh : FUSED_SHAPES)
+        if (sh[0] == tx && sh[1] == ty) return true;
+    return false;
+}
+
 
 }  // namespace
 
@@ -166,6 +166,75 @@ static int check_params(const lb3d_params *p)
 }
 
 namespace lb3d {
+// The one-pass kernel (binary, bdist 2, periodic) with a tile fitted to the
+// lattice, or the two-pass kernels.
+//
+// Which: the one-pass kernel moves 60% of the two-pass plan's bytes, but every
+// z-chunk computes 2 planes of psi more than it collides and its planes are a
+// serial chain, so it needs enough planes for all CUs.  Measured per step,
+// two-pass against one-pass with the tile below (us):
+//   FP32  64^3 24 / 26, 80^3 41 / 41, 90x100x77 54 / 50, 112^3 135 / 105,
+//         128^3 202 / 146, 200^3 757 / 555, 256^3 1592 / 1099;
+//   FP64  61x47x53 31 / 35, 64^3 44 / 45, 90x100x77 141 / 130,
+//         128^3 386 / 300, 256^3 3170 / 2390.
+// So the lines lie at 0.6 and 0.4 million sites.  Lees-Edwards stays on the two
+// passes, whose compact edge columns the one-pass plan does not have.
+//
+// Tile: 512 threads (one work-group fills a CU's registers), the shape that
+// leaves the fewest threads idle over the whole plane.  FP32 prefers whole
+// rows, with no x halo, by 10% (256^3: 256x2 1.10 ms, 128x4 1.22-1.30; 160^3:
+// 160x3 294 us, 80x6 315); FP64 planes do not fit the L2 with their halos, so
+// there the halo sites count too (256^3: 64x8 2.39 ms, 128x4 2.49, 256x2 2.62;
+// 200^3: 100x5 1.24 ms, 50x10 1.31).
+//
+// z-chunk: the work-groups run in rounds of 256 (one per CU), each lz + 2
+// planes long; the fewest planes in a row win (200^3 FP32: 240 work-groups of
+// 67 planes 555 us, 480 of 34 614).
+Plan default_plan(const lb3d_params &p)
+{
+    Plan q;
+    const bool fp64 = p.precision == LB3D_FP64;
+    const int64_t sites = (int64_t)p.nx * p.ny * p.nz;
+    if (p.ncomp != 2 || p.bdist != 2 || p.inv_fluid != 0 || p.boundary != LB3D_BC_PERIODIC) return q;
+    if (sites < (fp64 ? 400000 : 600000)) return q;
+    const int T = 512, CUS = 256;
+    double best = 0.0;
+    for (int kx = 1; kx <= p.nx; kx++) {
+        const int tx = (p.nx + kx - 1) / kx;
+        if (tx < 16 && kx > 1) break;
+        int ty = T / tx < p.ny ? T / tx : p.ny;
+        if (ty > fused2_sites(T) / (tx + 2) - 2) ty = fused2_sites(T) / (tx + 2) - 2;
+        if (ty < 1) continue;
+        const int ky = (p.ny + ty - 1) / ty;
+        ty = (p.ny + ky - 1) / ky;
+        // more than 256 sites, or the kernel would be that of a smaller work-group
+        if (tx * ty <= T / 2) continue;
+        const double nh = 2.0 * (tx + 2) + 2.0 * ty;
+        const double cost = (double)kx * ky *
+                            (fp64 ? (T + 0.2 * nh) * (1.0 + 4.0 / tx) : (kx > 1 ? 1.1 : 1.0) * T);
+        if (best == 0.0 || cost < best) {
+            best = cost;
+            q.tx = tx;
+            q.ty = ty;
+            q.fused = true;
+        }
+    }
+    if (!q.fused) return q;
+    const int64_t tiles = (int64_t)((p.nx + q.tx - 1) / q.tx) * ((p.ny + q.ty - 1) / q.ty);
+    int64_t planes = 0;
+    for (int kz = 1; kz <= p.nz; kz++) {
+        const int lz = (p.nz + kz - 1) / kz;
+        const int64_t c = (tiles * ((p.nz + lz - 1) / lz) + CUS - 1) / CUS * (lz + 2);
+        if (!planes || c < planes) {
+            planes = c;
+            q.lz = lz;
+        }
+    }
+    q.stage = 0;
+    q.xg = 32;
+    return q;
+}
+
 void reduce_sanity(const double *h, unsigned nb, int ncomp, int nx, int ny, int nz, lb3d_sanity *out)
 {
     std::memset(out, 0, sizeof *out);
@@ -332,14 +401,9 @@ int lb3d_gpu_create(const lb3d_params *p, lb3d_ctx **out)
         (e = hipMalloc((void **)&c->d_partials, (size_t)c->L->diag_blocks() * NSAN * sizeof(double))) !=
             hipSuccess)
         return cleanup(LB3D_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-    if (p->ncomp == 2 && c->L->fused_supported(32, 4, true)) {
-        // default one-pass plan where it exists; lb3d_gpu_autotune picks the measured best
-        c->plan.fused = true;
-        c->plan.tx = c->L->fused_supported(64, 4, true) ? 64 : 32;
-        c->plan.ty = 4;
-        c->plan.lz = p->nz < 64 ? p->nz : 64;
-        c->plan.xg = 0;
-    }
+    // lb3d_gpu_autotune picks the measured best
+    c->plan = default_plan(*p);
+    if (c->plan.fused && !c->L->fused_supported(c->plan.tx, c->plan.ty, c->plan.stage)) c->plan = Plan();
     c->L->xg = c->plan.xg;
     c->host_le.shear_u = p->shear_u;
     c->host_le.shear_tmp = p->shear_u;
@@ -834,6 +898,17 @@ int lb3d_gpu_autotune(lb3d_ctx *c, int32_t trial_steps, char *report, int32_t re
     Plan two;
     two.fused = false;
     cands.push_back(two);
+    // the untuned plan's tile, which is fitted to the lattice
+    const Plan fit = c->L->walls ? Plan() : default_plan(c->p);
+    if (fit.fused)
+        for (int lz : {fit.lz, (fit.lz + 1) / 2}) {
+            Plan q = fit;
+            q.lz = lz;
+            if (c->L->fused_supported(q.tx, q.ty, q.stage) && (cands.size() < 2 || lz != fit.lz)) cands.push_back(q);
+        }
+    auto name = [&](const Plan &q) {
+        return !q.fused ? "two-pass" : (listed_shape(c->p.ncomp, q.tx, q.ty) ? "fused" : "fitted");
+    };
     if (c->p.ncomp == 3) {
         const int lzs[] = {8, 16, 32, 64};
         for (int k = 0; k < N_FUSED_SHAPES; k++)
@@ -855,6 +930,7 @@ int lb3d_gpu_autotune(lb3d_ctx *c, int32_t trial_steps, char *report, int32_t re
         for (int k = 0; k < N_FUSED_SHAPES; k++)
             for (int st = 0; st < 3; st++)
                 for (int lz : lzs) {
+                    if (!listed_shape(2, FUSED_SHAPES[k][0], FUSED_SHAPES[k][1])) continue;
                     if (!c->L->fused_supported(FUSED_SHAPES[k][0], FUSED_SHAPES[k][1], st)) continue;
                     if (lz > c->p.nz && lz != 16) continue;
                     Plan q;
@@ -919,7 +995,7 @@ int lb3d_gpu_autotune(lb3d_ctx *c, int32_t trial_steps, char *report, int32_t re
         HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
         per = ms / trial_steps;
         char buf[112];
-        std::snprintf(buf, sizeof buf, "%s %dx%d lz=%d %s xg=%u %.4f ms\n", q.fused ? "fused" : "two-pass",
+        std::snprintf(buf, sizeof buf, "%s %dx%d lz=%d %s xg=%u %.4f ms\n", name(q),
                       q.fused ? q.tx : 0, q.fused ? q.ty : 0, q.fused ? q.lz : 0,
                       q.fused ? STAGE_NAMES[q.stage] : "-", q.xg, per);
         rep += buf;
@@ -946,7 +1022,7 @@ int lb3d_gpu_autotune(lb3d_ctx *c, int32_t trial_steps, char *report, int32_t re
     c->tuned = true;
     drop_graph(c);
     char buf[112];
-    std::snprintf(buf, sizeof buf, "chosen: %s %dx%d lz=%d %s xg=%u %.4f ms\n", bestp.fused ? "fused" : "two-pass",
+    std::snprintf(buf, sizeof buf, "chosen: %s %dx%d lz=%d %s xg=%u %.4f ms\n", name(bestp),
                   bestp.fused ? bestp.tx : 0, bestp.fused ? bestp.ty : 0, bestp.fused ? bestp.lz : 0,
                   bestp.fused ? STAGE_NAMES[bestp.stage] : "-", bestp.xg, best);
     rep += buf;
@@ -973,7 +1049,7 @@ int lb3d_gpu_set_plan(lb3d_ctx *c, int32_t fused, int32_t tx, int32_t ty, int32_
             return fail(LB3D_EINVAL, "the binary one-pass kernel needs bdist 2");
         if (c->p.ncomp == 3 && (fused != 3 || c->le))
             return fail(LB3D_EINVAL, "the ternary one-pass kernel is fused = 3 on periodic lattices");
-        bool ok = c->L->fused_supported(tx, ty, q.stage);
+        bool ok = listed_shape(c->p.ncomp, tx, ty) && c->L->fused_supported(tx, ty, q.stage);
         if (!ok || lz < 1) return fail(LB3D_EINVAL, "no such tile shape");
         q.tx = tx;
         q.ty = ty;

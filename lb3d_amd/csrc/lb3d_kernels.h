@@ -156,17 +156,19 @@ __device__ __forceinline__ R pull(const R *__restrict__ f, const R *__restrict__
                                   const Phys<R> &P, int c, int i, int x, int y, int z)
 {
     int xs = x - CX[i], ys = wrap1(y - CY[i], P.ny), zs = wrap1(z - CZ[i], P.nz);
-    if (LE) {
-        if (xs < 0 || xs >= P.nx) {
-            int fc = xs < 0 ? 0 : 1;
-            uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz;
-            return ld_plane(plane_of(face_pc, (uint32_t)(fc * C + c) * 19u + (uint32_t)i, plane),
-                            (uint32_t)zs * (uint32_t)P.ny + (uint32_t)ys);
-        }
-    } else {
-        xs = wrap1(xs, P.nx);
+    if constexpr (LE) {
+        const R *base = plane_of(f, (uint32_t)c * 19u + (uint32_t)i, P.ns);
+        if (CX[i] == 0) return ld_pop<NT>(base, sidx(xs, ys, zs, P.nx, P.ny));
+        // the lane whose source lies outside 0..nx-1 reads the halo plane
+        // through the same load: a selected address, not a branch, so that a
+        // site's loads stay in one block and are issued together
+        const bool out = CX[i] > 0 ? xs < 0 : xs >= P.nx;
+        const uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz;
+        const R *face = plane_of(face_pc, (uint32_t)((CX[i] > 0 ? 0 : 1) * C + c) * 19u + (uint32_t)i, plane);
+        const uint32_t q = out ? (uint32_t)zs * (uint32_t)P.ny + (uint32_t)ys : sidx(xs, ys, zs, P.nx, P.ny);
+        return ld_pop<NT>(out ? face : base, q);
     }
-    return ld_pop<NT>(plane_of(f, (uint32_t)c * 19u + (uint32_t)i, P.ns), sidx(xs, ys, zs, P.nx, P.ny));
+    return ld_pop<NT>(plane_of(f, (uint32_t)c * 19u + (uint32_t)i, P.ns), sidx(wrap1(xs, P.nx), ys, zs, P.nx, P.ny));
 }
 
 // Pull through one base pointer: element (c*19 + i)*ns + site, addressed as a
@@ -204,17 +206,16 @@ __device__ __forceinline__ R aux_at(const R *__restrict__ aux, const R *__restri
                                     const Phys<R> &P, int k, int x, int y, int z)
 {
     int ys = wrap1(y, P.ny), zs = wrap1(z, P.nz);
-    if (LE) {
-        if (x < 0 || x >= P.nx) {
-            int fc = x < 0 ? 0 : 1;
-            uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz;
-            return ld_plane(plane_of(face_aux, (uint32_t)(fc * 4 + k), plane),
-                            (uint32_t)zs * (uint32_t)P.ny + (uint32_t)ys);
-        }
-    } else {
-        x = wrap1(x, P.nx);
+    if constexpr (LE) {
+        // a selected address, not a branch (see pull)
+        const bool out = x < 0 || x >= P.nx;
+        const uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz;
+        const R *base = plane_of(aux, (uint32_t)k, P.ns);
+        const R *face = plane_of(face_aux, (uint32_t)((x < 0 ? 0 : 4) + k), plane);
+        const uint32_t q = out ? (uint32_t)zs * (uint32_t)P.ny + (uint32_t)ys : sidx(x, ys, zs, P.nx, P.ny);
+        return ld_plane(out ? face : base, q);
     }
-    return ld_plane(plane_of(aux, (uint32_t)k, P.ns), sidx(x, ys, zs, P.nx, P.ny));
+    return ld_plane(plane_of(aux, (uint32_t)k, P.ns), sidx(wrap1(x, P.nx), ys, zs, P.nx, P.ny));
 }
 
 // psi(rho) = 1 - exp(-rho) (get_psi, code/lb3d_force_shanchen.F90:334-353);
@@ -1132,53 +1133,76 @@ __global__ __launch_bounds__(256) void k_collide(Phys<R> P, const R *__restrict_
 // written to memory (Lees-Edwards halo columns read face_pc / face_aux).
 // Each population is read once by its owner; halo pulls re-read neighbours'
 // data, which adjacent tiles on the same XCD fetch at the same time.
-template <typename R, bool Dev, bool LE>
-__device__ __forceinline__ void psi_at(const Phys<R> &P, const R *__restrict__ f,
-                                       const R *__restrict__ face_pc,
-                                       const R *__restrict__ face_aux, int x, int y, int z,
-                                       R &p0, R &p1)
-{
-    if (LE && (x < 0 || x >= P.nx)) {
-        uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz;
-        int fc = x < 0 ? 0 : 1;
-        uint32_t q = (uint32_t)wrap1(z, P.nz) * (uint32_t)P.ny + (uint32_t)wrap1(y, P.ny);
-        p0 = ld_plane(plane_of(face_aux, (uint32_t)(fc * 4 + 0), plane), q);
-        p1 = ld_plane(plane_of(face_aux, (uint32_t)(fc * 4 + 1), plane), q);
-        return;
-    }
-    int xs = wrap1(x, P.nx), ys = wrap1(y, P.ny), zs = wrap1(z, P.nz);
-    R r0 = R(0), r1 = R(0);
+// The sources of one column's pulls: the 9 in-plane element offsets of
+// (x - c_x, y - c_y), index 3 (c_y + 1) + c_x + 1.  Plane and z offset of a
+// population are uniform, so a pull is a scalar base plus one of these.
+template <typename R, bool LE>
+struct PullXY {
+    uint32_t o[9];
+    uint32_t ys[3];   // Lees-Edwards: y - c_y, and whether x - 1 / x + 1 lies outside
+    bool lo, hi;
+    __device__ __forceinline__ PullXY(const Phys<R> &P, int x, int y)
+    {
+        const int xs[3] = {wrap1(x + 1, P.nx), x, wrap1(x - 1, P.nx)};
 #pragma unroll
-    for (int i = 0; i < 19; i++) {
-        r0 = r0 + pull<R, 2, LE>(f, face_pc, P, 0, i, xs, ys, zs) * R(GD[i]);
-        r1 = r1 + pull<R, 2, LE>(f, face_pc, P, 1, i, xs, ys, zs) * R(GD[i]);
+        for (int b = 0; b < 3; b++) {
+            ys[b] = (uint32_t)wrap1(y + 1 - b, P.ny);
+#pragma unroll
+            for (int a = 0; a < 3; a++) o[3 * b + a] = (uint32_t)xs[a] + (uint32_t)P.nx * ys[b];
+        }
+        lo = x == 0;
+        hi = x == P.nx - 1;
     }
-    p0 = psi_of<Dev>(r0, P.emr0[0]);
-    p1 = psi_of<Dev>(r1, P.emr0[1]);
-}
+    // population (c, i) of plane z, pulled; ns: P.ns (opaque, so that the plane
+    // offsets are added up in the scalar unit where they are used instead of
+    // held in 76 scalar registers)
+    __device__ __forceinline__ R operator()(const R *__restrict__ f, const R *__restrict__ face_pc, const Phys<R> &P,
+                                            uint32_t ns, int c, int i, const uint32_t (&zo)[3],
+                                            const int (&zs)[3]) const
+    {
+        const R *base = f + (size_t)((uint32_t)(c * 19 + i) * ns + zo[CZ[i] + 1]);
+        const uint32_t off = o[3 * (CY[i] + 1) + CX[i] + 1];
+        if constexpr (LE) {
+            if (CX[i] != 0) {  // a selected address, not a branch (see pull)
+                const bool out = CX[i] > 0 ? lo : hi;
+                const uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz;
+                const R *face = face_pc + (size_t)((uint32_t)(((CX[i] > 0 ? 0 : 2) + c) * 19 + i) * plane +
+                                                   (uint32_t)zs[CZ[i] + 1] * (uint32_t)P.ny);
+                return ld_plane(out ? face : base, out ? ys[CY[i] + 1] : off);
+            }
+        }
+        return ld_plane(base, off);
+    }
+};
 
 // SM selects where the streamed populations of plane k wait for the collide:
 // 0 registers (pulled one plane ahead), 1 an LDS stage (pulled one plane
 // ahead), 2 nowhere: the collide pulls them again, once for the moments and
 // once for the relaxation (L2 hits one plane after the psi pass read them),
 // which leaves the fewest live registers.
-template <typename R, bool Dev, bool LE, int TX, int TY, int SM>
-__global__ __launch_bounds__(TX *TY) void k_fused2(Phys<R> P, const R *__restrict__ f,
-                                                    const R *__restrict__ face_pc,
-                                                    const R *__restrict__ face_aux,
-                                                    R *__restrict__ fout, int lz, uint32_t xg)
+//
+// The tile is a run-time shape of tx columns and ty rows with tx * ty <= T and
+// (tx + 2) * (ty + 2) <= fused2_sites(T), so that it can be fitted to the
+// lattice.
+constexpr int fused2_sites(int T) { return T == 512 ? 1040 : (T == 256 ? 528 : 208); }
+template <typename R, bool Dev, bool LE, int T, int SM>
+__global__ __launch_bounds__(T) void k_fused2(Phys<R> P, const R *__restrict__ f,
+                                              const R *__restrict__ face_pc,
+                                              const R *__restrict__ face_aux,
+                                              R *__restrict__ fout, int TX, int TY, int lz, uint32_t xg)
 {
-    constexpr int T = TX * TY, LX = TX + 2, LY = TY + 2, LP = LX * LY;
-    constexpr int NH = 2 * LX + 2 * TY;  // halo positions per plane
+    constexpr int LP = fused2_sites(T);
+    const int LX = TX + 2;
+    const int NH = 2 * LX + 2 * TY;  // halo positions per plane
     // psi of the tile + halo, plane p in slot p - z0 + 1 (mod 4): the collide of
     // plane k reads planes k-1..k+1 while a thread that is done with it may
     // already fill plane k+2, so one barrier per plane suffices
-    __shared__ R ring[4][2][LP];
+    __shared__ R ring[4][2][LP + 1];
     // populations of plane k+1: in LDS, one column per thread (SM 1), or in registers (SM 0)
     __shared__ R stage[SM == 1 ? 38 : 1][SM == 1 ? T : 1];
     R nxt[2][19];
     const int tid = threadIdx.x;
-    const int lx = tid % TX, ly = tid / TX;
+    const int ly = tid / TX, lx = tid - ly * TX;
     // tile (bx, by, bz) of a gx x gy x gz grid, x fastest, placed by xcd_tile
     const uint32_t gx = ((uint32_t)P.nx + TX - 1) / TX, gy = ((uint32_t)P.ny + TY - 1) / TY;
     const uint32_t gz = ((uint32_t)P.nz + lz - 1) / (uint32_t)lz;
@@ -1186,11 +1210,13 @@ __global__ __launch_bounds__(TX *TY) void k_fused2(Phys<R> P, const R *__restric
     if (tl >= gx * gy * gz) return;  // uniform over the block
     const int x0 = (int)(tl % gx) * TX, y0 = (int)((tl / gx) % gy) * TY, z0 = (int)(tl / (gx * gy)) * lz;
     const int x = x0 + lx, y = y0 + ly;
-    const bool own = x < P.nx && y < P.ny;
+    const bool slot = ly < TY;  // the threads beyond the tile only fill halo slots
+    const bool own = slot && x < P.nx && y < P.ny;
     const int zend = min(z0 + lz, P.nz);
     if (z0 >= zend) return;  // uniform over the block
     // LDS positions this thread fills besides its own: up to NHS halo slots
-    constexpr int NHS = (NH + T - 1) / T;  // halo positions per thread
+    // (no shape has more than 2 T halo positions)
+    constexpr int NHS = 2;
     int hq[NHS], hgx[NHS], hgy[NHS];
     bool hv[NHS];
 #pragma unroll
@@ -1207,51 +1233,133 @@ __global__ __launch_bounds__(TX *TY) void k_fused2(Phys<R> P, const R *__restric
         // needed: at most one site beyond the lattice in x and y
         hv[r] = h < NH && x0 + ax <= P.nx && y0 + ay <= P.ny;
     }
-    const bool mid_needed = !own && x <= P.nx && y <= P.ny;  // an interior slot acting as halo
     const int me = (ly + 1) * LX + (lx + 1);
 
-    // psi of plane zp for the tile and halo into ring slot; the owner's
-    // streamed populations of that plane go to its stage column
-    auto fill = [&](int zp, int slot) __attribute__((always_inline)) {
-        // opaque copies of the lane coordinates: keeps the compiler from
-        // hoisting the 19 per-direction offsets out of the z loop (they
-        // would stay live in VGPRs across the collide)
-        int xo = x, yo = y;
-        asm volatile("" : "+v"(xo), "+v"(yo));
-        if (own) {
-            int zs = wrap1(zp, P.nz);
-            R r0 = R(0), r1 = R(0);
-#pragma unroll
-            for (int i = 0; i < 19; i++) {
-                R v0 = pull<R, 2, LE>(f, face_pc, P, 0, i, xo, yo, zs);
-                R v1 = pull<R, 2, LE>(f, face_pc, P, 1, i, xo, yo, zs);
-                if constexpr (SM == 1) {
-                    stage[i][tid] = v0;
-                    stage[19 + i][tid] = v1;
-                } else if constexpr (SM == 0) {
-                    nxt[0][i] = v0;
-                    nxt[1][i] = v1;
-                }
-                r0 = r0 + v0 * R(GD[i]);
-                r1 = r1 + v1 * R(GD[i]);
-            }
-            ring[slot][0][me] = psi_of<Dev>(r0, P.emr0[0]);
-            ring[slot][1][me] = psi_of<Dev>(r1, P.emr0[1]);
-        } else if (mid_needed) {
-            R p0, p1;
-            psi_at<R, Dev, LE>(P, f, face_pc, face_aux, x, y, zp, p0, p1);
-            ring[slot][0][me] = p0;
-            ring[slot][1][me] = p1;
+    // psi of plane zp for the tile and halo into ring slot; the streamed
+    // populations of the thread's own site go to its registers or stage
+    // column.  FP64 and Lees-Edwards: every thread pulls a site of the lattice
+    // (threads without one pull the wrapped or the first site), so that a
+    // plane's loads are one straight line of code; with the pulls in branches
+    // of their own the compiler waited for nearly every load by itself (FP64
+    // 128^3: 461 -> 300 us a step, 256^3: 3.58 -> 2.39 ms).  FP32 periodic
+    // (BR): the branches, and every load's address by itself; the straight
+    // line issues the loads in one burst and is slower there (256^3: 1.16
+    // against 1.10 ms, 200^3: 0.65 against 0.56 ms).
+    constexpr bool BR = sizeof(R) == 4 && !LE;
+    const bool need = slot && x <= P.nx && y <= P.ny;
+    const int xw = need && x < P.nx ? x : 0, yw = need && y < P.ny ? y : 0;
+    // a thread whose psi nobody reads writes it to a spare slot: a branch here
+    // would leave its loads unfinished on one path, and the compiler then
+    // waits for everything, the stores of the collide too, in every plane
+    const int mine = need ? me : LP;
+    auto put = [&](int slot_, int q, int gx, int gy, int zp, R p0, R p1) __attribute__((always_inline)) {
+        if (LE && (gx < 0 || gx >= P.nx)) {  // a halo column: its moments are in face_aux
+            uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz;
+            int fc = gx < 0 ? 0 : 1;
+            uint32_t t = (uint32_t)wrap1(zp, P.nz) * (uint32_t)P.ny + (uint32_t)wrap1(gy, P.ny);
+            p0 = ld_plane(plane_of(face_aux, (uint32_t)(fc * 4 + 0), plane), t);
+            p1 = ld_plane(plane_of(face_aux, (uint32_t)(fc * 4 + 1), plane), t);
         }
+        ring[slot_][0][q] = p0;
+        ring[slot_][1][q] = p1;
+    };
+    auto psi_site = [&](int rs, int q, int gx, int gy, int zp, int zc) __attribute__((always_inline)) {
+        int xs = wrap1(gx, P.nx), ys = wrap1(gy, P.ny);
+        asm volatile("" : "+v"(xs), "+v"(ys));
+        R p0 = R(0), p1 = R(0);
+#pragma unroll
+        for (int i = 0; i < 19; i++) {
+            p0 = p0 + pull<R, 2, LE>(f, face_pc, P, 0, i, xs, ys, zc) * R(GD[i]);
+            p1 = p1 + pull<R, 2, LE>(f, face_pc, P, 1, i, xs, ys, zc) * R(GD[i]);
+        }
+        put(rs, q, gx, gy, zp, psi_of<Dev>(p0, P.emr0[0]), psi_of<Dev>(p1, P.emr0[1]));
+    };
+    auto fill = [&](int zp, int rs) __attribute__((always_inline)) {
+        const int zc = wrap1(zp, P.nz);
+        if constexpr (BR) {
+            int xo = x, yo = y;
+            asm volatile("" : "+v"(xo), "+v"(yo));
+            R r0 = R(0), r1 = R(0);
+            if (own) {
+#pragma unroll
+                for (int i = 0; i < 19; i++) {
+                    R v0 = pull<R, 2, LE>(f, face_pc, P, 0, i, xo, yo, zc);
+                    R v1 = pull<R, 2, LE>(f, face_pc, P, 1, i, xo, yo, zc);
+                    if constexpr (SM == 1) {
+                        stage[i][tid] = v0;
+                        stage[19 + i][tid] = v1;
+                    } else if constexpr (SM == 0) {
+                        nxt[0][i] = v0;
+                        nxt[1][i] = v1;
+                    }
+                    r0 = r0 + v0 * R(GD[i]);
+                    r1 = r1 + v1 * R(GD[i]);
+                }
+                put(rs, me, x, y, zp, psi_of<Dev>(r0, P.emr0[0]), psi_of<Dev>(r1, P.emr0[1]));
+            } else if (need) {
+                psi_site(rs, me, x, y, zp, zc);
+            }
+#pragma unroll
+            for (int r = 0; r < NHS; r++)
+                if (hv[r]) psi_site(rs, hq[r], hgx[r], hgy[r], zp, zc);
+            return;
+        }
+        // source planes zp + 1, zp, zp - 1 of c_z = -1, 0, 1
+        const int zs[3] = {wrap1(zc + 1, P.nz), zc, wrap1(zc - 1, P.nz)};
+        const uint32_t nxy = (uint32_t)P.nx * (uint32_t)P.ny;
+        const uint32_t zo[3] = {(uint32_t)zs[0] * nxy, (uint32_t)zs[1] * nxy, (uint32_t)zs[2] * nxy};
+        uint32_t ns = P.ns;
+        asm volatile("" : "+s"(ns));
+        // FP64: opaque copies of the lane coordinates keep the column's 9
+        // offsets from staying live across the collide
+        int xo = xw, yo = yw;
+        if constexpr (sizeof(R) == 8) asm volatile("" : "+v"(xo), "+v"(yo));
+        const PullXY<R, LE> own_xy(P, xo, yo);
+        R r0 = R(0), r1 = R(0);
+#pragma unroll
+        for (int i = 0; i < 19; i++) {
+            R v0 = own_xy(f, face_pc, P, ns, 0, i, zo, zs);
+            R v1 = own_xy(f, face_pc, P, ns, 1, i, zo, zs);
+            if constexpr (SM == 1) {
+                stage[i][tid] = v0;
+                stage[19 + i][tid] = v1;
+            } else if constexpr (SM == 0) {
+                nxt[0][i] = v0;
+                nxt[1][i] = v1;
+            }
+            r0 = r0 + v0 * R(GD[i]);
+            r1 = r1 + v1 * R(GD[i]);
+        }
+        put(rs, mine, x, y, zp, psi_of<Dev>(r0, P.emr0[0]), psi_of<Dev>(r1, P.emr0[1]));
 #pragma unroll
         for (int r = 0; r < NHS; r++)
             if (hv[r]) {
-                R p0, p1;
-                int gx = hgx[r], gy = hgy[r];
-                asm volatile("" : "+v"(gx), "+v"(gy));
-                psi_at<R, Dev, LE>(P, f, face_pc, face_aux, gx, gy, zp, p0, p1);
-                ring[slot][0][hq[r]] = p0;
-                ring[slot][1][hq[r]] = p1;
+                int gx = wrap1(hgx[r], P.nx), gy = wrap1(hgy[r], P.ny);
+                // the second round (tiles with more than T halo sites) computes its offsets anew
+                if (sizeof(R) == 8 || r > 0) asm volatile("" : "+v"(gx), "+v"(gy));
+                const PullXY<R, LE> xy(P, gx, gy);
+                R q[2] = {R(0), R(0)};
+                // all loads of a group are issued before the first is used
+                // (the scheduling barriers): left alone the compiler waits for
+                // each by itself where registers are short.  FP64: one
+                // component's 19 at a time; beside the two planes in
+                // registers 38 would not fit.
+                constexpr int NC = sizeof(R) == 8 ? 1 : 2;
+#pragma unroll
+                for (int c0 = 0; c0 < 2; c0 += NC) {
+                    R v[NC][19];
+#pragma unroll
+                    for (int i = 0; i < 19; i++)
+#pragma unroll
+                        for (int c = 0; c < NC; c++) v[c][i] = xy(f, face_pc, P, ns, c0 + c, i, zo, zs);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < 19; i++)
+#pragma unroll
+                        for (int c = 0; c < NC; c++) q[c0 + c] = q[c0 + c] + v[c][i] * R(GD[i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                put(rs, hq[r], hgx[r], hgy[r], zp, psi_of<Dev>(q[0], P.emr0[0]), psi_of<Dev>(q[1], P.emr0[1]));
             }
     };
     // prologue: planes z0-1 and z0

@@ -393,45 +393,41 @@ class LauncherT : public Launcher {
         unsigned n = 2u * 2u * 19u * (unsigned)P.ny * (unsigned)P.nz;
         k_le_gather_edges<R><<<(n + BLOCK - 1) / BLOCK, BLOCK, 0, s>>>(P, (const R *)b.f[b.cur], (R *)b.edge_pc);
     }
-    // LDS of k_fused2: the population stage plus the psi ring
-    template <int TX, int TY>
-    static constexpr bool fits()
-    {
-        return (38 * TX * TY + 8 * (TX + 2) * (TY + 2)) * sizeof(R) <= 160 * 1024;
-    }
     // stage: 0 registers, 1 LDS, 2 reload (k_fused2's SM)
-    template <int TX, int TY>
-    bool fused_t(const DevBufs &b, int lz, int stage, hipStream_t s, bool launch)
+    template <int T>
+    bool fused_t(const DevBufs &b, int tx, int ty, int lz, int stage, hipStream_t s, bool launch)
     {
+        if ((tx + 2) * (ty + 2) > fused2_sites(T)) return false;
         if (stage == 1) {
-            if constexpr (!fits<TX, TY>()) {
+            // LDS of the population stage plus the psi ring
+            if constexpr ((38 * T + 8 * fused2_sites(T)) * sizeof(R) > 160 * 1024) {
                 return false;
             } else {
-                if (launch) fused_go<TX, TY, 1>(b, lz, s);
+                if (launch) fused_go<T, 1>(b, tx, ty, lz, s);
                 return true;
             }
         }
         if (stage == 0) {
-            if (launch) fused_go<TX, TY, 0>(b, lz, s);
+            if (launch) fused_go<T, 0>(b, tx, ty, lz, s);
             return true;
         }
         if (stage == 2) {
-            if (launch) fused_go<TX, TY, 2>(b, lz, s);
+            if (launch) fused_go<T, 2>(b, tx, ty, lz, s);
             return true;
         }
         return false;
     }
-    template <int TX, int TY, int SM>
-    void fused_go(const DevBufs &b, int lz, hipStream_t s)
+    template <int T, int SM>
+    void fused_go(const DevBufs &b, int tx, int ty, int lz, hipStream_t s)
     {
-        unsigned grid = xcd_round(((P.nx + TX - 1) / TX) * ((P.ny + TY - 1) / TY) * ((P.nz + lz - 1) / lz));
+        unsigned grid = xcd_round(((P.nx + tx - 1) / tx) * ((P.ny + ty - 1) / ty) * ((P.nz + lz - 1) / lz));
         const R *f = (const R *)b.f[b.cur];
         R *fo = (R *)b.f[1 - b.cur];
         if (le)
-            k_fused2<R, Dev, true, TX, TY, SM><<<grid, TX * TY, 0, s>>>(P, f, (const R *)b.face_pc,
-                                                                         (const R *)b.face_aux, fo, lz, xg);
+            k_fused2<R, Dev, true, T, SM><<<grid, T, 0, s>>>(P, f, (const R *)b.face_pc, (const R *)b.face_aux, fo,
+                                                              tx, ty, lz, xg);
         else
-            k_fused2<R, Dev, false, TX, TY, SM><<<grid, TX * TY, 0, s>>>(P, f, nullptr, nullptr, fo, lz, xg);
+            k_fused2<R, Dev, false, T, SM><<<grid, T, 0, s>>>(P, f, nullptr, nullptr, fo, tx, ty, lz, xg);
     }
     // LDS of k_fused3: its rings of moments, psi and dipoles
     template <int TX, int TY>
@@ -478,15 +474,11 @@ class LauncherT : public Launcher {
             return false;
         }
         if (C != 2 || lz < 1 || P.bdist != 2) return false;
-        if (tx == 64 && ty == 4) return fused_t<64, 4>(b, lz, st, s, launch);
-        if (tx == 32 && ty == 8) return fused_t<32, 8>(b, lz, st, s, launch);
-        if (tx == 64 && ty == 8) return fused_t<64, 8>(b, lz, st, s, launch);
-        if (tx == 32 && ty == 16) return fused_t<32, 16>(b, lz, st, s, launch);
-        if (tx == 128 && ty == 4) return fused_t<128, 4>(b, lz, st, s, launch);
-        if (tx == 32 && ty == 4) return fused_t<32, 4>(b, lz, st, s, launch);
-        if (tx == 128 && ty == 2) return fused_t<128, 2>(b, lz, st, s, launch);
-        if (tx == 256 && ty == 2) return fused_t<256, 2>(b, lz, st, s, launch);
-        return false;
+        const int t = tx * ty;
+        if (tx < 1 || ty < 1 || t > 512) return false;
+        return t > 256 ? fused_t<512>(b, tx, ty, lz, st, s, launch)
+                       : (t > 128 ? fused_t<256>(b, tx, ty, lz, st, s, launch)
+                                  : fused_t<128>(b, tx, ty, lz, st, s, launch));
     }
     bool fused(const DevBufs &b, int tx, int ty, int lz, int stage, hipStream_t s) override
     {

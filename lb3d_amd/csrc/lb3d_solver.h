@@ -30,13 +30,25 @@ struct DevBufs {
     int cur = 0;
 };
 
+// How a timestep is executed: the two-pass sequence (moments, [dipole],
+// collide) or the one-pass z-march kernel with a tile shape (tx, ty) and a
+// z-chunk lz.
+struct Plan {
+    bool fused = false;
+    int tx = 64, ty = 4, lz = 0;
+    int stage = 1;      // plane k's populations: 0 registers, 1 LDS, 2 pulled again
+    uint32_t xg = 0;    // tiles per XCD chunk (xcd_tile): 1 plain order, 0 one run per XCD
+};
+// The plan of a lattice that nobody has tuned.
+Plan default_plan(const lb3d_params &p);
+
 // One precision's kernels for one parameter set.
 class Launcher {
   public:
     virtual ~Launcher() {}
     // chunk of consecutive tiles per XCD in the stepping kernels (xcd_tile);
-    // 1 is the plain round-robin order
-    uint32_t xg = 1;
+    // 0 is one run of tiles per XCD
+    uint32_t xg = 0;
     bool walls = false;  // the lattice has rock sites (the one-pass plans are then unavailable)
     virtual void moments(const DevBufs &b, hipStream_t s) = 0;
     virtual void dipole(const DevBufs &b, hipStream_t s) = 0;
@@ -115,7 +127,7 @@ class BatchLauncher {
 };
 
 Launcher *make_launcher_fp64(const lb3d_params &p);
-// one two-pass timestep over caller-provided buffers (no allocation)
+// one timestep of the default plan over caller-provided buffers (no allocation)
 void step_buffers_fp64(const lb3d_params &p, const DevBufs &b, hipStream_t s);
 void step_buffers_fp32(const lb3d_params &p, const DevBufs &b, hipStream_t s);
 Launcher *make_launcher_fp32(const lb3d_params &p);

@@ -274,3 +274,32 @@ def test_lees_edwards_edge_columns_follow_every_state_change(precision):
     g.time_loop(12)
     got = g.populations()
     assert np.array_equal(got, want), f"after upload: max {np.abs(got - want).max()}"
+
+
+@pytest.mark.parametrize("precision,dims", [
+    (LB3D_FP32_DEV, (97, 83, 75)),      # one row of tiles, threads without a site, ragged last chunk
+    (LB3D_FP32_DEV, (601, 37, 27)),     # rows longer than a work-group, last tile narrower
+    (LB3D_FP32_DEV, (3, 501, 401)),     # rows of 3 sites
+    (LB3D_FP32_DEV, (640, 1000, 1)),    # one plane
+    (LB3D_FP64, (61, 83, 80)),
+    (LB3D_FP64, (130, 2, 1601)),        # fewer rows than a tile holds
+    (LB3D_FP64, (333, 41, 30)),
+])
+def test_untuned_one_pass_plan_equals_two_pass_bitwise(precision, dims):
+    """A lattice large enough for the one-pass kernel runs it untuned, with a
+    tile fitted to its extents; the results are the two-pass plan's."""
+    kw = dict(ncomp=2, precision=precision, g_br=0.09)
+    want = None
+    for two_pass in (True, False):
+        g = Lattice(*dims, **kw)
+        g.init_noise(5, amp=(0.02, 0.02, 0.0))
+        if two_pass:
+            g.set_plan(0)
+        g.time_loop(3)
+        names = list(g.profile_steps(1)[0])
+        assert names == (["moments", "collide"] if two_pass else ["fused"])
+        got = g.populations()
+        if want is None:
+            want = got
+        g.close()
+    assert np.array_equal(got, want), f"max {np.abs(got - want).max()}"

@@ -143,7 +143,8 @@ int lb3d_gpu_advection(lb3d_ctx *ctx);                           /* code/lb3d_ad
 int lb3d_gpu_collision(lb3d_ctx *ctx);                           /* code/lb3d_collision.F90:41-291 */
 
 /* nsteps whole timesteps nt+1 .. nt+nsteps (the body of lb3d_time_loop,
- * code/lb3d_time_loop.F90:58-92), replayed from a captured HIP graph. */
+ * code/lb3d_time_loop.F90:58-92); a long run replays them from a captured HIP
+ * graph. */
 int lb3d_gpu_run_steps(lb3d_ctx *ctx, int32_t nsteps);
 /* Timing support (not a reference routine): lb3d_gpu_run_steps between two
  * HIP events recorded on the context's stream; *ms is the elapsed time
@@ -266,7 +267,7 @@ int lb3d_gpu_step_noalloc(const lb3d_params *p, const void *f_in, void *f_out, c
  * Batched ensemble (not a reference routine: the reference runs one lattice
  * per job).  Many independent periodic lattices of uneven sizes -- parameter
  * sweeps, seeds -- advanced together: each timestep is one persistent launch
- * per phase over all lattices, replayed from a captured HIP graph.  All
+ * per phase over all lattices (long runs replay a captured HIP graph).  All
  * lattices share ncomp and precision; every other parameter is per lattice
  * (bdist 0-6, body force; no walls or invasion).
  */

@@ -3,7 +3,7 @@
 // advanced together.  All lattices live in slices of shared buffers; one
 // timestep is the moments, dipole and collide phases, each a single
 // persistent launch over a work list of (lattice, 256-site tile) items, and
-// whole steps are replayed from a captured HIP graph.  The persistent grid
+// long runs replay whole steps from a captured HIP graph.  The persistent grid
 // size is chosen by lb3d_gpu_batch_autotune.
 #include <hip/hip_runtime.h>
 
@@ -38,6 +38,8 @@ struct lb3d_batch {
     uint32_t nitems = 0;
     hipStream_t stream = nullptr;
     hipGraphExec_t graph = nullptr;
+    int graph_len = 0;       // steps of the captured graph
+    int64_t plan_steps = 0;  // steps run on the current plan (a graph is captured after GRAPH_AFTER)
     int cur = 0, nt = 0;
     unsigned nwg = 2048;     // persistent grid size, a multiple of 8
     uint32_t xg = 0;         // work items per XCD chunk (xcd_tile)
@@ -161,6 +163,7 @@ void enqueue_batch_step(lb3d_batch *b)
 
 int drop_graph(lb3d_batch *b)
 {
+    b->plan_steps = 0;
     if (b->graph) {
         (void)hipGraphExecDestroy(b->graph);
         b->graph = nullptr;
@@ -264,8 +267,9 @@ int ensure_graph(lb3d_batch *b)
     b->cur = 0;
     hipGraph_t g = nullptr;
     BTRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_batch_step(b);
-    enqueue_batch_step(b);
+    const int units = b->cm_cols ? 1 : (b->sequential ? b->nlat : (int)b->groups.size() - 1);
+    const int len = graph_steps(units * b->C);
+    for (int q = 0; q < len; q++) enqueue_batch_step(b);
     hipError_t e = hipStreamEndCapture(b->stream, &g);
     b->cur = saved;
     if (e != hipSuccess) return set_error(LB3D_EHIP, (std::string("hipStreamEndCapture: ") + hipGetErrorString(e)).c_str());
@@ -275,6 +279,7 @@ int ensure_graph(lb3d_batch *b)
         b->graph = nullptr;
         return set_error(LB3D_EHIP, (std::string("hipGraphInstantiate: ") + hipGetErrorString(e)).c_str());
     }
+    b->graph_len = len;
     return LB3D_OK;
 }
 
@@ -429,16 +434,18 @@ int lb3d_gpu_batch_run_steps(lb3d_batch *b, int32_t nsteps)
     clear_error();
     if (!b || nsteps < 0) return set_error(LB3D_EINVAL, "bad argument");
     if (nsteps == 0) return LB3D_OK;
-    int rc = ensure_graph(b);
-    if (rc) return rc;
     if (b->cm_cols && !b->aux_ok) prime_aux(b);
     int left = nsteps;
-    if (b->cur == 1) {
-        enqueue_batch_step(b);
-        left--;
+    if (b->plan_steps >= GRAPH_AFTER) {
+        if (int rc = ensure_graph(b)) return rc;
+        if (b->cur == 1) {
+            enqueue_batch_step(b);
+            left--;
+        }
+        for (; left >= b->graph_len; left -= b->graph_len) BTRY(hipGraphLaunch(b->graph, b->stream));
     }
-    for (; left >= 2; left -= 2) BTRY(hipGraphLaunch(b->graph, b->stream));
-    if (left == 1) enqueue_batch_step(b);
+    for (; left > 0; left--) enqueue_batch_step(b);
+    b->plan_steps += nsteps;
     BTRY(hipGetLastError());
     b->nt += nsteps;
     b->aux_ok = b->cm_cols != 0;
@@ -451,8 +458,8 @@ int lb3d_gpu_batch_run_steps_timed(lb3d_batch *b, int32_t nsteps, double *ms)
     if (!b || !ms || nsteps < 1) return set_error(LB3D_EINVAL, "bad argument");
     // prepared before the first event: the graph, and the moments the
     // collide-moments plan carries
-    int rc = ensure_graph(b);
-    if (rc) return rc;
+    int rc = LB3D_OK;
+    if (b->plan_steps >= GRAPH_AFTER && (rc = ensure_graph(b))) return rc;
     if (b->cm_cols && !b->aux_ok) prime_aux(b);
     hipEvent_t e[2] = {nullptr, nullptr};
     struct Ev {

@@ -87,6 +87,8 @@ struct lb3d_ctx {
     bool aux_valid = false;
     LEState host_le{};
     hipGraphExec_t graph = nullptr;
+    int graph_len = 0;     // steps of the captured graph
+    int64_t plan_steps = 0;  // steps run on the current plan (a graph is captured after GRAPH_AFTER)
     double *d_partials = nullptr;
     uint8_t *rock_dev = nullptr;  // rock mask (lattices with walls)
     size_t f_bytes = 0, aux_bytes = 0, db_bytes = 0;
@@ -128,6 +130,7 @@ static void flip(lb3d_ctx *c) { set_cur(c, 1 - c->b.cur); }
 
 static void drop_graph(lb3d_ctx *c)
 {
+    c->plan_steps = 0;
     if (c->graph) {
         (void)hipGraphExecDestroy(c->graph);
         c->graph = nullptr;
@@ -459,8 +462,9 @@ static double w_of(int i) { return i < 18 ? 1.0 / 36.0 : 1.0 / 3.0; }
 static int set_walls(lb3d_ctx *c, const uint8_t *mask)
 {
     const size_t ns = (size_t)c->p.nx * c->p.ny * c->p.nz;
-    // a captured graph holds the kernels of the old wall state
-    drop_graph(c);
+    // a captured graph holds the kernels of the old wall state (the mask
+    // itself is read from the same buffer by every replay)
+    if ((mask != nullptr) != (c->b.rock != nullptr)) drop_graph(c);
     if (!mask) {
         c->L->walls = false;
         c->b.rock = nullptr;
@@ -800,13 +804,14 @@ static int enqueue_step(lb3d_ctx *c)
 static int ensure_graph(lb3d_ctx *c)
 {
     if (c->graph) return LB3D_OK;
-    // two steps starting from cur = 0 (A -> B -> A)
+    // an even number of steps starting from cur = 0 (A -> B -> ... -> A)
+    const int len = graph_steps(c->plan.fused ? (c->le ? 4 : 1) : (c->le ? 4 : c->p.ncomp));
     int saved = c->b.cur;
     set_cur(c, 0);
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_step(c);
-    if (rc == LB3D_OK) rc = enqueue_step(c);
+    int rc = LB3D_OK;
+    for (int q = 0; q < len && rc == LB3D_OK; q++) rc = enqueue_step(c);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     set_cur(c, saved);
     if (rc) {
@@ -820,6 +825,7 @@ static int ensure_graph(lb3d_ctx *c)
         c->graph = nullptr;
         return fail(LB3D_EHIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
     }
+    c->graph_len = len;
     return LB3D_OK;
 }
 
@@ -845,15 +851,19 @@ int lb3d_gpu_run_steps(lb3d_ctx *c, int32_t nsteps)
     if (nsteps == 0) return LB3D_OK;
     int rc = sync_le_counter(c);
     if (rc) return rc;
-    if ((rc = ensure_graph(c))) return rc;
     ensure_edges(c);
     int left = nsteps;
-    if (c->b.cur == 1) {
-        if ((rc = enqueue_step(c))) return rc;
-        left--;
+    if (c->plan_steps >= GRAPH_AFTER) {
+        if ((rc = ensure_graph(c))) return rc;
+        if (c->b.cur == 1) {
+            if ((rc = enqueue_step(c))) return rc;
+            left--;
+        }
+        for (; left >= c->graph_len; left -= c->graph_len) HIP_TRY(hipGraphLaunch(c->graph, c->stream));
     }
-    for (; left >= 2; left -= 2) HIP_TRY(hipGraphLaunch(c->graph, c->stream));
-    if (left == 1 && (rc = enqueue_step(c))) return rc;
+    for (; left > 0; left--)
+        if ((rc = enqueue_step(c))) return rc;
+    c->plan_steps += nsteps;
     HIP_TRY(hipGetLastError());
     c->edges_ok = compact_edges(c);
     c->nt += nsteps;
@@ -868,7 +878,7 @@ int lb3d_gpu_run_steps_timed(lb3d_ctx *c, int32_t nsteps, double *ms)
     if (c->state != IDLE) return fail(LB3D_ESTATE, "run_steps needs a completed timestep");
     int rc = sync_le_counter(c);
     if (rc) return rc;
-    if ((rc = ensure_graph(c))) return rc;
+    if (c->plan_steps >= GRAPH_AFTER && (rc = ensure_graph(c))) return rc;
     Events ev(2);
     HIP_TRY(ev.create());
     hipEvent_t e0 = ev[0], e1 = ev[1];

@@ -42,6 +42,22 @@ struct Plan {
 // The plan of a lattice that nobody has tuned.
 Plan default_plan(const lb3d_params &p);
 
+// Steps of a captured graph, and when one is captured.  Measured per step
+// (us), plain launches against graphs of 2, 16 and 64 steps: 16^3 binary FP64
+// 10.0 against 12.3, 9.6, 9.3; 32^3 binary FP64 11.6 / 13.5, 10.8, 10.5; 32^3
+// ternary FP32 15.4 / 17.0, 14.6, 14.3; 128^3 ternary 359 / 363, 359, 358: a
+// graph launch costs about 4 us more than a kernel launch, a kernel inside it
+// about 0.4 us less, and capturing one 0.4-0.7 ms plus 10 us per kernel.  So
+// a graph holds an even number of steps of at least GRAPH_KERNELS kernels, and
+// is captured once GRAPH_AFTER steps on one plan have shown a long run.
+constexpr int GRAPH_KERNELS = 48;
+constexpr int64_t GRAPH_AFTER = 1024;
+inline int graph_steps(int kernels_per_step)
+{
+    const int k = (GRAPH_KERNELS + 2 * kernels_per_step - 1) / (2 * kernels_per_step);
+    return 2 * (k < 1 ? 1 : k);
+}
+
 // One precision's kernels for one parameter set.
 class Launcher {
   public:

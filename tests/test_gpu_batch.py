@@ -218,3 +218,22 @@ def test_batch_every_equilibrium_form_with_body_force(ncomp, precision):
             assert np.abs(plans[0].populations(k) - o.populations()).max() <= 1e-11
     for b in plans:
         b.close()
+
+
+def test_long_batch_runs_replay_a_graph_bitwise():
+    """After 1024 steps on one plan the batch replays a captured graph; the
+    lattices stay bitwise those of a batch stepped one by one."""
+    dims = [(8, 6, 6), (6, 10, 7)]
+    a, b = (Batch(dims, ncomp=3, precision=LB3D_FP32_DEV) for _ in range(2))
+    for x in (a, b):
+        for k in range(2):
+            x.init_noise(k, 5 + k, amp=(0.01, 0.01, 0.01))
+    counts = [1025, 37, 40]
+    for n in counts:
+        a.time_loop(n)
+    for _ in range(sum(counts)):
+        b.time_loop(1)
+        if b.nt % 500 == 0:
+            b.set_groups(0)  # drops the plan's graph: b stays on single launches
+    for k in range(2):
+        assert np.array_equal(a.populations(k), b.populations(k))

@@ -303,3 +303,37 @@ def test_untuned_one_pass_plan_equals_two_pass_bitwise(precision, dims):
             want = got
         g.close()
     assert np.array_equal(got, want), f"max {np.abs(got - want).max()}"
+
+
+@pytest.mark.parametrize("kw", [
+    dict(ncomp=2), dict(ncomp=3, precision=LB3D_FP32_DEV),
+    dict(ncomp=2, boundary=LB3D_BC_LEES_EDWARDS, shear_u=0.04),
+])
+def test_long_runs_replay_a_graph_bitwise(kw):
+    """A run that exceeds 1024 steps on one plan replays a captured graph;
+    odd counts before and after it, a re-initialisation and an upload keep
+    giving the states of single steps."""
+    dims = (8, 6, 6)
+    g, ref = (Lattice(*dims, **kw) for _ in range(2))
+    for L in (g, ref):
+        L.init_noise(3, amp=(0.01, 0.01, 0.01))
+        L.bc_init()
+    counts = [1025, 53, 1, 48, 102]
+    for n in counts:
+        g.time_loop(n)
+    for _ in range(sum(counts)):
+        ref.time_step()
+    assert g.nt == ref.nt == sum(counts)
+    assert np.array_equal(g.populations(), ref.populations())
+    sites = ref.download_sites()
+    for again in ("noise", "sites"):
+        for L in (g, ref):
+            if again == "noise":
+                L.init_noise(4, amp=(0.02, 0.01, 0.01))
+            else:
+                L.upload_sites(sites)
+            L.bc_init()
+        g.time_loop(99)
+        for _ in range(99):
+            ref.time_step()
+        assert np.array_equal(g.populations(), ref.populations()), again

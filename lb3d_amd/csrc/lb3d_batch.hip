@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "lb3d_kernels.h"
+#include "lb3d_readback.h"
 #include "lb3d_solver.h"
 
 using namespace lb3d;
@@ -35,6 +36,7 @@ struct lb3d_batch {
     void *f[2] = {nullptr, nullptr};
     void *aux = nullptr, *db = nullptr, *lat = nullptr, *items = nullptr;
     double *partials = nullptr;
+    DevScratch io;  // pieces of read-backs, kept for the next
     uint32_t nitems = 0;
     hipStream_t stream = nullptr;
     hipGraphExec_t graph = nullptr;
@@ -380,6 +382,7 @@ int lb3d_gpu_batch_destroy(lb3d_batch *b)
     for (void *q : {b->aux, b->aux1, b->db, b->lat, b->items, (void *)b->partials, b->cm_items, b->edge_items,
                     b->edge_sites})
         if (q) (void)hipFree(q);
+    b->io.release();
     if (b->stream) (void)hipStreamDestroy(b->stream);
     for (Launcher *l : b->L) delete l;
     delete b->B;
@@ -420,12 +423,9 @@ int lb3d_gpu_batch_get_populations(lb3d_batch *b, int32_t k, double *out)
 {
     clear_error();
     if (!b || k < 0 || k >= b->nlat || !out) return set_error(LB3D_EINVAL, "bad argument");
-    size_t bytes = (size_t)b->C * 19 * b->ns[k] * b->rs;
-    std::vector<unsigned char> h(bytes);
-    DevBufs v = view(b, k);
-    BTRY(hipMemcpyAsync(h.data(), v.f[b->cur], bytes, hipMemcpyDeviceToHost, b->stream));
-    BTRY(hipStreamSynchronize(b->stream));
-    device_layout_to_pops(b->p[k], h.data(), out);
+    const void *f = view(b, k).f[b->cur];
+    BTRY(b->rs == 4 ? fetch_populations<float>(b->io, b->stream, b->p[k], f, out)
+                    : fetch_populations<double>(b->io, b->stream, b->p[k], f, out));
     return LB3D_OK;
 }
 

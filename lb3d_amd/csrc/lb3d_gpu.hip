@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "lb3d_kernels.h"
+#include "lb3d_readback.h"
 #include "lb3d_solver.h"
 
 using namespace lb3d;
@@ -91,6 +92,8 @@ struct lb3d_ctx {
     int64_t plan_steps = 0;  // steps run on the current plan (a graph is captured after GRAPH_AFTER)
     double *d_partials = nullptr;
     uint8_t *rock_dev = nullptr;  // rock mask (lattices with walls)
+    DevScratch io;                // pieces of read-backs and uploads, kept for the next
+    uint32_t *rock_count = nullptr;  // rock sites of an upload
     size_t f_bytes = 0, aux_bytes = 0, db_bytes = 0;
     size_t aux_elems = 0;  // elements of the aux field
     Plan plan;
@@ -334,22 +337,6 @@ int aos_to_device_layout(const lb3d_params &p, const double *N, int h, int sd,
     return LB3D_OK;
 }
 
-void device_layout_to_pops(const lb3d_params &p, const unsigned char *fb, double *out)
-{
-    const int C = p.ncomp;
-    const size_t ns = (size_t)p.nx * p.ny * p.nz;
-    if (p.precision == LB3D_FP32_DEV) {
-        const float *h = (const float *)fb;
-        for (int k = 0; k < C; k++)
-            for (int i = 0; i < 19; i++) {
-                double base = (i < 18 ? 1.0 / 36.0 : 1.0 / 3.0) * rho0_of(p, k);
-                size_t off = ((size_t)k * 19 + i) * ns;
-                for (size_t q = 0; q < ns; q++) out[off + q] = base + (double)h[off + q];
-            }
-    } else {
-        std::memcpy(out, fb, (size_t)C * 19 * ns * sizeof(double));
-    }
-}
 }  // namespace lb3d
 
 extern "C" {
@@ -433,6 +420,8 @@ int lb3d_gpu_destroy(lb3d_ctx *c)
     if (c->b.le) (void)hipFree(c->b.le);
     if (c->d_partials) (void)hipFree(c->d_partials);
     if (c->rock_dev) (void)hipFree(c->rock_dev);
+    if (c->rock_count) (void)hipFree(c->rock_count);
+    c->io.release();
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c->L;
     delete c;
@@ -457,50 +446,96 @@ static bool is_dev(const lb3d_ctx *c) { return c->p.precision == LB3D_FP32_DEV; 
 static double rho0_of(const lb3d_ctx *c, int k) { return lb3d::rho0_of(c->p, k); }
 static double w_of(int i) { return i < 18 ? 1.0 / 36.0 : 1.0 / 3.0; }
 
-// Rock mask on the device (nullptr: no walls).  With walls only the two-pass
+// Walls on (the mask is in rock_dev) or off.  With walls only the two-pass
 // plan exists, so a one-pass plan falls back to it.
-static int set_walls(lb3d_ctx *c, const uint8_t *mask)
+static void set_walls(lb3d_ctx *c, bool on)
 {
-    const size_t ns = (size_t)c->p.nx * c->p.ny * c->p.nz;
     // a captured graph holds the kernels of the old wall state (the mask
     // itself is read from the same buffer by every replay)
-    if ((mask != nullptr) != (c->b.rock != nullptr)) drop_graph(c);
-    if (!mask) {
-        c->L->walls = false;
-        c->b.rock = nullptr;
-        return LB3D_OK;
-    }
-    if (!c->rock_dev) HIP_TRY(hipMalloc((void **)&c->rock_dev, ns));
-    HIP_TRY(hipMemcpyAsync(c->rock_dev, mask, ns, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    c->b.rock = c->rock_dev;
-    c->L->walls = true;
-    if (c->plan.fused) {
+    if (on != (c->b.rock != nullptr)) drop_graph(c);
+    c->L->walls = on;
+    c->b.rock = on ? c->rock_dev : nullptr;
+    if (on && c->plan.fused) {
         c->plan = Plan();
         c->L->xg = c->plan.xg;
     }
-    return LB3D_OK;
 }
+
+// Site records in pieces of whole z planes of at most REC_BYTES (or one plane).
+constexpr size_t REC_BYTES = 64u << 20;
+static RecLayout rec_layout(const lb3d_params &p, int h, int sd)
+{
+    RecLayout L;
+    L.nx = p.nx;
+    L.ny = p.ny;
+    L.nz = p.nz;
+    L.h = h;
+    L.sd = sd;
+    L.C = p.ncomp;
+    L.ns = (uint32_t)p.nx * (uint32_t)p.ny * (uint32_t)p.nz;
+    L.rock_r = p.rock_colour_r;
+    L.rock_b = p.rock_colour_b;
+    return L;
+}
+static int rec_planes(size_t plane_bytes, int total)
+{
+    const size_t k = REC_BYTES / plane_bytes;
+    return k < 1 ? 1 : (k > (size_t)total ? total : (int)k);
+}
+
+static int rebuild_aux(lb3d_ctx *c);
 
 int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, int32_t nt0)
 {
     g_err.clear();
     if (!c || !N) return fail(LB3D_EINVAL, "NULL argument");
-    std::vector<unsigned char> fb, dbb;
-    std::vector<uint8_t> rock;
-    size_t nrock = 0;
-    int rc = aos_to_device_layout(c->p, N, h, sd, fb, dbb, &rock, &nrock);
-    if (rc) return rc;
-    if (nrock && (c->p.ncomp != 2 || c->le))
-        return fail(LB3D_EINVAL, "rock sites (walls) are supported on periodic binary lattices");
-    if (nrock && c->p.inv_fluid == 12)
-        return fail(LB3D_EINVAL, "rock sites (walls) and the Zou-He boundary are not supported together");
-    if ((rc = set_walls(c, nrock ? rock.data() : nullptr))) return rc;
-    set_cur(c, 0);
-    HIP_TRY(hipMemcpyAsync(c->b.f[0], fb.data(), c->f_bytes, hipMemcpyHostToDevice, c->stream));
-    if (c->p.ncomp == 3)
-        HIP_TRY(hipMemcpyAsync(c->b.db, dbb.data(), c->db_bytes, hipMemcpyHostToDevice, c->stream));
+    const lb3d_params &p = c->p;
+    if (sd != (p.ncomp == 3 ? 79 : 49)) return fail(LB3D_EINVAL, "site_doubles must be 79 (ternary) or 49 (binary)");
+    if (h < 1) return fail(LB3D_EINVAL, "halo_extent must be >= 1");
+    const bool walls_ok = p.ncomp == 2 && !c->le && p.inv_fluid != 12;
+    // The records are converted into the buffers that do not hold the state,
+    // which becomes current only once the rock sites are known to be
+    // supported.  (Where they are not, what those buffers hold, the input of
+    // the last step, may still be asked for: its moments are kept first.)
+    int rc = LB3D_OK;
+    if (!walls_ok && (rc = rebuild_aux(c))) return rc;
+    if (!c->rock_count) HIP_TRY(hipMalloc((void **)&c->rock_count, sizeof(uint32_t)));
+    const RecLayout L = rec_layout(p, h, sd);
+    if (walls_ok && !c->rock_dev) HIP_TRY(hipMalloc((void **)&c->rock_dev, L.ns));
+    const PopBase pb = pop_base(p);
+    const int to = 1 - c->b.cur;
+    const uint32_t nxy = (uint32_t)p.nx * (uint32_t)p.ny;
+    const size_t plane = (size_t)(p.nx + 2 * h) * (size_t)(p.ny + 2 * h) * (size_t)sd;  // doubles
+    const int per = rec_planes(plane * 8, p.nz);
+    HIP_TRY(c->io.ensure((size_t)per * plane * 8));
+    const uint32_t zero = 0;
+    HIP_TRY(hipMemcpyAsync(c->rock_count, &zero, sizeof zero, hipMemcpyHostToDevice, c->stream));
+    for (int z = 0; z < p.nz; z += per) {
+        const int k = p.nz - z < per ? p.nz - z : per;
+        HIP_TRY(hipMemcpyAsync(c->io.p, N + (size_t)(z + h) * plane, (size_t)k * plane * 8, hipMemcpyHostToDevice,
+                               c->stream));
+        const uint32_t n = (uint32_t)k * nxy, nb = (n + REC_SITES - 1) / REC_SITES;
+        const size_t lds = (size_t)REC_SITES * sd * 8;
+        auto go = [&](auto r) {
+            using R = decltype(r);
+            k_put_sites<R><<<nb, 256, lds, c->stream>>>((const double *)c->io.p, (uint32_t)(z + h), L, pb,
+                                                        (uint32_t)z * nxy, n, (R *)c->b.f[to], (R *)c->dbk[to],
+                                                        walls_ok ? c->rock_dev : nullptr, c->rock_count);
+        };
+        is_dev(c) ? go(float()) : go(double());
+        HIP_TRY(hipGetLastError());
+    }
+    uint32_t nrock = 0;
+    HIP_TRY(hipMemcpyAsync(&nrock, c->rock_count, sizeof nrock, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    if (nrock && !walls_ok) {
+        c->aux_from_prev = false;  // f[1 - cur] holds the refused records
+        if (p.ncomp != 2 || c->le)
+            return fail(LB3D_EINVAL, "rock sites (walls) are supported on periodic binary lattices");
+        return fail(LB3D_EINVAL, "rock sites (walls) and the Zou-He boundary are not supported together");
+    }
+    set_walls(c, nrock != 0);
+    set_cur(c, to);
     c->nt = nt0;
     c->host_le.nt = nt0;
     c->state = IDLE;
@@ -515,8 +550,7 @@ int lb3d_gpu_init_noise(lb3d_ctx *c, uint64_t seed, const double rho_mean[3], co
 {
     g_err.clear();
     if (!c || !rho_mean || !amp) return fail(LB3D_EINVAL, "NULL argument");
-    int rc = set_walls(c, nullptr);
-    if (rc) return rc;
+    set_walls(c, false);
     set_cur(c, 0);
     c->L->init_noise(c->b, seed, rho_mean, amp, dipoles, c->stream);
     HIP_TRY(hipGetLastError());
@@ -534,10 +568,9 @@ int lb3d_gpu_get_populations(lb3d_ctx *c, double *out)
 {
     g_err.clear();
     if (!c || !out) return fail(LB3D_EINVAL, "NULL argument");
-    std::vector<unsigned char> h(c->f_bytes);
-    HIP_TRY(hipMemcpyAsync(h.data(), c->b.f[c->b.cur], c->f_bytes, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    device_layout_to_pops(c->p, h.data(), out);
+    const void *f = c->b.f[c->b.cur];
+    HIP_TRY(is_dev(c) ? fetch_populations<float>(c->io, c->stream, c->p, f, out)
+                      : fetch_populations<double>(c->io, c->stream, c->p, f, out));
     return LB3D_OK;
 }
 
@@ -564,96 +597,30 @@ int lb3d_gpu_download_sites(lb3d_ctx *c, double *N, int32_t h, int32_t sd)
     const int C = c->p.ncomp;
     if (sd != (C == 3 ? 79 : 49)) return fail(LB3D_EINVAL, "site_doubles must be 79 (ternary) or 49 (binary)");
     if (h < 1) return fail(LB3D_EINVAL, "halo_extent must be >= 1");
-    const int nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
-    const size_t ns = (size_t)nx * ny * nz;
-    std::vector<double> pops((size_t)C * 19 * ns);
-    int rc = lb3d_gpu_get_populations(c, pops.data());
-    if (rc) return rc;
-    const bool dev = is_dev(c);
-    const size_t rs = c->L->real_bytes();
-    std::vector<double> aux, db;
-    auto fetch = [&](const void *src, size_t count, std::vector<double> &dst) -> int {
-        dst.resize(count);
-        if (rs == 8) {
-            HIP_TRY(hipMemcpyAsync(dst.data(), src, count * 8, hipMemcpyDeviceToHost, c->stream));
-            HIP_TRY(hipStreamSynchronize(c->stream));
-        } else {
-            std::vector<float> t(count);
-            HIP_TRY(hipMemcpyAsync(t.data(), src, count * 4, hipMemcpyDeviceToHost, c->stream));
-            HIP_TRY(hipStreamSynchronize(c->stream));
-            for (size_t q = 0; q < count; q++) dst[q] = (double)t[q];
-        }
-        return LB3D_OK;
-    };
-    if ((rc = rebuild_aux(c))) return rc;
-    if (c->aux_valid && (rc = fetch(c->b.aux, c->aux_elems, aux))) return rc;
-    if (C == 3 && (rc = fetch(c->b.db, 3 * ns, db))) return rc;
-    std::vector<uint8_t> rock;
-    if (c->b.rock) {
-        rock.resize(ns);
-        HIP_TRY(hipMemcpyAsync(rock.data(), c->b.rock, ns, hipMemcpyDeviceToHost, c->stream));
+    if (int rc = rebuild_aux(c)) return rc;
+    const RecLayout L = rec_layout(c->p, h, sd);
+    const PopBase pb = pop_base(c->p);
+    const int lz = c->p.nz + 2 * h;
+    const size_t recs = (size_t)(c->p.nx + 2 * h) * (size_t)(c->p.ny + 2 * h), plane = recs * (size_t)sd;
+    const int per = rec_planes(plane * 8, lz);
+    HIP_TRY(c->io.ensure((size_t)per * plane * 8));
+    for (int z = 0; z < lz; z += per) {
+        const int k = lz - z < per ? lz - z : per;
+        const uint32_t n = (uint32_t)(recs * (size_t)k), nb = (n + REC_SITES - 1) / REC_SITES;
+        const size_t lds = (size_t)REC_SITES * sd * 8;
+        auto go = [&](auto r) {
+            using R = decltype(r);
+            k_get_sites<R><<<nb, 256, lds, c->stream>>>(
+                (const R *)c->b.f[c->b.cur], c->aux_valid ? (const R *)c->b.aux : nullptr, (const R *)c->b.db,
+                c->b.rock, pb, rho0_of(c, 0), rho0_of(c, 1), rho0_of(c, 2), L, (uint32_t)(recs * (size_t)z), n,
+                (double *)c->io.p);
+        };
+        is_dev(c) ? go(float()) : go(double());
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipMemcpyAsync(N + (size_t)z * plane, c->io.p, (size_t)k * plane * 8, hipMemcpyDeviceToHost,
+                               c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
     }
-    const size_t lx = nx + 2 * h, ly = ny + 2 * h, lz = nz + 2 * h;
-    const int rock_off = C == 3 ? 78 : 48;
-    auto rec = [&](size_t x, size_t y, size_t z) { return N + (x + lx * (y + ly * z)) * sd; };
-    for (int z = 0; z < nz; z++)
-        for (int y = 0; y < ny; y++)
-            for (int x = 0; x < nx; x++) {
-                double *S = rec(x + h, y + h, z + h);
-                size_t s = (size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * z);
-                std::memset(S, 0, sizeof(double) * sd);
-                for (int k = 0; k < C; k++) {
-                    double rho = 0.0, m[3] = {0.0, 0.0, 0.0};
-                    for (int i = 0; i < 19; i++) {
-                        double v = pops[((size_t)k * 19 + i) * ns + s];
-                        S[24 * k + i] = v;
-                        double ng = v * (double)host::GD[i];
-                        rho = rho + ng;
-                        m[0] = m[0] + ng * (double)host::CX[i];
-                        m[1] = m[1] + ng * (double)host::CY[i];
-                        m[2] = m[2] + ng * (double)host::CZ[i];
-                    }
-                    if (c->aux_valid) {
-                        double r = aux[(size_t)(C + k) * ns + s];
-                        rho = dev ? rho0_of(c, k) + r : r;
-                    }
-                    S[24 * k + 19] = rho;
-                    for (int a = 0; a < 3; a++) S[24 * k + 20 + a] = m[a];
-                }
-                if (C == 3)
-                    for (int a = 0; a < 3; a++) {
-                        S[72 + a] = c->aux_valid ? aux[aux3_vec_off(ns) + 4 * s + 1 + a] : 0.0;
-                        S[75 + a] = db[(size_t)a * ns + s];
-                    }
-                S[rock_off] = 0.0;
-                if (!rock.empty() && rock[s]) {
-                    // rock sites with the colours lbe_init_rock_colour gives them
-                    S[rock_off] = 1.0;
-                    if (c->p.rock_colour_r > 0) S[23] = c->p.rock_colour_r;
-                    if (c->p.rock_colour_b > 0) S[24 + 23] = c->p.rock_colour_b;
-                }
-            }
-    // halo: periodic images of the interior (x, then y over full x, then z)
-    for (size_t z = h; z < (size_t)nz + h; z++)
-        for (size_t y = h; y < (size_t)ny + h; y++)
-            for (int k = 1; k <= h; k++) {
-                std::memcpy(rec(h - k, y, z), rec(nx + h - k, y, z), sizeof(double) * sd);
-                std::memcpy(rec(nx + h - 1 + k, y, z), rec(h - 1 + k, y, z), sizeof(double) * sd);
-            }
-    for (size_t z = h; z < (size_t)nz + h; z++)
-        for (int k = 1; k <= h; k++)
-            for (size_t x = 0; x < lx; x++) {
-                std::memcpy(rec(x, h - k, z), rec(x, ny + h - k, z), sizeof(double) * sd);
-                std::memcpy(rec(x, ny + h - 1 + k, z), rec(x, h - 1 + k, z), sizeof(double) * sd);
-            }
-    for (int k = 1; k <= h; k++)
-        for (size_t y = 0; y < ly; y++)
-            for (size_t x = 0; x < lx; x++) {
-                std::memcpy(rec(x, y, h - k), rec(x, y, nz + h - k), sizeof(double) * sd);
-                std::memcpy(rec(x, y, nz + h - 1 + k), rec(x, y, h - 1 + k), sizeof(double) * sd);
-            }
-    (void)lz;
     return LB3D_OK;
 }
 
@@ -1084,29 +1051,15 @@ int lb3d_gpu_get_density(lb3d_ctx *c, double *out)
 {
     g_err.clear();
     if (!c || !out) return fail(LB3D_EINVAL, "NULL argument");
-    const int C = c->p.ncomp;
-    const size_t ns = (size_t)c->p.nx * c->p.ny * c->p.nz;
-    // one component plane at a time keeps the host buffer small
-    std::vector<double> plane(ns);
-    std::vector<float> planef(is_dev(c) ? ns : 0);
-    const size_t rs = c->L->real_bytes();
-    for (int k = 0; k < C; k++) {
-        double *rho = out + (size_t)k * ns;
-        for (size_t s = 0; s < ns; s++) rho[s] = 0.0;
-        for (int i = 0; i < 19; i++) {
-            const char *src = (const char *)c->b.f[c->b.cur] + ((size_t)k * 19 + i) * ns * rs;
-            if (is_dev(c)) {
-                HIP_TRY(hipMemcpyAsync(planef.data(), src, ns * 4, hipMemcpyDeviceToHost, c->stream));
-                HIP_TRY(hipStreamSynchronize(c->stream));
-                double base = w_of(i) * rho0_of(c, k);
-                for (size_t s = 0; s < ns; s++) rho[s] = rho[s] + (base + (double)planef[s]) * (double)host::GD[i];
-            } else {
-                HIP_TRY(hipMemcpyAsync(plane.data(), src, ns * 8, hipMemcpyDeviceToHost, c->stream));
-                HIP_TRY(hipStreamSynchronize(c->stream));
-                for (size_t s = 0; s < ns; s++) rho[s] = rho[s] + plane[s] * (double)host::GD[i];
-            }
-        }
-    }
+    const uint32_t ns = (uint32_t)c->p.nx * (uint32_t)c->p.ny * (uint32_t)c->p.nz;
+    const PopBase pb = pop_base(c->p);
+    const void *f = c->b.f[c->b.cur];
+    HIP_TRY(fetch_f64(c->io, c->stream, out, (uint64_t)c->p.ncomp * ns, [&](uint32_t q, uint32_t m, double *o) {
+        if (is_dev(c))
+            k_get_density<float><<<(m + 255) / 256, 256, 0, c->stream>>>((const float *)f, pb, ns, q, m, o);
+        else
+            k_get_density<double><<<(m + 255) / 256, 256, 0, c->stream>>>((const double *)f, pb, ns, q, m, o);
+    }));
     return LB3D_OK;
 }
 
@@ -1114,35 +1067,15 @@ int lb3d_gpu_get_momentum(lb3d_ctx *c, double *out)
 {
     g_err.clear();
     if (!c || !out) return fail(LB3D_EINVAL, "NULL argument");
-    const int C = c->p.ncomp;
-    const size_t ns = (size_t)c->p.nx * c->p.ny * c->p.nz;
-    std::vector<double> plane(ns);
-    std::vector<float> planef(is_dev(c) ? ns : 0);
-    const size_t rs = c->L->real_bytes();
-    for (int k = 0; k < C; k++) {
-        double *P = out + (size_t)k * 3 * ns;
-        for (size_t s = 0; s < 3 * ns; s++) P[s] = 0.0;
-        for (int i = 0; i < 19; i++) {
-            const char *src = (const char *)c->b.f[c->b.cur] + ((size_t)k * 19 + i) * ns * rs;
-            if (is_dev(c)) {
-                HIP_TRY(hipMemcpyAsync(planef.data(), src, ns * 4, hipMemcpyDeviceToHost, c->stream));
-                HIP_TRY(hipStreamSynchronize(c->stream));
-                double base = w_of(i) * rho0_of(c, k);
-                for (size_t s = 0; s < ns; s++) plane[s] = base + (double)planef[s];
-            } else {
-                HIP_TRY(hipMemcpyAsync(plane.data(), src, ns * 8, hipMemcpyDeviceToHost, c->stream));
-                HIP_TRY(hipStreamSynchronize(c->stream));
-            }
-            // P += g_i n_i c_i, i ascending (lb3d_update_velocity)
-            const double g = (double)host::GD[i];
-            const int cv[3] = {host::CX[i], host::CY[i], host::CZ[i]};
-            for (int a = 0; a < 3; a++) {
-                if (cv[a] == 0) continue;
-                double *Pa = P + (size_t)a * ns;
-                for (size_t s = 0; s < ns; s++) Pa[s] = Pa[s] + (plane[s] * g) * (double)cv[a];
-            }
-        }
-    }
+    const uint32_t ns = (uint32_t)c->p.nx * (uint32_t)c->p.ny * (uint32_t)c->p.nz;
+    const PopBase pb = pop_base(c->p);
+    const void *f = c->b.f[c->b.cur];
+    HIP_TRY(fetch_f64(c->io, c->stream, out, (uint64_t)c->p.ncomp * 3u * ns, [&](uint32_t q, uint32_t m, double *o) {
+        if (is_dev(c))
+            k_get_momentum<float><<<(m + 255) / 256, 256, 0, c->stream>>>((const float *)f, pb, ns, q, m, o);
+        else
+            k_get_momentum<double><<<(m + 255) / 256, 256, 0, c->stream>>>((const double *)f, pb, ns, q, m, o);
+    }));
     return LB3D_OK;
 }
 

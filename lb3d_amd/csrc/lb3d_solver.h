@@ -159,8 +159,6 @@ void clear_error();
 int aos_to_device_layout(const lb3d_params &p, const double *whole_N, int halo, int site_doubles,
                          std::vector<unsigned char> &f_bytes, std::vector<unsigned char> &db_bytes,
                          std::vector<uint8_t> *rock = nullptr, size_t *nrock = nullptr);
-// The inverse for the populations: device bytes -> FP64 populations.
-void device_layout_to_pops(const lb3d_params &p, const unsigned char *f_bytes, double *out);
 double rho0_of(const lb3d_params &p, int c);
 
 // Parameters in the kernels' working type.

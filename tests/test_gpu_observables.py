@@ -111,3 +111,79 @@ def test_full_sanity_ties_keep_the_last_site(precision):
     assert s["fluid_sites"] == 720 and s["fast_sites"] == 0
     assert (s["max_pos"][:2] == [12, 10, 6]).all()
     assert (s["max_pos"][2] == 0).all()
+
+
+@pytest.mark.parametrize("precision", [LB3D_FP64, LB3D_FP32_DEV])
+@pytest.mark.parametrize("ncomp,dims,halo", [
+    (2, (5, 3, 2), 1),          # fewer records than a block holds
+    (3, (7, 9, 5), 3),          # a halo wider than one site
+    (2, (2, 1, 1), 4),          # a halo wider than the lattice
+    (2, (131, 130, 129), 1),    # several pieces of densities and of records
+    (3, (57, 61, 66), 1),
+])
+def test_device_conversions_equal_the_host_sums_bitwise(precision, ncomp, dims, halo):
+    """Uploads, downloads, densities and momenta are converted on the device in
+    the order of a host conversion: bitwise the numpy values."""
+    nx, ny, nz = dims
+    sd = 79 if ncomp == 3 else 49
+    r = np.random.default_rng(7)
+    N = np.full((nz + 2 * halo, ny + 2 * halo, nx + 2 * halo, sd), np.nan)  # the halo is not read
+    I = N[halo:-halo, halo:-halo, halo:-halo]
+    I[...] = 0.0
+    for c in range(ncomp):
+        I[..., 24 * c:24 * c + 19] = r.random((nz, ny, nx, 19)) / 20
+    if ncomp == 3:
+        I[..., 75:78] = r.random((nz, ny, nx, 3)) - 0.5
+    w = np.array([1.0 / 36.0] * 18 + [1.0 / 3.0]) * 0.7
+    g = Lattice(nx, ny, nz, ncomp=ncomp, precision=precision)
+    for _ in range(2):  # the second upload lands in the other buffer
+        g.upload_sites(N, halo_extent=halo, nt0=3)
+    assert g.nt == 3
+    want = np.stack([np.moveaxis(I[..., 24 * c:24 * c + 19], -1, 0) for c in range(ncomp)])
+    if precision == LB3D_FP32_DEV:
+        ww = w[None, :, None, None, None]
+        want = ww + (want - ww).astype(np.float32).astype(np.float64)
+    pops = g.populations()
+    assert np.array_equal(pops, want)
+    rho = np.zeros((ncomp, nz, ny, nx))
+    mom = np.zeros((ncomp, 3, nz, ny, nx))
+    for i in range(19):
+        rho = rho + pops[:, i] * G[i]
+        for a, cv in enumerate((CX, CY, CZ)):
+            if cv[i]:
+                mom[:, a] = mom[:, a] + (pops[:, i] * G[i]) * float(cv[i])
+    assert np.array_equal(g.density(), rho)
+    assert np.array_equal(g.momentum(), mom)
+    J = np.zeros((nz, ny, nx, sd))
+    for c in range(ncomp):
+        J[..., 24 * c:24 * c + 19] = np.moveaxis(pops[c], 0, -1)
+        J[..., 24 * c + 19] = rho[c]
+        J[..., 24 * c + 20:24 * c + 23] = np.moveaxis(mom[c], 0, -1)
+    if ncomp == 3:
+        db = I[..., 75:78]
+        J[..., 75:78] = db if precision == LB3D_FP64 else db.astype(np.float32)
+    pad = ((halo, halo),) * 3 + ((0, 0),)
+    assert np.array_equal(g.download_sites(halo_extent=halo), np.pad(J, pad, mode="wrap"))
+
+
+def test_refused_rock_sites_leave_the_state():
+    """Records with rock sites are refused on a ternary lattice; state, step
+    counter and the moments of the last advection stay."""
+    g = Lattice(6, 5, 4, ncomp=3)
+    g.init_noise(1, amp=(0.01, 0.01, 0.01))
+    g.set_plan(3, 32, 4, 4)  # one-pass: the moments are rebuilt when asked for
+    g.time_loop(2)
+    before = g.download_sites()
+    g2 = Lattice(6, 5, 4, ncomp=3)
+    g2.init_noise(1, amp=(0.01, 0.01, 0.01))
+    g2.set_plan(3, 32, 4, 4)
+    g2.time_loop(2)
+    bad = before.copy()
+    bad[2, 2, 2, 78] = 1.0
+    with pytest.raises(LB3DError):
+        g2.upload_sites(bad)
+    assert g2.nt == 2
+    assert np.array_equal(g2.download_sites(), before)
+    g.time_loop(1)
+    g2.time_loop(1)
+    assert np.array_equal(g.populations(), g2.populations())

@@ -183,20 +183,36 @@ __device__ __forceinline__ R pull_flat(const R *__restrict__ f, const Phys<R> &P
     return ld_plane(f, ((uint32_t)c * 19u + (uint32_t)i) * P.ns + sidx(xs, ys, zs, P.nx, P.ny));
 }
 
+// The rock neighbours of a site: bit i is set where x + c_i is rock, bit 18
+// where the site itself is.
+template <typename R>
+__device__ __forceinline__ uint32_t rock_bits(const uint8_t *__restrict__ rock, const Phys<R> &P, int x, int y, int z)
+{
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < 19; i++) {
+        const uint32_t q = sidx(wrap1(x + CX[i], P.nx), wrap1(y + CY[i], P.ny), wrap1(z + CZ[i], P.nz), P.nx, P.ny);
+        m |= (rock[q] != 0 ? 1u : 0u) << i;
+    }
+    return m;
+}
+
 // Pull with walls (periodic binary lattices with rock sites): a rock site
 // keeps its own populations (code/lb3d_advection.F90:126), and a fluid site
 // whose source x - c_i is rock takes its own n_bounce(i) instead, the
-// half-way bounce-back of code/lb3d_bc_bounce.F90:53-90.
+// half-way bounce-back of code/lb3d_bc_bounce.F90:53-90.  The cases select an
+// index, not a branch: with a branch per direction each of the 76 loads of a
+// site waited for its own rock flag (48x40x56 FP64: moments and collide
+// 18 + 43 us a step).
 template <typename R, int C>
-__device__ __forceinline__ R pull_rock(const R *__restrict__ f, const uint8_t *__restrict__ rock,
-                                       const Phys<R> &P, int c, int i, int x, int y, int z, bool self_rock)
+__device__ __forceinline__ R pull_rock(const R *__restrict__ f, uint32_t bits, const Phys<R> &P, int c, int i, int x,
+                                       int y, int z)
 {
-    const uint32_t s = sidx(x, y, z, P.nx, P.ny);
-    if (self_rock) return ld_plane(plane_of(f, (uint32_t)c * 19u + (uint32_t)i, P.ns), s);
-    int xs = wrap1(x - CX[i], P.nx), ys = wrap1(y - CY[i], P.ny), zs = wrap1(z - CZ[i], P.nz);
-    uint32_t q = sidx(xs, ys, zs, P.nx, P.ny);
-    if (rock[q]) return ld_plane(plane_of(f, (uint32_t)c * 19u + (uint32_t)BOUNCE[i], P.ns), s);
-    return ld_plane(plane_of(f, (uint32_t)c * 19u + (uint32_t)i, P.ns), q);
+    const bool self = (bits >> 18) & 1u, src = (bits >> BOUNCE[i]) & 1u;  // x - c_i = x + c_bounce(i)
+    const uint32_t q = sidx(wrap1(x - CX[i], P.nx), wrap1(y - CY[i], P.ny), wrap1(z - CZ[i], P.nz), P.nx, P.ny);
+    const uint32_t own = sidx(x, y, z, P.nx, P.ny);
+    const uint32_t k = (uint32_t)c * 19u + (!self && src ? (uint32_t)BOUNCE[i] : (uint32_t)i);
+    return f[k * P.ns + (self || src ? own : q)];
 }
 
 // Value k of the aux field at the neighbour (x+dx, y+dy, z+dz); for LE the
@@ -438,8 +454,8 @@ __device__ __forceinline__ void moments_core(const Phys<R> &P, const R *__restri
             return;
         }
     }
-    bool self_rock = false;
-    if constexpr (Rock) self_rock = rock[sidx(x, y, z, P.nx, P.ny)] != 0;
+    uint32_t bits = 0;
+    if constexpr (Rock) bits = rock_bits(rock, P, x, y, z);
 #pragma unroll
     for (int ii = 0; ii < 19; ii++) {
         const int i = dir_at<Dev && C == 3>(ii);
@@ -447,7 +463,7 @@ __device__ __forceinline__ void moments_core(const Phys<R> &P, const R *__restri
         for (int c = 0; c < C; c++) {
             R v;
             if constexpr (Rock)
-                v = pull_rock<R, C>(f, rock, P, c, i, x, y, z, self_rock);
+                v = pull_rock<R, C>(f, bits, P, c, i, x, y, z);
             else if constexpr (Flat)
                 v = pull_flat<R, C>(f, P, c, i, x, y, z);
             else
@@ -480,9 +496,16 @@ __device__ __forceinline__ void moments_site(const Phys<R> &P, const R *__restri
         ((V4<R> *)aux)[s] = V4<R>{psi_of<Dev>(rho[0], P.emr0[0]), psi_of<Dev>(rho[1], P.emr0[1]),
                                   psi_of<Dev>(rho[2], P.emr0[2]), rho[2]};
     } else {
+        // a rock site's psi is that of its density and rock colour, which is
+        // how the fluid next to it sees it (sc_forces_wall)
+        bool self_rock = false;
+        if constexpr (Rock) self_rock = rock[s] != 0;
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            st_plane(aux + (size_t)c * P.ns, s, psi_of<Dev>(rho[c], P.emr0[c]));
+            R r = rho[c];
+            if constexpr (Rock)
+                if (self_rock) r = r + P.rock_col[c];
+            st_plane(aux + (size_t)c * P.ns, s, psi_of<Dev>(r, P.emr0[c]));
             st_plane(aux + (size_t)(C + c) * P.ns, s, rho[c]);
         }
     }
@@ -716,34 +739,25 @@ __device__ __forceinline__ void sc_forces3(const Phys<R> &P, const R (&dbx)[3], 
 // psi values are used whole (FP32 form: psi0 + deviation), since the wall
 // and fluid sums no longer run over all 18 directions.
 template <typename R, bool Dev>
-__device__ __forceinline__ void sc_forces_wall(const Phys<R> &P, const R *__restrict__ aux,
-                                               const uint8_t *__restrict__ rock, int x, int y, int z,
-                                               uint32_t s, R F[2][3])
+__device__ __forceinline__ void sc_forces_wall(const Phys<R> &P, const R *__restrict__ aux, uint32_t bits, int x,
+                                               int y, int z, uint32_t s, R F[2][3])
 {
     R frb[3] = {R(0), R(0), R(0)}, fbr[3] = {R(0), R(0), R(0)};
     R fwr[3] = {R(0), R(0), R(0)}, fwb[3] = {R(0), R(0), R(0)};
 #pragma unroll
     for (int i = 0; i < 18; i++) {
-        int xa = wrap1(x + CX[i], P.nx), ya = wrap1(y + CY[i], P.ny), za = wrap1(z + CZ[i], P.nz);
-        uint32_t q = sidx(xa, ya, za, P.nx, P.ny);
-        R pr, pb;
-        const bool wall = rock[q] != 0;
-        if (wall) {
-            pr = psi_of<Dev>(ld_plane(plane_of(aux, 2u, P.ns), q) + P.rock_col[0], P.emr0[0]);
-            pb = psi_of<Dev>(ld_plane(plane_of(aux, 3u, P.ns), q) + P.rock_col[1], P.emr0[1]);
-        } else {
-            pr = ld_plane(aux, q);
-            pb = ld_plane(plane_of(aux, 1u, P.ns), q);
-        }
+        R pr = aux_at<R, false>(aux, nullptr, P, 0, x + CX[i], y + CY[i], z + CZ[i]);
+        R pb = aux_at<R, false>(aux, nullptr, P, 1, x + CX[i], y + CY[i], z + CZ[i]);
         if constexpr (Dev) {
             pr = P.psi0[0] + pr;
             pb = P.psi0[1] + pb;
         }
-        R green_r = pb * R(GD[i]), green_b = pr * R(GD[i]);
-        R *sr = wall ? fwb : frb, *sb = wall ? fwr : fbr;
-        if (CX[i] != 0) { sr[0] = sr[0] + green_r * R(CX[i]); sb[0] = sb[0] + green_b * R(CX[i]); }
-        if (CY[i] != 0) { sr[1] = sr[1] + green_r * R(CY[i]); sb[1] = sb[1] + green_b * R(CY[i]); }
-        if (CZ[i] != 0) { sr[2] = sr[2] + green_r * R(CZ[i]); sb[2] = sb[2] + green_b * R(CZ[i]); }
+        const bool wall = (bits >> i) & 1u;
+        const R gr = pb * R(GD[i]), gb = pr * R(GD[i]);
+        const R fr = wall ? R(0) : gr, fb = wall ? R(0) : gb, wr = wall ? gr : R(0), wb = wall ? gb : R(0);
+        if (CX[i] != 0) { frb[0] = frb[0] + fr * R(CX[i]); fbr[0] = fbr[0] + fb * R(CX[i]); fwb[0] = fwb[0] + wr * R(CX[i]); fwr[0] = fwr[0] + wb * R(CX[i]); }
+        if (CY[i] != 0) { frb[1] = frb[1] + fr * R(CY[i]); fbr[1] = fbr[1] + fb * R(CY[i]); fwb[1] = fwb[1] + wr * R(CY[i]); fwr[1] = fwr[1] + wb * R(CY[i]); }
+        if (CZ[i] != 0) { frb[2] = frb[2] + fr * R(CZ[i]); fbr[2] = fbr[2] + fb * R(CZ[i]); fwb[2] = fwb[2] + wr * R(CZ[i]); fwr[2] = fwr[2] + wb * R(CZ[i]); }
     }
     R psr = ld_plane(aux, s), psb = ld_plane(plane_of(aux, 1u, P.ns), s);
     if constexpr (Dev) {
@@ -840,7 +854,7 @@ __global__ __launch_bounds__(256) void k_forces(Phys<R> P, const R *__restrict__
 #pragma unroll
             for (int c = 0; c < C; c++) F[c][0] = F[c][1] = F[c][2] = R(0);
         } else {
-            sc_forces_wall<R, Dev>(P, aux, rock, x, y, z, s, F);
+            sc_forces_wall<R, Dev>(P, aux, rock_bits(rock, P, x, y, z), x, y, z, s, F);
         }
     } else {
         sc_forces<R, Dev, C, false>(P, aux, nullptr, db, x, y, z, s, F);
@@ -1046,18 +1060,18 @@ __device__ __forceinline__ void collide_site(const Phys<R> &P, const R *__restri
     R F[C][3];
     if constexpr (Rock) {
         static_assert(C == 2 && !LE, "walls: periodic binary lattices");
-        const bool self_rock = rock[s] != 0;
+        const uint32_t bits = rock_bits(rock, P, x, y, z);
+        sc_forces_wall<R, Dev>(P, aux, bits, x, y, z, s, F);
+        // only fluid sites feel the Shan-Chen force (code/lb3d_collision.F90:160-172)
+        if ((bits >> 18) & 1u) {
+#pragma unroll
+            for (int c = 0; c < C; c++) F[c][0] = F[c][1] = F[c][2] = R(0);
+        }
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int i = 0; i < 19; i++)
 #pragma unroll
-            for (int c = 0; c < C; c++) n[c][i] = pull_rock<R, C>(f, rock, P, c, i, x, y, z, self_rock);
-        // only fluid sites feel the Shan-Chen force (code/lb3d_collision.F90:160-172)
-        if (self_rock) {
-#pragma unroll
-            for (int c = 0; c < C; c++) F[c][0] = F[c][1] = F[c][2] = R(0);
-        } else {
-            sc_forces_wall<R, Dev>(P, aux, rock, x, y, z, s, F);
-        }
+            for (int c = 0; c < C; c++) n[c][i] = pull_rock<R, C>(f, bits, P, c, i, x, y, z);
     } else {
         // the force stencil first, then the pulls (a compiler barrier keeps
         // them after it): the populations are not live while the stencil's

@@ -323,6 +323,7 @@ int lb3d_gpu_batch_create(int32_t nlat, const lb3d_params *params, lb3d_batch **
     for (int k = 0; k < nlat; k++) {
         b->p.push_back(params[k]);
         b->L.push_back(b->prec == LB3D_FP64 ? make_launcher_fp64(params[k]) : make_launcher_fp32(params[k]));
+        b->L.back()->xg = two_pass_plan(params[k]).xg;
         uint64_t n = (uint64_t)params[k].nx * params[k].ny * params[k].nz;
         b->ns.push_back(n);
         b->f_off.push_back(fo);

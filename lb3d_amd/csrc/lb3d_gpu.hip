@@ -179,26 +179,42 @@ namespace lb3d {
 // z-chunk computes 2 planes of psi more than it collides and its planes are a
 // serial chain, so it needs enough planes for all CUs.  Measured per step,
 // two-pass against one-pass with the tile below (us):
-//   FP32  64^3 24 / 26, 80^3 41 / 41, 90x100x77 54 / 50, 112^3 135 / 105,
-//         128^3 202 / 146, 200^3 757 / 555, 256^3 1592 / 1099;
-//   FP64  61x47x53 31 / 35, 64^3 44 / 45, 90x100x77 141 / 130,
+//   FP32  64^3 24 / 26, 80^3 41 / 41, 90x100x77 51 / 47, 96^3 70 / 58,
+//         112^3 135 / 103, 128^3 202 / 142, 200^3 757 / 554, 256^3 1592 / 1088;
+//   FP64  61x47x53 31 / 35, 64^3 44 / 45, 77x91x69 87 / 80, 90x100x77 141 / 130,
 //         128^3 386 / 300, 256^3 3170 / 2390.
 // So the lines lie at 0.6 and 0.4 million sites.  Lees-Edwards stays on the two
 // passes, whose compact edge columns the one-pass plan does not have.
 //
 // Tile: 512 threads (one work-group fills a CU's registers), the shape that
-// leaves the fewest threads idle over the whole plane.  FP32 prefers whole
-// rows, with no x halo, by 10% (256^3: 256x2 1.10 ms, 128x4 1.22-1.30; 160^3:
-// 160x3 294 us, 80x6 315); FP64 planes do not fit the L2 with their halos, so
-// there the halo sites count too (256^3: 64x8 2.39 ms, 128x4 2.49, 256x2 2.62;
-// 200^3: 100x5 1.24 ms, 50x10 1.31).
+// leaves the fewest threads idle over the whole plane.  A tile narrower than
+// the row pays for its x halo, the more the narrower it is (FP32, against the
+// time of the whole-row tile with as many tiles: 128 columns +10-18%, 100
+// +16%, 75 +4%, 64 +7%, 45 +11%, 42 +15%, 32 +25%, 30 +36%; 96^3: 96x5 58 us,
+// 32x16 65, 90x100x77: 90x5 47 us, 30x17 58).  FP64 planes do not fit the L2
+// with their halos, so there the halo sites count too (256^3: 64x8 2.39 ms,
+// 128x4 2.49, 256x2 2.62; 200^3: 100x5 1.24 ms, 50x10 1.31).
 //
 // z-chunk: the work-groups run in rounds of 256 (one per CU), each lz + 2
 // planes long; the fewest planes in a row win (200^3 FP32: 240 work-groups of
 // 67 planes 555 us, 480 of 34 614).
-Plan default_plan(const lb3d_params &p)
+//
+// XCD chunks of the two-pass plan: one run of tiles per XCD while the
+// populations fit the memory-side cache (90x100x77 ternary FP32 132 us, in
+// chunks of 8 136, plain order 143); beyond it the eight runs open eight times
+// as many DRAM pages as chunks of 8 tiles do (80x96x88 ternary FP64 256 / 237
+// us, 192^3 ternary FP32 1249 / 1199, 160^3 FP64 794 / 753).
+Plan two_pass_plan(const lb3d_params &p)
 {
     Plan q;
+    const uint64_t sites = (uint64_t)p.nx * (uint64_t)p.ny * (uint64_t)p.nz;
+    if (19u * (uint64_t)p.ncomp * sites * (p.precision == LB3D_FP64 ? 8u : 4u) > MALL_BYTES) q.xg = 8;
+    return q;
+}
+
+Plan default_plan(const lb3d_params &p)
+{
+    Plan q = two_pass_plan(p);
     const bool fp64 = p.precision == LB3D_FP64;
     const int64_t sites = (int64_t)p.nx * p.ny * p.nz;
     if (p.ncomp != 2 || p.bdist != 2 || p.inv_fluid != 0 || p.boundary != LB3D_BC_PERIODIC) return q;
@@ -216,8 +232,7 @@ Plan default_plan(const lb3d_params &p)
         // more than 256 sites, or the kernel would be that of a smaller work-group
         if (tx * ty <= T / 2) continue;
         const double nh = 2.0 * (tx + 2) + 2.0 * ty;
-        const double cost = (double)kx * ky *
-                            (fp64 ? (T + 0.2 * nh) * (1.0 + 4.0 / tx) : (kx > 1 ? 1.1 : 1.0) * T);
+        const double cost = (double)kx * ky * (fp64 ? T + 0.2 * nh : T) * (kx > 1 ? 1.04 + 6.0 / tx : 1.0);
         if (best == 0.0 || cost < best) {
             best = cost;
             q.tx = tx;
@@ -393,7 +408,7 @@ int lb3d_gpu_create(const lb3d_params *p, lb3d_ctx **out)
         return cleanup(LB3D_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     // lb3d_gpu_autotune picks the measured best
     c->plan = default_plan(*p);
-    if (c->plan.fused && !c->L->fused_supported(c->plan.tx, c->plan.ty, c->plan.stage)) c->plan = Plan();
+    if (c->plan.fused && !c->L->fused_supported(c->plan.tx, c->plan.ty, c->plan.stage)) c->plan = two_pass_plan(*p);
     c->L->xg = c->plan.xg;
     c->host_le.shear_u = p->shear_u;
     c->host_le.shear_tmp = p->shear_u;
@@ -456,7 +471,7 @@ static void set_walls(lb3d_ctx *c, bool on)
     c->L->walls = on;
     c->b.rock = on ? c->rock_dev : nullptr;
     if (on && c->plan.fused) {
-        c->plan = Plan();
+        c->plan = two_pass_plan(c->p);
         c->L->xg = c->plan.xg;
     }
 }
@@ -872,9 +887,7 @@ int lb3d_gpu_autotune(lb3d_ctx *c, int32_t trial_steps, char *report, int32_t re
     if (c->state != IDLE) return fail(LB3D_ESTATE, "autotune needs a completed timestep");
     if (trial_steps < 1) trial_steps = 1;
     std::vector<Plan> cands;
-    Plan two;
-    two.fused = false;
-    cands.push_back(two);
+    cands.push_back(two_pass_plan(c->p));
     // the untuned plan's tile, which is fitted to the lattice
     const Plan fit = c->L->walls ? Plan() : default_plan(c->p);
     if (fit.fused)

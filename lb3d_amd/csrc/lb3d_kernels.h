@@ -556,6 +556,33 @@ __device__ __forceinline__ R dot_c(int i, R a0, R a1, R a2)
     return t;
 }
 
+// Terms of the FP32 stencil sums, fused multiply-adds with the components of
+// c_i and the weight g_i as constants.
+__device__ constexpr int cvec(int i, int a) { return a == 0 ? CX[i] : (a == 1 ? CY[i] : CZ[i]); }
+// t += g_i c_i v
+__device__ __forceinline__ void acc_odd(int i, float v, float (&t)[3])
+{
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+        if (cvec(i, a) != 0) t[a] = __builtin_fmaf(float(GD[i] * cvec(i, a)), v, t[a]);
+}
+// t += g_i w (p - 2 c_i (c_i . p)): on an axis the component along it changes
+// sign; on a diagonal of the plane (a, b), p_a -> -p_a - 2 c_a c_b p_b and
+// likewise for b
+__device__ __forceinline__ void acc_reflected(int i, float p0, float p1, float p2, float w, float (&t)[3])
+{
+    const float p[3] = {p0, p1, p2};
+    const float gw = float(GD[i]) * w;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        t[a] = __builtin_fmaf(cvec(i, a) != 0 ? -gw : gw, p[a], t[a]);
+        if (GD[i] == 1 && cvec(i, a) != 0) {
+            const int b = cvec(i, (a + 1) % 3) != 0 ? (a + 1) % 3 : (a + 2) % 3;
+            t[a] = __builtin_fmaf(float(-2 * cvec(i, a) * cvec(i, b)) * w, p[b], t[a]);
+        }
+    }
+}
+
 // --------------------------------------------------------------------------
 // k_dipole: dipole relaxation, code/lb3d_collision.F90:296-403 (ternary).
 // The dipole update of one site from its own advected dipole hs = da(x) and
@@ -581,24 +608,45 @@ __device__ __forceinline__ void dipole_core(const Phys<R> &P, R hs0, R hs1, R hs
         sd2 = hs2 / sN;
     }
     R hc0 = R(0), hc1 = R(0), hc2 = R(0);
+    if constexpr (Dev) {
+        // FP32: the same sums with the products of c_i's components (-1, 0, 1)
+        // and g_i written out, 7 fused operations per neighbour in place of 17
+        // (430 -> 300 vector instructions; the pass was bound by them: 18
+        // neighbour vectors take 16 us of L1 at 128^3, the instructions took
+        // 23 of its 31 us).  The exact sign of g_bs is applied to the sum.
+        R hc[3] = {R(0), R(0), R(0)}, hs[3] = {hs0, hs1, hs2};
 #pragma unroll
-    for (int i = 0; i < 18; i++) {
-        // -sign(1,g_bs)*(rho_b - rho_r)(x+c_i)*g_i (raw densities, :361-369)
-        R gs = R(GD[i]);
-        R hc_m = -((P.sign_g_bs * get_drb(i)) * gs);
-        if (CX[i] != 0) hc0 = hc0 + hc_m * R(CX[i]);
-        if (CY[i] != 0) hc1 = hc1 + hc_m * R(CY[i]);
-        if (CZ[i] != 0) hc2 = hc2 + hc_m * R(CZ[i]);
-        R p0 = get_da(i, 0), p1 = get_da(i, 1), p2 = get_da(i, 2);
-        R hs_dot = R(2.0) * dot_c<R>(i, p0, p1, p2);
-        // (p - c_i hs_dot) g_i; a zero component of c_i leaves p
-        R q0 = p0, q1 = p1, q2 = p2;
-        if (CX[i] != 0) q0 = p0 - R(CX[i]) * hs_dot;
-        if (CY[i] != 0) q1 = p1 - R(CY[i]) * hs_dot;
-        if (CZ[i] != 0) q2 = p2 - R(CZ[i]) * hs_dot;
-        hs0 = hs0 + q0 * gs;
-        hs1 = hs1 + q1 * gs;
-        hs2 = hs2 + q2 * gs;
+        for (int i = 0; i < 18; i++) {
+            const R drb = get_drb(i);
+            acc_odd(i, drb, hc);
+            acc_reflected(i, get_da(i, 0), get_da(i, 1), get_da(i, 2), R(1), hs);
+        }
+        hc0 = -(P.sign_g_bs * hc[0]);
+        hc1 = -(P.sign_g_bs * hc[1]);
+        hc2 = -(P.sign_g_bs * hc[2]);
+        hs0 = hs[0];
+        hs1 = hs[1];
+        hs2 = hs[2];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 18; i++) {
+            // -sign(1,g_bs)*(rho_b - rho_r)(x+c_i)*g_i (raw densities, :361-369)
+            R gs = R(GD[i]);
+            R hc_m = -((P.sign_g_bs * get_drb(i)) * gs);
+            if (CX[i] != 0) hc0 = hc0 + hc_m * R(CX[i]);
+            if (CY[i] != 0) hc1 = hc1 + hc_m * R(CY[i]);
+            if (CZ[i] != 0) hc2 = hc2 + hc_m * R(CZ[i]);
+            R p0 = get_da(i, 0), p1 = get_da(i, 1), p2 = get_da(i, 2);
+            R hs_dot = R(2.0) * dot_c<R>(i, p0, p1, p2);
+            // (p - c_i hs_dot) g_i; a zero component of c_i leaves p
+            R q0 = p0, q1 = p1, q2 = p2;
+            if (CX[i] != 0) q0 = p0 - R(CX[i]) * hs_dot;
+            if (CY[i] != 0) q1 = p1 - R(CY[i]) * hs_dot;
+            if (CZ[i] != 0) q2 = p2 - R(CZ[i]) * hs_dot;
+            hs0 = hs0 + q0 * gs;
+            hs1 = hs1 + q1 * gs;
+            hs2 = hs2 + q2 * gs;
+        }
     }
     R h0 = hc0 + hs0, h1 = hc1 + hs1, h2 = hc2 + hs2;
     R h_m = P.beta * sqrt(h0 * h0 + h1 * h1 + h2 * h2);
@@ -673,43 +721,98 @@ __device__ __forceinline__ void sc_forces3(const Phys<R> &P, const R (&dbx)[3], 
     R frb[3] = {R(0), R(0), R(0)}, fbr[3] = {R(0), R(0), R(0)};
     R fcs[3] = {R(0), R(0), R(0)}, fsc[3] = {R(0), R(0), R(0)}, fss[3] = {R(0), R(0), R(0)};
     const R dbx0 = dbx[0], dbx1 = dbx[1], dbx2 = dbx[2];
-    const R dpsi_br = Dev ? P.psi0[1] - P.psi0[0] : R(0);
+    if constexpr (Dev) {
+        // FP32: the sums over the neighbours are linear in the site's own
+        // dipole x, so they are gathered as tensors and contracted with x once
+        // (about 20 fused operations per neighbour in place of 45):
+        //   fsc_k = sum_i g_i t (x_k - 2 c_k (c.x)),  t = psi_b - psi_r: from
+        //     the sums of t on the axes (ta), the diagonals of each plane (td)
+        //     and those weighted by the product of c's components (te);
+        //     psi_b0 - psi_r0, the constant part of t, drops out of the sum;
+        //   fss_k = 8 sum_i g_i [c_k (d.x) - 2 c_k (c.x)(c.d) + d_k (c.x) +
+        //     (c.d) x_k] = 8 (sum_l G_kl x_l + T x_k),  d = psi_s db:
+        //     G symmetric, G_kk from the diagonals alone, and the diagonals'
+        //     part of T = sum_i g_i (c.d) is minus half the trace of G.
+        R ta[3] = {R(0), R(0), R(0)}, td[3] = {R(0), R(0), R(0)}, te[3] = {R(0), R(0), R(0)};
+        R gd[3] = {R(0), R(0), R(0)}, go[3] = {R(0), R(0), R(0)}, tax = R(0);
+        // planes and off-diagonal elements: index 0 (y,z), 1 (x,z), 2 (x,y)
 #pragma unroll
-    for (int i = 0; i < 18; i++) {
-        const R c0 = R(CX[i]), c1 = R(CY[i]), c2 = R(CZ[i]);
-        const R gs = R(GD[i]);
-        R pr = get_psi(i, 0);
-        R pb = get_psi(i, 1);
-        R ps = get_psi(i, 2);
-        if constexpr (Dev) ps = P.psi0[2] + ps;
-        R green_r = pb * gs, green_b = pr * gs;
-        if (CX[i] != 0) { frb[0] = frb[0] + green_r * c0; fbr[0] = fbr[0] + green_b * c0; }
-        if (CY[i] != 0) { frb[1] = frb[1] + green_r * c1; fbr[1] = fbr[1] + green_b * c1; }
-        if (CZ[i] != 0) { frb[2] = frb[2] + green_r * c2; fbr[2] = fbr[2] + green_b * c2; }
-        // a zero component of c_i makes its terms exact zeros, which are
-        // skipped (dot_c and the conditionals); the rest keep the order
-        R d0 = get_db(i, 0) * ps;
-        R d1 = get_db(i, 1) * ps;
-        R d2 = get_db(i, 2) * ps;
-        R d_dotc = dot_c<R>(i, d0, d1, d2);
-        fcs[0] = fcs[0] + (CX[i] != 0 ? d0 - (R(2.0) * d_dotc) * c0 : d0) * gs;
-        fcs[1] = fcs[1] + (CY[i] != 0 ? d1 - (R(2.0) * d_dotc) * c1 : d1) * gs;
-        fcs[2] = fcs[2] + (CZ[i] != 0 ? d2 - (R(2.0) * d_dotc) * c2 : d2) * gs;
-        R di_dotc = dot_c<R>(i, dbx0, dbx1, dbx2);
-        R greenc_s = ((pb - pr) + dpsi_br) * gs;
-        fsc[0] = fsc[0] + greenc_s * (CX[i] != 0 ? dbx0 - (R(2.0) * di_dotc) * c0 : dbx0);
-        fsc[1] = fsc[1] + greenc_s * (CY[i] != 0 ? dbx1 - (R(2.0) * di_dotc) * c1 : dbx1);
-        fsc[2] = fsc[2] + greenc_s * (CZ[i] != 0 ? dbx2 - (R(2.0) * di_dotc) * c2 : dbx2);
-        R di_dot_d = d0 * dbx0 + d1 * dbx1 + d2 * dbx2;
-        R green_ss = R(8.0) * gs;
-        R a = di_dot_d - (R(2.0) * di_dotc) * d_dotc;
-        R q0 = d0 * di_dotc, q1 = d1 * di_dotc, q2 = d2 * di_dotc;
-        if (CX[i] != 0) q0 = a * c0 + d0 * di_dotc;
-        if (CY[i] != 0) q1 = a * c1 + d1 * di_dotc;
-        if (CZ[i] != 0) q2 = a * c2 + d2 * di_dotc;
-        fss[0] = fss[0] + green_ss * (q0 + d_dotc * dbx0);
-        fss[1] = fss[1] + green_ss * (q1 + d_dotc * dbx1);
-        fss[2] = fss[2] + green_ss * (q2 + d_dotc * dbx2);
+        for (int i = 0; i < 18; i++) {
+            const R pr = get_psi(i, 0), pb = get_psi(i, 1), ps = P.psi0[2] + get_psi(i, 2);
+            acc_odd(i, pb, frb);
+            acc_odd(i, pr, fbr);
+            const R d[3] = {get_db(i, 0), get_db(i, 1), get_db(i, 2)};
+            acc_reflected(i, d[0], d[1], d[2], ps, fcs);
+            const R t = pb - pr;
+            if (GD[i] == 2) {
+                const int a = CX[i] != 0 ? 0 : (CY[i] != 0 ? 1 : 2), b = (a + 1) % 3, e = (a + 2) % 3;
+                const R w = R(2 * cvec(i, a)) * ps;
+                ta[a] = ta[a] + t;
+                tax = __builtin_fmaf(w, d[a], tax);
+                // elements (a, b) and (a, e), stored at the third index
+                go[e] = __builtin_fmaf(w, d[b], go[e]);
+                go[b] = __builtin_fmaf(w, d[e], go[b]);
+            } else {
+                const int n = CX[i] == 0 ? 0 : (CY[i] == 0 ? 1 : 2), a = (n + 1) % 3, b = (n + 2) % 3;
+                const R wa = R(cvec(i, a)) * ps, wb = R(cvec(i, b)) * ps;
+                td[n] = td[n] + t;
+                te[n] = __builtin_fmaf(R(cvec(i, a) * cvec(i, b)), t, te[n]);
+                gd[a] = __builtin_fmaf(wb, d[b], gd[a]);  // G_aa / -2
+                gd[b] = __builtin_fmaf(wa, d[a], gd[b]);
+                go[n] = __builtin_fmaf(-wa, d[b], go[n]);
+                go[n] = __builtin_fmaf(-wb, d[a], go[n]);
+                go[b] = __builtin_fmaf(wa, d[n], go[b]);  // element (a, n)
+                go[a] = __builtin_fmaf(wb, d[n], go[a]);  // element (b, n)
+            }
+        }
+        const R x[3] = {dbx0, dbx1, dbx2};
+        const R T = tax + (gd[0] + gd[1] + gd[2]);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const int a = (k + 1) % 3, b = (k + 2) % 3;
+            // sum_i g_i t (1 - 2 c_k^2)
+            const R m = R(2.0) * ((ta[a] + ta[b]) - ta[k]) + ((td[k] - td[a]) - td[b]);
+            fsc[k] = __builtin_fmaf(m, x[k], R(-2.0) * __builtin_fmaf(te[b], x[a], te[a] * x[b]));
+            const R own = __builtin_fmaf(R(-2.0), gd[k], T);
+            fss[k] = R(8.0) * __builtin_fmaf(own, x[k], __builtin_fmaf(go[b], x[a], go[a] * x[b]));
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 18; i++) {
+            const R c0 = R(CX[i]), c1 = R(CY[i]), c2 = R(CZ[i]);
+            const R gs = R(GD[i]);
+            R pr = get_psi(i, 0);
+            R pb = get_psi(i, 1);
+            R ps = get_psi(i, 2);
+            R green_r = pb * gs, green_b = pr * gs;
+            if (CX[i] != 0) { frb[0] = frb[0] + green_r * c0; fbr[0] = fbr[0] + green_b * c0; }
+            if (CY[i] != 0) { frb[1] = frb[1] + green_r * c1; fbr[1] = fbr[1] + green_b * c1; }
+            if (CZ[i] != 0) { frb[2] = frb[2] + green_r * c2; fbr[2] = fbr[2] + green_b * c2; }
+            // a zero component of c_i makes its terms exact zeros, which are
+            // skipped (dot_c and the conditionals); the rest keep the order
+            R d0 = get_db(i, 0) * ps;
+            R d1 = get_db(i, 1) * ps;
+            R d2 = get_db(i, 2) * ps;
+            R d_dotc = dot_c<R>(i, d0, d1, d2);
+            fcs[0] = fcs[0] + (CX[i] != 0 ? d0 - (R(2.0) * d_dotc) * c0 : d0) * gs;
+            fcs[1] = fcs[1] + (CY[i] != 0 ? d1 - (R(2.0) * d_dotc) * c1 : d1) * gs;
+            fcs[2] = fcs[2] + (CZ[i] != 0 ? d2 - (R(2.0) * d_dotc) * c2 : d2) * gs;
+            R di_dotc = dot_c<R>(i, dbx0, dbx1, dbx2);
+            R greenc_s = (pb - pr) * gs;
+            fsc[0] = fsc[0] + greenc_s * (CX[i] != 0 ? dbx0 - (R(2.0) * di_dotc) * c0 : dbx0);
+            fsc[1] = fsc[1] + greenc_s * (CY[i] != 0 ? dbx1 - (R(2.0) * di_dotc) * c1 : dbx1);
+            fsc[2] = fsc[2] + greenc_s * (CZ[i] != 0 ? dbx2 - (R(2.0) * di_dotc) * c2 : dbx2);
+            R di_dot_d = d0 * dbx0 + d1 * dbx1 + d2 * dbx2;
+            R green_ss = R(8.0) * gs;
+            R a = di_dot_d - (R(2.0) * di_dotc) * d_dotc;
+            R q0 = d0 * di_dotc, q1 = d1 * di_dotc, q2 = d2 * di_dotc;
+            if (CX[i] != 0) q0 = a * c0 + d0 * di_dotc;
+            if (CY[i] != 0) q1 = a * c1 + d1 * di_dotc;
+            if (CZ[i] != 0) q2 = a * c2 + d2 * di_dotc;
+            fss[0] = fss[0] + green_ss * (q0 + d_dotc * dbx0);
+            fss[1] = fss[1] + green_ss * (q1 + d_dotc * dbx1);
+            fss[2] = fss[2] + green_ss * (q2 + d_dotc * dbx2);
+        }
     }
     R psr = ps_own[0], psb = ps_own[1], pss = ps_own[2];
     if constexpr (Dev) {

@@ -39,8 +39,9 @@ struct Plan {
     int stage = 1;      // plane k's populations: 0 registers, 1 LDS, 2 pulled again
     uint32_t xg = 0;    // tiles per XCD chunk (xcd_tile): 1 plain order, 0 one run per XCD
 };
-// The plan of a lattice that nobody has tuned.
+// The plan of a lattice that nobody has tuned, and its two-pass plan.
 Plan default_plan(const lb3d_params &p);
+Plan two_pass_plan(const lb3d_params &p);
 
 // Steps of a captured graph, and when one is captured.  Measured per step
 // (us), plain launches against graphs of 2, 16 and 64 steps: 16^3 binary FP64

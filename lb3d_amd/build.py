@@ -51,7 +51,7 @@ def build_hip(jobs=4):
         if p.wait() != 0:
             raise SystemExit("hipcc failed")
     tmp = LIB + ".tmp"
-    run([HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp] + objs)
+    run([HIPCC, "-shared", "-fPIC", "-pthread", f"--offload-arch={ARCH}", "-o", tmp] + objs)
     os.replace(tmp, LIB)
     tmp = PROBE + ".tmp"
     run([HIPCC, os.path.join(CSRC, "lb3d_bwprobe.hip"), "-shared", "-o", tmp] + COMMON)

@@ -36,7 +36,6 @@ struct lb3d_batch {
     void *f[2] = {nullptr, nullptr};
     void *aux = nullptr, *db = nullptr, *lat = nullptr, *items = nullptr;
     double *partials = nullptr;
-    DevScratch io;  // pieces of read-backs, kept for the next
     uint32_t nitems = 0;
     hipStream_t stream = nullptr;
     hipGraphExec_t graph = nullptr;
@@ -313,6 +312,7 @@ int lb3d_gpu_batch_create(int32_t nlat, const lb3d_params *params, lb3d_batch **
         if (q.ncomp == 3 && !(q.tau_d > 0.0)) return set_error(LB3D_EINVAL, "tau_d must be positive");
     }
     lb3d_batch *b = new lb3d_batch();
+    io_users(1);
     b->nlat = nlat;
     b->C = p0.ncomp;
     b->prec = p0.precision;
@@ -383,11 +383,11 @@ int lb3d_gpu_batch_destroy(lb3d_batch *b)
     for (void *q : {b->aux, b->aux1, b->db, b->lat, b->items, (void *)b->partials, b->cm_items, b->edge_items,
                     b->edge_sites})
         if (q) (void)hipFree(q);
-    b->io.release();
     if (b->stream) (void)hipStreamDestroy(b->stream);
     for (Launcher *l : b->L) delete l;
     delete b->B;
     delete b;
+    io_users(-1);
     return LB3D_OK;
 }
 
@@ -425,8 +425,8 @@ int lb3d_gpu_batch_get_populations(lb3d_batch *b, int32_t k, double *out)
     clear_error();
     if (!b || k < 0 || k >= b->nlat || !out) return set_error(LB3D_EINVAL, "bad argument");
     const void *f = view(b, k).f[b->cur];
-    BTRY(b->rs == 4 ? fetch_populations<float>(b->io, b->stream, b->p[k], f, out)
-                    : fetch_populations<double>(b->io, b->stream, b->p[k], f, out));
+    BTRY(b->rs == 4 ? fetch_populations<float>(b->stream, b->p[k], f, out)
+                    : fetch_populations<double>(b->stream, b->p[k], f, out));
     return LB3D_OK;
 }
 

@@ -92,8 +92,6 @@ struct lb3d_ctx {
     int64_t plan_steps = 0;  // steps run on the current plan (a graph is captured after GRAPH_AFTER)
     double *d_partials = nullptr;
     uint8_t *rock_dev = nullptr;  // rock mask (lattices with walls)
-    DevScratch io;                // pieces of read-backs and uploads, kept for the next
-    uint32_t *rock_count = nullptr;  // rock sites of an upload
     size_t f_bytes = 0, aux_bytes = 0, db_bytes = 0;
     size_t aux_elems = 0;  // elements of the aux field
     Plan plan;
@@ -172,6 +170,61 @@ static int check_params(const lb3d_params *p)
 }
 
 namespace lb3d {
+namespace {
+std::mutex g_io_mu;
+HostIO *g_io[IO_KEPT] = {};
+int g_io_users = 0;
+}  // namespace
+
+HostIO *io_lend()
+{
+    int dev = -1;
+    (void)hipGetDevice(&dev);
+    {
+        std::lock_guard<std::mutex> lock(g_io_mu);
+        for (HostIO *&q : g_io)
+            if (q && q->device == dev) {
+                HostIO *io = q;
+                q = nullptr;
+                return io;
+            }
+    }
+    HostIO *io = new HostIO();
+    io->device = dev;
+    return io;
+}
+
+void io_give_back(HostIO *io)
+{
+    if (io->cap <= IO_KEPT_BYTES) {
+        std::lock_guard<std::mutex> lock(g_io_mu);
+        if (g_io_users > 0)
+            for (HostIO *&q : g_io)
+                if (!q) {
+                    q = io;
+                    return;
+                }
+    }
+    io->release();
+    delete io;
+}
+
+void io_users(int change)
+{
+    HostIO *gone[IO_KEPT] = {};
+    {
+        std::lock_guard<std::mutex> lock(g_io_mu);
+        g_io_users += change;
+        if (g_io_users == 0)
+            for (size_t k = 0; k < IO_KEPT; k++) std::swap(gone[k], g_io[k]);
+    }
+    for (HostIO *io : gone)
+        if (io) {
+            io->release();
+            delete io;
+        }
+}
+
 // The one-pass kernel (binary, bdist 2, periodic) with a tile fitted to the
 // lattice, or the two-pass kernels.
 //
@@ -368,6 +421,7 @@ int lb3d_gpu_create(const lb3d_params *p, lb3d_ctx **out)
     int rc = check_params(p);
     if (rc) return rc;
     lb3d_ctx *c = new lb3d_ctx();
+    io_users(1);
     c->p = *p;
     c->le = p->boundary == LB3D_BC_LEES_EDWARDS;
     c->L = p->precision == LB3D_FP64 ? make_launcher_fp64(*p) : make_launcher_fp32(*p);
@@ -435,11 +489,10 @@ int lb3d_gpu_destroy(lb3d_ctx *c)
     if (c->b.le) (void)hipFree(c->b.le);
     if (c->d_partials) (void)hipFree(c->d_partials);
     if (c->rock_dev) (void)hipFree(c->rock_dev);
-    if (c->rock_count) (void)hipFree(c->rock_count);
-    c->io.release();
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c->L;
     delete c;
+    io_users(-1);
     return LB3D_OK;
 }
 
@@ -476,8 +529,7 @@ static void set_walls(lb3d_ctx *c, bool on)
     }
 }
 
-// Site records in pieces of whole z planes of at most REC_BYTES (or one plane).
-constexpr size_t REC_BYTES = 64u << 20;
+// Site records.
 static RecLayout rec_layout(const lb3d_params &p, int h, int sd)
 {
     RecLayout L;
@@ -492,12 +544,6 @@ static RecLayout rec_layout(const lb3d_params &p, int h, int sd)
     L.rock_b = p.rock_colour_b;
     return L;
 }
-static int rec_planes(size_t plane_bytes, int total)
-{
-    const size_t k = REC_BYTES / plane_bytes;
-    return k < 1 ? 1 : (k > (size_t)total ? total : (int)k);
-}
-
 static int rebuild_aux(lb3d_ctx *c);
 
 int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, int32_t nt0)
@@ -514,40 +560,48 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
     // the last step, may still be asked for: its moments are kept first.)
     int rc = LB3D_OK;
     if (!walls_ok && (rc = rebuild_aux(c))) return rc;
-    if (!c->rock_count) HIP_TRY(hipMalloc((void **)&c->rock_count, sizeof(uint32_t)));
     const RecLayout L = rec_layout(p, h, sd);
-    if (walls_ok && !c->rock_dev) HIP_TRY(hipMalloc((void **)&c->rock_dev, L.ns));
+    // the mask goes to the aux field, which holds nothing after an upload, and
+    // from there to its own memory if there are rock sites
+    uint8_t *mask = nullptr;
+    if (walls_ok) {
+        mask = (uint8_t *)c->b.aux;
+        c->aux_valid = false;
+    }
+    IoLoan io;
     const PopBase pb = pop_base(p);
     const int to = 1 - c->b.cur;
     const uint32_t nxy = (uint32_t)p.nx * (uint32_t)p.ny;
     const size_t plane = (size_t)(p.nx + 2 * h) * (size_t)(p.ny + 2 * h) * (size_t)sd;  // doubles
-    const int per = rec_planes(plane * 8, p.nz);
-    HIP_TRY(c->io.ensure((size_t)per * plane * 8));
-    const uint32_t zero = 0;
-    HIP_TRY(hipMemcpyAsync(c->rock_count, &zero, sizeof zero, hipMemcpyHostToDevice, c->stream));
-    for (int z = 0; z < p.nz; z += per) {
-        const int k = p.nz - z < per ? p.nz - z : per;
-        HIP_TRY(hipMemcpyAsync(c->io.p, N + (size_t)(z + h) * plane, (size_t)k * plane * 8, hipMemcpyHostToDevice,
-                               c->stream));
-        const uint32_t n = (uint32_t)k * nxy, nb = (n + REC_SITES - 1) / REC_SITES;
-        const size_t lds = (size_t)REC_SITES * sd * 8;
+    // pieces of whole z planes
+    const size_t piece = plane * 8 * (IO_PIECE < plane * 8 ? 1 : IO_PIECE / (plane * 8));
+    const size_t lds = (size_t)REC_SITES * sd * 8;
+    HIP_TRY(io->ensure(1));
+    HIP_TRY(hipMemsetAsync(io->count, 0, sizeof(uint32_t), c->stream));
+    HIP_TRY(io->up(c->stream, N + (size_t)h * plane, (size_t)p.nz * plane * 8, piece, [&](size_t at, size_t len, void *buf) {
+        const uint32_t z = (uint32_t)(at / (plane * 8)), n = (uint32_t)(len / (plane * 8)) * nxy;
+        const uint32_t nb = (n + REC_SITES - 1) / REC_SITES;
         auto go = [&](auto r) {
             using R = decltype(r);
-            k_put_sites<R><<<nb, 256, lds, c->stream>>>((const double *)c->io.p, (uint32_t)(z + h), L, pb,
-                                                        (uint32_t)z * nxy, n, (R *)c->b.f[to], (R *)c->dbk[to],
-                                                        walls_ok ? c->rock_dev : nullptr, c->rock_count);
+            k_put_sites<R><<<nb, 256, lds, c->stream>>>((const double *)buf, z + (uint32_t)h, L, pb, z * nxy, n,
+                                                        (R *)c->b.f[to], (R *)c->dbk[to],
+                                                        mask, io->count);
         };
         is_dev(c) ? go(float()) : go(double());
-        HIP_TRY(hipGetLastError());
-    }
+    }));
     uint32_t nrock = 0;
-    HIP_TRY(hipMemcpyAsync(&nrock, c->rock_count, sizeof nrock, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipMemcpyAsync(io->pin[0], io->count, sizeof nrock, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    std::memcpy(&nrock, io->pin[0], sizeof nrock);
     if (nrock && !walls_ok) {
         c->aux_from_prev = false;  // f[1 - cur] holds the refused records
         if (p.ncomp != 2 || c->le)
             return fail(LB3D_EINVAL, "rock sites (walls) are supported on periodic binary lattices");
         return fail(LB3D_EINVAL, "rock sites (walls) and the Zou-He boundary are not supported together");
+    }
+    if (nrock) {
+        if (!c->rock_dev) HIP_TRY(hipMalloc((void **)&c->rock_dev, L.ns));
+        HIP_TRY(hipMemcpyAsync(c->rock_dev, mask, L.ns, hipMemcpyDeviceToDevice, c->stream));
     }
     set_walls(c, nrock != 0);
     set_cur(c, to);
@@ -584,8 +638,8 @@ int lb3d_gpu_get_populations(lb3d_ctx *c, double *out)
     g_err.clear();
     if (!c || !out) return fail(LB3D_EINVAL, "NULL argument");
     const void *f = c->b.f[c->b.cur];
-    HIP_TRY(is_dev(c) ? fetch_populations<float>(c->io, c->stream, c->p, f, out)
-                      : fetch_populations<double>(c->io, c->stream, c->p, f, out));
+    HIP_TRY(is_dev(c) ? fetch_populations<float>(c->stream, c->p, f, out)
+                      : fetch_populations<double>(c->stream, c->p, f, out));
     return LB3D_OK;
 }
 
@@ -615,27 +669,21 @@ int lb3d_gpu_download_sites(lb3d_ctx *c, double *N, int32_t h, int32_t sd)
     if (int rc = rebuild_aux(c)) return rc;
     const RecLayout L = rec_layout(c->p, h, sd);
     const PopBase pb = pop_base(c->p);
-    const int lz = c->p.nz + 2 * h;
-    const size_t recs = (size_t)(c->p.nx + 2 * h) * (size_t)(c->p.ny + 2 * h), plane = recs * (size_t)sd;
-    const int per = rec_planes(plane * 8, lz);
-    HIP_TRY(c->io.ensure((size_t)per * plane * 8));
-    for (int z = 0; z < lz; z += per) {
-        const int k = lz - z < per ? lz - z : per;
-        const uint32_t n = (uint32_t)(recs * (size_t)k), nb = (n + REC_SITES - 1) / REC_SITES;
-        const size_t lds = (size_t)REC_SITES * sd * 8;
+    const size_t recs = (size_t)(c->p.nx + 2 * h) * (size_t)(c->p.ny + 2 * h) * (size_t)(c->p.nz + 2 * h);
+    const size_t rec = (size_t)sd * 8, lds = (size_t)REC_SITES * rec;
+    const size_t piece = IO_PIECE / (REC_SITES * rec) * (REC_SITES * rec);  // whole blocks of records
+    IoLoan io;
+    HIP_TRY(io->down(c->stream, N, recs * rec, piece, [&](size_t at, size_t len, void *buf) -> const void * {
+        const uint32_t n = (uint32_t)(len / rec), nb = (n + REC_SITES - 1) / REC_SITES;
         auto go = [&](auto r) {
             using R = decltype(r);
             k_get_sites<R><<<nb, 256, lds, c->stream>>>(
                 (const R *)c->b.f[c->b.cur], c->aux_valid ? (const R *)c->b.aux : nullptr, (const R *)c->b.db,
-                c->b.rock, pb, rho0_of(c, 0), rho0_of(c, 1), rho0_of(c, 2), L, (uint32_t)(recs * (size_t)z), n,
-                (double *)c->io.p);
+                c->b.rock, pb, rho0_of(c, 0), rho0_of(c, 1), rho0_of(c, 2), L, (uint32_t)(at / rec), n, (double *)buf);
         };
         is_dev(c) ? go(float()) : go(double());
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(N + (size_t)z * plane, c->io.p, (size_t)k * plane * 8, hipMemcpyDeviceToHost,
-                               c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
-    }
+        return buf;
+    }));
     return LB3D_OK;
 }
 
@@ -1067,7 +1115,7 @@ int lb3d_gpu_get_density(lb3d_ctx *c, double *out)
     const uint32_t ns = (uint32_t)c->p.nx * (uint32_t)c->p.ny * (uint32_t)c->p.nz;
     const PopBase pb = pop_base(c->p);
     const void *f = c->b.f[c->b.cur];
-    HIP_TRY(fetch_f64(c->io, c->stream, out, (uint64_t)c->p.ncomp * ns, [&](uint32_t q, uint32_t m, double *o) {
+    HIP_TRY(fetch_f64(c->stream, out, (uint64_t)c->p.ncomp * ns, [&](uint32_t q, uint32_t m, double *o) {
         if (is_dev(c))
             k_get_density<float><<<(m + 255) / 256, 256, 0, c->stream>>>((const float *)f, pb, ns, q, m, o);
         else
@@ -1083,7 +1131,7 @@ int lb3d_gpu_get_momentum(lb3d_ctx *c, double *out)
     const uint32_t ns = (uint32_t)c->p.nx * (uint32_t)c->p.ny * (uint32_t)c->p.nz;
     const PopBase pb = pop_base(c->p);
     const void *f = c->b.f[c->b.cur];
-    HIP_TRY(fetch_f64(c->io, c->stream, out, (uint64_t)c->p.ncomp * 3u * ns, [&](uint32_t q, uint32_t m, double *o) {
+    HIP_TRY(fetch_f64(c->stream, out, (uint64_t)c->p.ncomp * 3u * ns, [&](uint32_t q, uint32_t m, double *o) {
         if (is_dev(c))
             k_get_momentum<float><<<(m + 255) / 256, 256, 0, c->stream>>>((const float *)f, pb, ns, q, m, o);
         else

@@ -120,6 +120,7 @@ def test_full_sanity_ties_keep_the_last_site(precision):
     (2, (2, 1, 1), 4),          # a halo wider than the lattice
     (2, (131, 130, 129), 1),    # several pieces of densities and of records
     (3, (57, 61, 66), 1),
+    (2, (151, 150, 3), 1),      # one z plane of records larger than a piece
 ])
 def test_device_conversions_equal_the_host_sums_bitwise(precision, ncomp, dims, halo):
     """Uploads, downloads, densities and momenta are converted on the device in
@@ -187,3 +188,29 @@ def test_refused_rock_sites_leave_the_state():
     g.time_loop(1)
     g2.time_loop(1)
     assert np.array_equal(g.populations(), g2.populations())
+
+
+def test_transfers_of_several_threads_do_not_mix():
+    """Transfer buffers are shared by all contexts, one set per transfer: two
+    threads reading back and uploading their own lattices at the same time
+    see their own data."""
+    import threading
+    lats = [Lattice(60, 61, 62, ncomp=2), Lattice(33, 70, 41, ncomp=3, precision=LB3D_FP32_DEV)]
+    for k, g in enumerate(lats):
+        g.init_noise(k, amp=(0.02, 0.01, 0.01))
+    want = [(g.populations(), g.download_sites(), g.density()) for g in lats]
+    bad = []
+
+    def work(g, w):
+        for _ in range(6):
+            g.upload_sites(w[1])
+            got = (g.populations(), g.download_sites(), g.density())
+            if not all(np.array_equal(a, b) for a, b in zip(got, w)):
+                bad.append(g)
+
+    ts = [threading.Thread(target=work, args=a) for a in zip(lats, want)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad

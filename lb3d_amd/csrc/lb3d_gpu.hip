@@ -59,9 +59,9 @@ struct Events {
     hipEvent_t &operator[](size_t i) { return e[i]; }
 };
 
-const char *const KNAMES[] = {"le_neighbours", "le_faces_pc", "moments",
+const char *const KNAMES[] = {"le_faces_pc", "moments",
                               "le_faces_aux",  "dipole",      "collide", "fused"};
-enum { K_LEN = 0, K_LE6, K_MOM, K_LE8, K_DIP, K_COL, K_FUS, K_COUNT };
+enum { K_LE6 = 0, K_MOM, K_LE8, K_DIP, K_COL, K_FUS, K_COUNT };
 
 const char *const STAGE_NAMES[3] = {"regs", "lds", "reload"};
 
@@ -103,17 +103,15 @@ struct lb3d_ctx {
     // expects it whatever the host did before
     void *dbk[2] = {nullptr, nullptr};
     // Lees-Edwards: the edge columns b.edge_pc hold f[cur]'s (written by the
-    // two-pass collide, else gathered before the next halo-plane pass)
+    // last kernel of a step, else gathered before the next halo-plane pass)
     bool edges_ok = false;
 };
 
-// The halo-plane kernels read the compact edge columns on the two-pass
-// plan, whose moments and collide passes write them.
-static bool compact_edges(const lb3d_ctx *c) { return !c->plan.fused; }
-
+// The halo-plane kernels read the compact edge columns, which every step
+// writes.
 static void ensure_edges(lb3d_ctx *c)
 {
-    if (c->le && compact_edges(c) && !c->edges_ok) {
+    if (c->le && !c->edges_ok) {
         c->L->le_gather_edges(c->b, c->stream);
         c->edges_ok = true;
     }
@@ -225,7 +223,7 @@ void io_users(int change)
         }
 }
 
-// The one-pass kernel (binary, bdist 2, periodic) with a tile fitted to the
+// The one-pass kernel (binary, bdist 2) with a tile fitted to the
 // lattice, or the two-pass kernels.
 //
 // Which: the one-pass kernel moves 60% of the two-pass plan's bytes, but every
@@ -236,8 +234,13 @@ void io_users(int change)
 //         112^3 135 / 103, 128^3 202 / 142, 200^3 757 / 554, 256^3 1592 / 1088;
 //   FP64  61x47x53 31 / 35, 64^3 44 / 45, 77x91x69 87 / 80, 90x100x77 141 / 130,
 //         128^3 386 / 300, 256^3 3170 / 2390.
-// So the lines lie at 0.6 and 0.4 million sites.  Lees-Edwards stays on the two
-// passes, whose compact edge columns the one-pass plan does not have.
+// So the lines lie at 0.6 and 0.4 million sites.  Lees-Edwards, whose one-pass
+// plan streams the edge columns once more for the post-advection halo planes:
+//   FP32  96^3 89 / 95, 110x88x112 126 / 130, 256x64x64 112 / 107, 89x135x140
+//         212 / 201, 128^3 222 / 200, 107x246x103 347 / 283, 192^3 689 / 601;
+//   FP64  140x41x93 126 / 122, 60x84x111 134 / 128, 96^3 187 / 181, 256x64x64
+//         223 / 194, 128^3 421 / 358, 160^3 840 / 775:
+// 1.5 and 0.5 million sites.
 //
 // Tile: 512 threads (one work-group fills a CU's registers), the shape that
 // leaves the fewest threads idle over the whole plane.  A tile narrower than
@@ -246,7 +249,8 @@ void io_users(int change)
 // +16%, 75 +4%, 64 +7%, 45 +11%, 42 +15%, 32 +25%, 30 +36%; 96^3: 96x5 58 us,
 // 32x16 65, 90x100x77: 90x5 47 us, 30x17 58).  FP64 planes do not fit the L2
 // with their halos, so there the halo sites count too (256^3: 64x8 2.39 ms,
-// 128x4 2.49, 256x2 2.62; 200^3: 100x5 1.24 ms, 50x10 1.31).
+// 128x4 2.49, 256x2 2.62; 200^3: 100x5 1.24 ms, 50x10 1.31); and with
+// Lees-Edwards (256x64x64 FP32: 64x8 95 us, 128x4 103, 256x2 106).
 //
 // z-chunk: the work-groups run in rounds of 256 (one per CU), each lz + 2
 // planes long; the fewest planes in a row win (200^3 FP32: 240 work-groups of
@@ -270,8 +274,9 @@ Plan default_plan(const lb3d_params &p)
     Plan q = two_pass_plan(p);
     const bool fp64 = p.precision == LB3D_FP64;
     const int64_t sites = (int64_t)p.nx * p.ny * p.nz;
-    if (p.ncomp != 2 || p.bdist != 2 || p.inv_fluid != 0 || p.boundary != LB3D_BC_PERIODIC) return q;
-    if (sites < (fp64 ? 400000 : 600000)) return q;
+    const bool le = p.boundary == LB3D_BC_LEES_EDWARDS;
+    if (p.ncomp != 2 || p.bdist != 2 || p.inv_fluid != 0 || !(le || p.boundary == LB3D_BC_PERIODIC)) return q;
+    if (sites < (le ? (fp64 ? 500000 : 1500000) : (fp64 ? 400000 : 600000))) return q;
     const int T = 512, CUS = 256;
     double best = 0.0;
     for (int kx = 1; kx <= p.nx; kx++) {
@@ -285,7 +290,7 @@ Plan default_plan(const lb3d_params &p)
         // more than 256 sites, or the kernel would be that of a smaller work-group
         if (tx * ty <= T / 2) continue;
         const double nh = 2.0 * (tx + 2) + 2.0 * ty;
-        const double cost = (double)kx * ky * (fp64 ? T + 0.2 * nh : T) * (kx > 1 ? 1.04 + 6.0 / tx : 1.0);
+        const double cost = (double)kx * ky * (fp64 || le ? T + 0.2 * nh : T) * (kx > 1 ? 1.04 + 6.0 / tx : 1.0);
         if (best == 0.0 || cost < best) {
             best = cost;
             q.tx = tx;
@@ -449,8 +454,8 @@ int lb3d_gpu_create(const lb3d_params *p, lb3d_ctx **out)
         return cleanup(LB3D_ENOMEM, std::string("hipMalloc db: ") + hipGetErrorString(e));
     set_cur(c, 0);
     if (c->le) {
-        if ((e = hipMalloc(&c->b.edge_pc, 2 * 2 * 19 * plane * rs)) != hipSuccess ||
-            (e = hipMalloc(&c->b.edge_adv, 2 * 2 * 19 * plane * rs)) != hipSuccess)
+        const size_t edges = EDGE_SITES * plane * rs;
+        if ((e = hipMalloc(&c->b.edge_pc, edges)) != hipSuccess || (e = hipMalloc(&c->b.edge_adv, edges)) != hipSuccess)
             return cleanup(LB3D_ENOMEM, std::string("hipMalloc LE edge columns: ") + hipGetErrorString(e));
         if ((e = hipMalloc(&c->b.face_pc, 2 * 2 * 19 * plane * rs)) != hipSuccess ||
             (e = hipMalloc(&c->b.face_aux, 2 * 4 * plane * rs)) != hipSuccess)
@@ -733,7 +738,7 @@ int lb3d_gpu_bc_apply(lb3d_ctx *c, int32_t stage, int32_t nt)
         if (c->le) {
             ensure_edges(c);
             launch_le_neighbours(c, nt);
-            c->L->le_faces(c->b, false, compact_edges(c), c->stream);
+            c->L->le_faces(c->b, false, false, c->stream);
             HIP_TRY(hipGetLastError());
         }
         c->nt = nt;
@@ -741,7 +746,7 @@ int lb3d_gpu_bc_apply(lb3d_ctx *c, int32_t stage, int32_t nt)
     } else if (stage == 8) {
         if (c->state != AFTER_ADV) return fail(LB3D_ESTATE, "bc_apply(8) must follow advection");
         if (c->le) {
-            c->L->le_faces(c->b, true, compact_edges(c), c->stream);
+            c->L->le_faces(c->b, true, c->plan.fused, c->stream);
             HIP_TRY(hipGetLastError());
         }
         c->state = AFTER_BC8;
@@ -798,7 +803,7 @@ int lb3d_gpu_collision(lb3d_ctx *c)
     if (rc) return rc;
     HIP_TRY(hipGetLastError());
     flip(c);
-    c->edges_ok = compact_edges(c);
+    c->edges_ok = true;
     c->state = IDLE;
     mark_stepped(c);
     return LB3D_OK;
@@ -807,25 +812,18 @@ int lb3d_gpu_collision(lb3d_ctx *c)
 // One whole timestep on the stream (graph-capturable: kernels only).
 static int enqueue_step(lb3d_ctx *c)
 {
-    // Lees-Edwards, two-pass plan: the halo-plane kernels compute the step's
-    // offset state from the stored one and the collide stores it (no launch
-    // of k_le_neighbours); the edge columns are valid (ensure_edges before
-    // the steps are enqueued).  One-pass plan: k_le_neighbours, then the
-    // halo planes from the lattice.
-    const bool merged = c->le && !c->plan.fused;
+    // Lees-Edwards: the halo-plane kernels compute the step's offset state from
+    // the stored one and the step's last kernel stores it (no launch of
+    // k_le_neighbours); the edge columns are valid (ensure_edges before the
+    // steps are enqueued).
+    if (c->le) c->L->le_faces(c->b, false, false, c->stream, -1);
+    if (!c->plan.fused) c->L->moments(c->b, c->stream);
     if (c->le) {
-        if (!merged) launch_le_neighbours(c, -1);
-        c->L->le_faces(c->b, false, compact_edges(c), c->stream, merged ? -1 : LE_STATE_AS_IS);
+        c->L->le_faces(c->b, true, c->plan.fused, c->stream, -1);
+        c->L->set_le_commit(-1);
     }
-    if (c->plan.fused) {
-        if (c->le) c->L->le_faces(c->b, true, false, c->stream);
-    } else {
-        c->L->moments(c->b, c->stream);
-        if (c->le) c->L->le_faces(c->b, true, true, c->stream, -1);
-    }
-    if (merged) c->L->set_le_commit(-1);
     int rc = launch_collision(c);
-    if (merged) c->L->set_le_commit(LE_STATE_AS_IS);
+    c->L->set_le_commit(LE_STATE_AS_IS);
     if (rc) return rc;
     flip(c);
     return LB3D_OK;
@@ -835,7 +833,7 @@ static int ensure_graph(lb3d_ctx *c)
 {
     if (c->graph) return LB3D_OK;
     // an even number of steps starting from cur = 0 (A -> B -> ... -> A)
-    const int len = graph_steps(c->plan.fused ? (c->le ? 4 : 1) : (c->le ? 4 : c->p.ncomp));
+    const int len = graph_steps(c->plan.fused ? (c->le ? 3 : 1) : (c->le ? 4 : c->p.ncomp));
     int saved = c->b.cur;
     set_cur(c, 0);
     hipGraph_t g = nullptr;
@@ -895,7 +893,7 @@ int lb3d_gpu_run_steps(lb3d_ctx *c, int32_t nsteps)
         if ((rc = enqueue_step(c))) return rc;
     c->plan_steps += nsteps;
     HIP_TRY(hipGetLastError());
-    c->edges_ok = compact_edges(c);
+    c->edges_ok = true;
     c->nt += nsteps;
     mark_stepped(c);
     return LB3D_OK;
@@ -1015,11 +1013,11 @@ int lb3d_gpu_autotune(lb3d_ctx *c, int32_t trial_steps, char *report, int32_t re
         c->L->xg = q.xg;
         auto trial = [&]() {
             // (the edge columns are those of the state, gathered before the
-            // trials; the two-pass trials' collide overwrites them with
-            // values of the trial, which are not the state's)
-            if (c->le) c->L->le_faces(c->b, false, !q.fused, c->stream);
+            // trials; a trial's collision overwrites them with values of the
+            // trial, which are not the state's)
+            if (c->le) c->L->le_faces(c->b, false, false, c->stream);
             if (!q.fused) c->L->moments(c->b, c->stream);
-            if (c->le) c->L->le_faces(c->b, true, !q.fused, c->stream);
+            if (c->le) c->L->le_faces(c->b, true, q.fused, c->stream);
             return launch_collision(c);
         };
         if (int rc = trial()) return rc;  // warm-up
@@ -1232,7 +1230,7 @@ int lb3d_gpu_le_halo(lb3d_ctx *c, double *out)
     if (rc) return rc;
     // the stage-6 x-halo planes of the current populations and offset
     ensure_edges(c);
-    c->L->le_faces(c->b, false, compact_edges(c), c->stream);
+    c->L->le_faces(c->b, false, false, c->stream);
     HIP_TRY(hipGetLastError());
     const size_t plane = (size_t)c->p.ny * c->p.nz;
     const size_t n = 2 * 2 * 19 * plane;
@@ -1409,20 +1407,10 @@ int lb3d_gpu_profile_steps(lb3d_ctx *c, int32_t nsteps, int32_t max_kernels, con
     HIP_TRY(hipEventRecord(t0, c->stream));
     for (int st = 0; st < nsteps; st++) {
         auto mark = [&](int k) { used[(size_t)st * K_COUNT + k] = 1; };
-        // as enqueue_step: the two-pass plan advances the Lees-Edwards state
-        // in its halo-plane kernels and collide, the one-pass plan launches
-        // k_le_neighbours
-        const bool merged = c->le && !c->plan.fused;
-        if (c->le) {
-            if (!merged) {
-                HIP_TRY(rec(st, K_LEN, true));
-                launch_le_neighbours(c, -1);
-                HIP_TRY(rec(st, K_LEN, false));
-                mark(K_LEN);
-            }
+        if (c->le) {  // as enqueue_step
             HIP_TRY(rec(st, K_LE6, true));
             ensure_edges(c);
-            c->L->le_faces(c->b, false, compact_edges(c), c->stream, merged ? -1 : LE_STATE_AS_IS);
+            c->L->le_faces(c->b, false, false, c->stream, -1);
             HIP_TRY(rec(st, K_LE6, false));
             mark(K_LE6);
         }
@@ -1434,10 +1422,11 @@ int lb3d_gpu_profile_steps(lb3d_ctx *c, int32_t nsteps, int32_t max_kernels, con
         }
         if (c->le) {
             HIP_TRY(rec(st, K_LE8, true));
-            c->L->le_faces(c->b, true, compact_edges(c), c->stream, merged ? -1 : LE_STATE_AS_IS);
+            c->L->le_faces(c->b, true, c->plan.fused, c->stream, -1);
             HIP_TRY(rec(st, K_LE8, false));
             mark(K_LE8);
         }
+        if (c->le) c->L->set_le_commit(-1);
         if (c->plan.fused) {
             HIP_TRY(rec(st, K_FUS, true));
             if (!c->L->fused(c->b, c->plan.tx, c->plan.ty, c->plan.lz, c->plan.stage, c->stream))
@@ -1452,14 +1441,13 @@ int lb3d_gpu_profile_steps(lb3d_ctx *c, int32_t nsteps, int32_t max_kernels, con
                 mark(K_DIP);
             }
             HIP_TRY(rec(st, K_COL, true));
-            if (merged) c->L->set_le_commit(-1);
             c->L->collide(c->b, c->stream);
-            if (merged) c->L->set_le_commit(LE_STATE_AS_IS);
             HIP_TRY(rec(st, K_COL, false));
             mark(K_COL);
         }
+        c->L->set_le_commit(LE_STATE_AS_IS);
         flip(c);
-        c->edges_ok = compact_edges(c);
+        c->edges_ok = true;
     }
     HIP_TRY(hipEventRecord(t1, c->stream));
     HIP_TRY(hipGetLastError());

@@ -19,6 +19,8 @@
 // entries hold psi(rho) - psi(rho0_c).
 #pragma once
 
+#include <type_traits>
+
 #include "lb3d_lattice.h"
 
 namespace lb3d {
@@ -100,7 +102,8 @@ __device__ __forceinline__ LEState le_advance(LEState s, int nz, int nt_set)
     s.shear_sum = s.shear_sum + s.shear_u;
     // lelo = mod(int(2.*shear_sum), nz): truncation, sign of the dividend
     long t = (long)(2.0 * s.shear_sum);
-    s.lelo = (int)(t % (long)nz);
+    // (a 64-bit remainder is a hundred instructions; the offset hardly ever needs it)
+    s.lelo = t == (long)(int)t ? (int)t % nz : (int)(t % (long)nz);
     double lf = 2.0 * s.shear_sum;
     s.lefrac = fabs(lf - trunc(lf));
     return s;
@@ -367,34 +370,51 @@ __device__ __forceinline__ void zou_he_planes(const Phys<R> &P, R (&n)[19], int 
 
 // Lees-Edwards edge columns: the populations of the x = nx-1 (col 0) and
 // x = 0 (col 1) sites in a compact site-major layout
-// edge[(col*ny*nz + z*ny + y)*38 + c*19 + i].  A site's 38 values share two
+// edge[((z*ny + y)*2 + col)*38 + c*19 + i].  A site's 38 values share two
 // or three cache lines, so the one lane of a row that writes them touches
-// those lines only, and the halo-plane kernels read them contiguously (in
-// the lattice layout each of them lies on its own cache line).
-template <typename T, typename R>
-__device__ __forceinline__ T *edge_site(T *edge, const Phys<R> &P, int col, uint32_t q)
+// those lines only, and the halo-plane kernels read them by whole sites (in
+// the lattice layout each of them lies on its own cache line).  The columns
+// alternate, so that all a wave writes is near one address.
+constexpr uint32_t EDGE_SITES = 2 * 38;  // values of both columns at one (y, z)
+template <typename T>
+__device__ __forceinline__ T *edge_site(T *edge, int col, uint32_t q)
 {
-    return edge + ((uint32_t)col * ((uint32_t)P.ny * (uint32_t)P.nz) + q) * 38u;
+    return edge + (q * EDGE_SITES + (uint32_t)col * 38u);
 }
 
-// Stores population (c, i) of an edge-column site into the compact layout
-// from the register that already holds it; e is null off the edge columns
-// (and when no edge buffer is given), so the other lanes store nothing.
+// Stores population (c, i) of an edge-column site from the register that
+// already holds it.  Buffer stores: the lanes off the edge columns have an
+// offset outside the buffer, which the hardware drops.  As a store under an
+// exec mask, each of the 38 was a branch in the middle of the relaxation, and
+// the FP32 one-pass step of 128^3 took 185 us instead of 171 (256x64x64 94 /
+// 88; FP64 128^3 327 / 320).
 template <typename R>
 struct EdgeSink {
-    R *e;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t off;
     __device__ __forceinline__ void operator()(int c, int i, R v) const
     {
-        if (e) e[c * 19 + i] = v;
+        const uint32_t o = off + (uint32_t)(c * 19 + i) * (uint32_t)sizeof(R);
+        if constexpr (sizeof(R) == 4) {
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, o, 0, 0);
+        } else {
+            typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), rsrc, o, 0, 0);
+        }
     }
 };
+// The site (x, y, z) of this lane; the lanes of a wave are in order of q, at
+// most 63 apart (each row has a lane at least).
 template <typename R>
 __device__ __forceinline__ EdgeSink<R> edge_sink(R *edge, const Phys<R> &P, int x, int y, int z)
 {
-    R *e = nullptr;
-    if (edge && (x == 0 || x == P.nx - 1))  // nx >= 2: a site is at most one column
-        e = edge_site(edge, P, x == 0 ? 1 : 0, (uint32_t)z * (uint32_t)P.ny + (uint32_t)y);
-    return EdgeSink<R>{e};
+    constexpr uint32_t BYTES = 64 * EDGE_SITES * (uint32_t)sizeof(R);
+    const uint32_t q = (uint32_t)z * (uint32_t)P.ny + (uint32_t)y;
+    const uint32_t q0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)q);
+    const uint32_t off = ((q - q0) * EDGE_SITES + (x == 0 ? 38u : 0u)) * (uint32_t)sizeof(R);
+    // nx >= 2: a site is in at most one column
+    return EdgeSink<R>{__builtin_amdgcn_make_buffer_rsrc(edge_site(edge, 0, q0), 0, (int)BYTES, 0x00027000),
+                       x == 0 || x == P.nx - 1 ? off : BYTES};
 }
 
 template <typename R, bool Dev, int C, bool LE, bool Rock = false, bool ZH = false, bool Flat = false>
@@ -445,11 +465,13 @@ __device__ __forceinline__ void moments_core(const Phys<R> &P, const R *__restri
             for (int i = 0; i < 19; i++)
 #pragma unroll
                 for (int c = 0; c < C; c++) rho[c] = rho[c] + n[c][i] * R(GD[i]);
-            const EdgeSink<R> es = edge_sink(edge, P, x, y, z);
+            if (x == 0 || x == P.nx - 1) {
+                R *e = edge_site(edge, x == 0 ? 1 : 0, (uint32_t)z * (uint32_t)P.ny + (uint32_t)y);
 #pragma unroll
-            for (int c = 0; c < C; c++)
+                for (int c = 0; c < C; c++)
 #pragma unroll
-                for (int i = 0; i < 19; i++) es(c, i, n[c][i]);
+                    for (int i = 0; i < 19; i++) e[c * 19 + i] = n[c][i];
+            }
             da[0] = da[1] = da[2] = R(0);
             return;
         }
@@ -528,7 +550,7 @@ __global__ __launch_bounds__(256) void k_moments(Phys<R> P, const R *__restrict_
 }
 
 // Fills the edge columns of the pre-advection halo planes from the
-// populations f (when no collide of the two-pass plan has written them).
+// populations f (when no step has written them).
 template <typename R>
 __global__ __launch_bounds__(256) void k_le_gather_edges(Phys<R> P, const R *__restrict__ f, R *__restrict__ edge_pc)
 {
@@ -538,7 +560,7 @@ __global__ __launch_bounds__(256) void k_le_gather_edges(Phys<R> P, const R *__r
     const uint32_t ci = t % 38u, q = (t / 38u) % plane, col = t / (38u * plane);
     const int y = (int)(q % (uint32_t)P.ny), z = (int)(q / (uint32_t)P.ny);
     const int x = col == 0 ? P.nx - 1 : 0;
-    edge_pc[t] = f[ci * P.ns + sidx(x, y, z, P.nx, P.ny)];
+    edge_site(edge_pc, (int)col, q)[ci] = f[ci * P.ns + sidx(x, y, z, P.nx, P.ny)];
 }
 
 // --------------------------------------------------------------------------
@@ -1306,8 +1328,12 @@ template <typename R, bool Dev, bool LE, int T, int SM>
 __global__ __launch_bounds__(T) void k_fused2(Phys<R> P, const R *__restrict__ f,
                                               const R *__restrict__ face_pc,
                                               const R *__restrict__ face_aux,
-                                              R *__restrict__ fout, int TX, int TY, int lz, uint32_t xg)
+                                              R *__restrict__ fout, int TX, int TY, int lz, uint32_t xg,
+                                              R *__restrict__ edge_pc, LEState *__restrict__ le_commit, int le_adv)
 {
+    // Lees-Edwards: the step's state replaces the stored one (see k_collide)
+    if constexpr (LE)
+        if (le_commit && blockIdx.x == 0 && threadIdx.x == 0) *le_commit = le_advance(*le_commit, P.nz, le_adv);
     constexpr int LP = fused2_sites(T);
     const int LX = TX + 2;
     const int NH = 2 * LX + 2 * TY;  // halo positions per plane
@@ -1526,15 +1552,22 @@ __global__ __launch_bounds__(T) void k_fused2(Phys<R> P, const R *__restrict__ f
             F[0][0] = (-(P.g_br * frb0)) * psr;
             F[0][1] = (-(P.g_br * frb1)) * psr;
             F[0][2] = (-(P.g_br * frb2)) * psr;
-            if constexpr (SM == 2)
-                bgk_site_g<R, Dev, 2, 2, true>(
-                    P,
-                    [&](int c, int i) __attribute__((always_inline)) {
-                        return pull<R, 2, LE>(f, face_pc, P, c, i, x, y, k);
-                    },
-                    F, x, y, k, sidx(x, y, k, P.nx, P.ny), fout);
+            const uint32_t sk = sidx(x, y, k, P.nx, P.ny);
+            auto relax = [&](auto sink) __attribute__((always_inline)) {
+                if constexpr (SM == 2)
+                    bgk_site_g<R, Dev, 2, 2, true>(
+                        P,
+                        [&](int c, int i) __attribute__((always_inline)) {
+                            return pull<R, 2, LE>(f, face_pc, P, c, i, x, y, k);
+                        },
+                        F, x, y, k, sk, fout, sink);
+                else
+                    bgk_site<R, Dev, 2, 2>(P, cur, F, x, y, k, sk, fout, sink);
+            };
+            if constexpr (LE)  // the edge columns' post-collision populations
+                relax(edge_sink(edge_pc, P, x, y, k));
             else
-                bgk_site<R, Dev, 2, 2>(P, cur, F, x, y, k, sidx(x, y, k, P.nx, P.ny), fout);
+                relax(NoSink());
         }
     }
 }
@@ -1786,19 +1819,28 @@ __global__ __launch_bounds__(TX *TY) void k_fused3(
 // populations (stage 6), written to face_pc.  Post = true: the sources are
 // the post-advection populations (pulled through face_pc, stage 8) and only
 // the halo moments are written to face_aux.
-template <typename R, bool Dev, bool Post>
-__device__ __forceinline__ R le_src(const Phys<R> &P, const R *__restrict__ f,
-                                    const R *__restrict__ face_pc, int c, int i, int x, int y, int z)
+// --------------------------------------------------------------------------
+
+// Streamed population (c, i) of an edge-column site (x = nx-1 for Low, x = 0
+// otherwise; y, z), as pull gives it: from the post-collision edge columns
+// where the source lies in the same column, the halo plane face_pc where it
+// lies outside, the lattice for the column next to it.
+template <typename R, bool Low>
+__device__ __forceinline__ R le_streamed(const Phys<R> &P, const R *__restrict__ f, const R *__restrict__ face_pc,
+                                         const R *__restrict__ edge, int c, int i, int y, int z)
 {
-    if constexpr (Post)
-        return pull<R, 2, true>(f, face_pc, P, c, i, x, y, z);
-    else
-        return f[((uint32_t)c * 19u + (uint32_t)i) * P.ns + sidx(x, y, z, P.nx, P.ny)];
+    const int ys = wrap1(y - CY[i], P.ny), zs = wrap1(z - CZ[i], P.nz);
+    const uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz, q = (uint32_t)zs * (uint32_t)P.ny + (uint32_t)ys;
+    if (CX[i] == 0) return edge_site(edge, Low ? 0 : 1, q)[c * 19 + i];
+    if (CX[i] == (Low ? -1 : 1)) return face_pc[((uint32_t)((Low ? 2 : 0) + c) * 19u + (uint32_t)i) * plane + q];
+    return f[((uint32_t)c * 19u + (uint32_t)i) * P.ns + sidx(Low ? P.nx - 2 : 1, ys, zs, P.nx, P.ny)];
 }
 
+// The velocity shift of an interpolated halo site n: df = rho_c*(feq(u -+ 2U) -
+// feq(u)), and whether a shifted population would be negative.
 template <typename R, bool Dev>
-__device__ __forceinline__ void le_correct(const Phys<R> &P, const LEState &L, R n[2][19],
-                                           const R base[2][19], bool low)
+__device__ __forceinline__ bool le_shift(const Phys<R> &P, const LEState &L, const R (&n)[2][19], R (&df)[2][19],
+                                         bool low)
 {
     // moments of the interpolated halo site
     R rN[2], p[2][3];
@@ -1838,7 +1880,6 @@ __device__ __forceinline__ void le_correct(const Phys<R> &P, const LEState &L, R
         boltz_dist<R>(P.bdist, ux, uy, uzs, R(0), R(0), R(0), b1);
         boltz_dist<R>(P.bdist, ux, uy, uz, R(0), R(0), R(0), b2);
     }
-    R df[2][19];
     bool neg = false;
 #pragma unroll
     for (int i = 0; i < 19; i++) {
@@ -1851,13 +1892,22 @@ __device__ __forceinline__ void le_correct(const Phys<R> &P, const LEState &L, R
             if (full < R(0)) neg = true;
         }
     }
+    return neg;
+}
+
+// n := the shifted site; where that would be negative, base(c, i) (the site
+// itself on the low plane, the finished low site on the high one) plus as
+// much of the shift as leaves every population positive.
+template <typename R, bool Dev, typename Base>
+__device__ __forceinline__ void le_finish(const Phys<R> &P, R (&n)[2][19], const R (&df)[2][19], bool neg, Base base)
+{
     if (neg) {
         bool allpos = true;
 #pragma unroll
         for (int c = 0; c < 2; c++)
 #pragma unroll
             for (int i = 0; i < 19; i++) {
-                R full = Dev ? (i < 18 ? P.wrho0_move[c] : P.wrho0_rest[c]) + base[c][i] : base[c][i];
+                R full = Dev ? (i < 18 ? P.wrho0_move[c] : P.wrho0_rest[c]) + base(c, i) : base(c, i);
                 if (!(full > R(0))) allpos = false;
             }
         R scale = R(0);
@@ -1867,7 +1917,7 @@ __device__ __forceinline__ void le_correct(const Phys<R> &P, const LEState &L, R
             for (int c = 0; c < 2; c++)
 #pragma unroll
                 for (int i = 0; i < 19; i++) {
-                    R full = Dev ? (i < 18 ? P.wrho0_move[c] : P.wrho0_rest[c]) + base[c][i] : base[c][i];
+                    R full = Dev ? (i < 18 ? P.wrho0_move[c] : P.wrho0_rest[c]) + base(c, i) : base(c, i);
                     R v = -df[c][i] / full;
                     if (first || v > scale) scale = v;
                     first = false;
@@ -1877,7 +1927,7 @@ __device__ __forceinline__ void le_correct(const Phys<R> &P, const LEState &L, R
 #pragma unroll
         for (int c = 0; c < 2; c++)
 #pragma unroll
-            for (int i = 0; i < 19; i++) n[c][i] = use ? base[c][i] + df[c][i] / scale : base[c][i];
+            for (int i = 0; i < 19; i++) n[c][i] = use ? base(c, i) + df[c][i] / scale : base(c, i);
     } else {
 #pragma unroll
         for (int c = 0; c < 2; c++)
@@ -1895,76 +1945,88 @@ __device__ __forceinline__ int wrapz1(int k, int n)
 
 // One work-group of 2 * LE_SITES threads serves LE_SITES halo columns
 // (y, z): its first wave builds the x = 0 plane's sites, the second the
-// x = nx+1 plane's, both interpolating at once; the high side's clamp then
-// reads the finished low site from LDS.
-constexpr int LE_SITES = 64;
-// Compact: the sources come from the edge columns (edge: the pre-advection
-// ones, or for Post the streamed ones) instead of the lattice.
+// x = nx+1 plane's.  Both interpolate and shift at once; only where a shifted
+// site of the high plane would be negative does it wait for the finished low
+// site (its clamp reads it from LDS).
+//
+// The sources come from the edge columns (edge: the pre-advection ones, or for
+// Post the streamed ones that the moments pass keeps).  Stream (Post, one-pass
+// plan): no pass has streamed the edge columns, so each site pulls its two
+// sources from the pre-advection columns (edge) and what lies next to them.
+// The planes are small (4,096 sites a side at 256x64x64): the kernel is a
+// chain of latencies, 5 us and its launch (FP64 8 us while the high side began
+// after the low one and the offset took a 64-bit remainder, now 7.5).  Reading
+// the sources as contiguous elements through LDS, whole lines a load, took
+// 0.6 us longer: the addresses of 76 elements cost more than their lines.
 // adv: LE_STATE_AS_IS, or the step's state is le_advance(*Lp, nz, adv) (the
-// collide of the step stores it; every block computes it alike)
-template <typename R, bool Dev, bool Post, bool Compact = false>
+// last kernel of the step stores it; every block computes it alike)
+constexpr int LE_SITES = 64;
+template <typename R, bool Dev, bool Post, bool Stream = false>
 __global__ __launch_bounds__(2 * LE_SITES) void k_le_faces(Phys<R> P, const LEState *__restrict__ Lp,
                                                            const R *__restrict__ f, R *__restrict__ face_pc,
                                                            R *__restrict__ face_aux,
                                                            const R *__restrict__ edge, int adv)
 {
-    __shared__ R lo_done[2][19][LE_SITES];  // the corrected low-plane sites
+    constexpr int ROW = 39;  // 38 values a site, padded against bank conflicts
+    __shared__ R sh[LE_SITES * ROW];  // the low sites, finished
     const uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz;
     const int j = threadIdx.x % LE_SITES;
     const bool low = threadIdx.x < LE_SITES;  // wave-uniform
-    const uint32_t t = blockIdx.x * LE_SITES + j;
+    const uint32_t t0 = blockIdx.x * LE_SITES, t = t0 + j;
     const bool live = t < plane;
     const LEState L = adv == LE_STATE_AS_IS ? *Lp : le_advance(*Lp, P.nz, adv);
     const int y = live ? (int)(t % (uint32_t)P.ny) : 0, z = live ? (int)(t / (uint32_t)P.ny) : 0;  // 0-based
     const int z1 = z + 1;                                                                           // 1-based
     const int lelo = L.lelo, bsh = lelo >= 0 ? 0 : -1;
     const R fr = R(L.lefrac), omf = R(1.0) - R(L.lefrac);
-    R n[2][19];
+    R n[2][19], df[2][19];
+    bool neg = false;
+    // low (x=0):    (1-f) N(nx, y, z+lelo+b) + f N(nx, y, z+lelo+1+b)
+    // high (x=nx+1): f N(1, y, z-lelo-1-b)   + (1-f) N(1, y, z-lelo-b)
     if (live) {
-        // low (x=0):    (1-f) N(nx, y, z+lelo+b) + f N(nx, y, z+lelo+1+b)
-        // high (x=nx+1): f N(1, y, z-lelo-1-b)   + (1-f) N(1, y, z-lelo-b)
-        const int xs = low ? P.nx - 1 : 0;
-        const int za = low ? wrapz1(z1 + lelo + bsh, P.nz) : wrapz1(z1 - lelo - 1 - bsh, P.nz);
-        const int zb = low ? wrapz1(z1 + lelo + 1 + bsh, P.nz) : wrapz1(z1 - lelo - bsh, P.nz);
-        const R wa = low ? omf : fr, wb = low ? fr : omf;
-        const int col = low ? 0 : 1;
-        const uint32_t qa = (uint32_t)za * (uint32_t)P.ny + (uint32_t)y, qb = (uint32_t)zb * (uint32_t)P.ny + (uint32_t)y;
+        // the two sources of the site, z planes za and zb
+        auto pull2 = [&](auto side, int za, int zb, R wa, R wb) __attribute__((always_inline)) {
+            constexpr bool lo = decltype(side)::value;
+            R a[2][19], b[2][19];
+            const R *ea = edge_site(edge, lo ? 0 : 1, (uint32_t)za * (uint32_t)P.ny + (uint32_t)y);
+            const R *eb = edge_site(edge, lo ? 0 : 1, (uint32_t)zb * (uint32_t)P.ny + (uint32_t)y);
 #pragma unroll
-        for (int c = 0; c < 2; c++)
+            for (int c = 0; c < 2; c++)
 #pragma unroll
-            for (int i = 0; i < 19; i++) {
-                R a, b;
-                if constexpr (Compact) {
-                    a = edge_site(edge, P, col, qa)[c * 19 + i];
-                    b = edge_site(edge, P, col, qb)[c * 19 + i];
-                } else {
-                    a = le_src<R, Dev, Post>(P, f, face_pc, c, i, xs, y, za);
-                    b = le_src<R, Dev, Post>(P, f, face_pc, c, i, xs, y, zb);
+                for (int i = 0; i < 19; i++) {
+                    a[c][i] = Stream ? le_streamed<R, lo>(P, f, face_pc, edge, c, i, y, za) : ea[c * 19 + i];
+                    b[c][i] = Stream ? le_streamed<R, lo>(P, f, face_pc, edge, c, i, y, zb) : eb[c * 19 + i];
                 }
-                n[c][i] = wa * a + wb * b;
-            }
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int i = 0; i < 19; i++) n[c][i] = wa * a[c][i] + wb * b[c][i];
+        };
+        if (low)
+            pull2(std::true_type{}, wrapz1(z1 + lelo + bsh, P.nz), wrapz1(z1 + lelo + 1 + bsh, P.nz), omf, fr);
+        else
+            pull2(std::false_type{}, wrapz1(z1 - lelo - 1 - bsh, P.nz), wrapz1(z1 - lelo - bsh, P.nz), fr, omf);
+        neg = le_shift<R, Dev>(P, L, n, df, low);
         if (low) {
+            // (le_finish's base is the site itself, which it overwrites last)
+            R *done = sh + j * ROW;
             R base[2][19];
 #pragma unroll
             for (int c = 0; c < 2; c++)
 #pragma unroll
                 for (int i = 0; i < 19; i++) base[c][i] = n[c][i];
-            le_correct<R, Dev>(P, L, n, base, true);
+            le_finish<R, Dev>(P, n, df, neg, [&](int c, int i) __attribute__((always_inline)) { return base[c][i]; });
 #pragma unroll
             for (int c = 0; c < 2; c++)
 #pragma unroll
-                for (int i = 0; i < 19; i++) lo_done[c][i][j] = n[c][i];
+                for (int i = 0; i < 19; i++) done[c * 19 + i] = n[c][i];
         }
     }
     __syncthreads();
     if (!live) return;
     if (!low) {
-        R base[2][19];
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-            for (int i = 0; i < 19; i++) base[c][i] = lo_done[c][i][j];
-        le_correct<R, Dev>(P, L, n, base, false);
+        const R *done = sh + j * ROW;
+        le_finish<R, Dev>(P, n, df, neg, [&](int c, int i) __attribute__((always_inline)) { return done[c * 19 + i]; });
     }
     const int fc = low ? 0 : 1;
     if constexpr (!Post) {

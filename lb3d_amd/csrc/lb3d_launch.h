@@ -369,22 +369,20 @@ class LauncherT : public Launcher {
         else
             n ? collide_bd<BD_GENERAL, true>(b, s) : collide_bd<BD_GENERAL, false>(b, s);
     }
-    void le_faces(const DevBufs &b, bool post, bool compact, hipStream_t s, int adv) override
+    void le_faces(const DevBufs &b, bool post, bool stream, hipStream_t s, int adv) override
     {
         unsigned plane = (unsigned)P.ny * (unsigned)P.nz;
         unsigned nb = (plane + LE_SITES - 1) / LE_SITES;
-        const R *f = (const R *)b.f[b.cur];
+        const R *f = (const R *)b.f[b.cur], *pc = (const R *)b.edge_pc;
         R *fp = (R *)b.face_pc, *fa = (R *)b.face_aux;
-        if (post && compact)
-            k_le_faces<R, Dev, true, true><<<nb, 2 * LE_SITES, 0, s>>>(P, b.le, f, fp, fa, (const R *)b.edge_adv, adv);
-        else if (post)
-            k_le_faces<R, Dev, true><<<nb, 2 * LE_SITES, 0, s>>>(P, b.le, f, fp, fa, nullptr, adv);
-        else if (compact)
-            k_le_faces<R, Dev, false, true><<<nb, 2 * LE_SITES, 0, s>>>(P, b.le, f, fp, fa, (const R *)b.edge_pc, adv);
+        if (!post)
+            k_le_faces<R, Dev, false><<<nb, 2 * LE_SITES, 0, s>>>(P, b.le, f, fp, fa, pc, adv);
+        else if (stream)
+            k_le_faces<R, Dev, true, true><<<nb, 2 * LE_SITES, 0, s>>>(P, b.le, f, fp, fa, pc, adv);
         else
-            k_le_faces<R, Dev, false><<<nb, 2 * LE_SITES, 0, s>>>(P, b.le, f, fp, fa, nullptr, adv);
+            k_le_faces<R, Dev, true><<<nb, 2 * LE_SITES, 0, s>>>(P, b.le, f, fp, fa, (const R *)b.edge_adv, adv);
     }
-    // the next two-pass collide stores le_advance(state, adv) unless adv is
+    // the next collide or one-pass step stores le_advance(state, adv) unless adv is
     // LE_STATE_AS_IS (then it leaves the state alone)
     int le_commit = LE_STATE_AS_IS;
     void set_le_commit(int adv) override { le_commit = adv; }
@@ -424,10 +422,12 @@ class LauncherT : public Launcher {
         const R *f = (const R *)b.f[b.cur];
         R *fo = (R *)b.f[1 - b.cur];
         if (le)
-            k_fused2<R, Dev, true, T, SM><<<grid, T, 0, s>>>(P, f, (const R *)b.face_pc, (const R *)b.face_aux, fo,
-                                                              tx, ty, lz, xg);
+            k_fused2<R, Dev, true, T, SM><<<grid, T, 0, s>>>(
+                P, f, (const R *)b.face_pc, (const R *)b.face_aux, fo, tx, ty, lz, xg, (R *)b.edge_pc,
+                le_commit == LE_STATE_AS_IS ? nullptr : b.le, le_commit);
         else
-            k_fused2<R, Dev, false, T, SM><<<grid, T, 0, s>>>(P, f, nullptr, nullptr, fo, tx, ty, lz, xg);
+            k_fused2<R, Dev, false, T, SM><<<grid, T, 0, s>>>(P, f, nullptr, nullptr, fo, tx, ty, lz, xg, nullptr,
+                                                               nullptr, LE_STATE_AS_IS);
     }
     // LDS of k_fused3: its rings of moments, psi and dipoles
     template <int TX, int TY>

@@ -70,13 +70,14 @@ class Launcher {
     virtual void moments(const DevBufs &b, hipStream_t s) = 0;
     virtual void dipole(const DevBufs &b, hipStream_t s) = 0;
     virtual void collide(const DevBufs &b, hipStream_t s) = 0;  // f[cur] -> f[1-cur]
-    // Lees-Edwards x-halo planes, pre- (post = false) or post-advection;
-    // compact: from the edge columns (b.edge_pc written by the two-pass
-    // collide or le_gather_edges, b.edge_adv by the moments pass)
+    // Lees-Edwards x-halo planes, pre- (post = false) or post-advection, from
+    // the edge columns b.edge_pc (written by the step's last kernel or
+    // le_gather_edges); post-advection from the streamed ones b.edge_adv that
+    // the moments pass has written, or (stream) by streaming b.edge_pc
     // adv: LE_STATE_AS_IS, or the halo-plane kernels compute the step's state
     // from the stored one (le_advance with nt_set = adv) and the next collide
     // stores it (set_le_commit)
-    virtual void le_faces(const DevBufs &b, bool post, bool compact, hipStream_t s, int adv = LE_STATE_AS_IS) = 0;
+    virtual void le_faces(const DevBufs &b, bool post, bool stream, hipStream_t s, int adv = LE_STATE_AS_IS) = 0;
     virtual void set_le_commit(int adv) = 0;
     // b.edge_pc from the populations f[cur]
     virtual void le_gather_edges(const DevBufs &b, hipStream_t s) = 0;

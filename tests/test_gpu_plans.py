@@ -305,6 +305,35 @@ def test_untuned_one_pass_plan_equals_two_pass_bitwise(precision, dims):
     assert np.array_equal(got, want), f"max {np.abs(got - want).max()}"
 
 
+@pytest.mark.parametrize("precision,dims", [
+    (LB3D_FP64, (2, 700, 401)),         # both edge columns in every row, 32 rows to a wave
+    (LB3D_FP64, (97, 83, 75)),
+    (LB3D_FP64, (333, 1511, 1)),        # one plane: every z offset wraps onto it
+    (LB3D_FP32_DEV, (256, 80, 75)),
+    (LB3D_FP32_DEV, (3, 1001, 501)),    # the columns next to the edges coincide
+])
+def test_untuned_lees_edwards_one_pass_plan_equals_two_pass_bitwise(precision, dims):
+    """The one-pass step writes the edge columns and the offset state that the
+    next step's halo planes read; staged steps (whose halo planes take the
+    state as it is) alternate with whole ones."""
+    states = []
+    for two_pass in (True, False):
+        g = Lattice(*dims, ncomp=2, precision=precision, g_br=0.09, boundary=LB3D_BC_LEES_EDWARDS, shear_u=0.07)
+        g.init_noise(5, amp=(0.3, 0.3, 0.0))
+        if two_pass:
+            g.set_plan(0)
+        g.bc_init()
+        g.time_loop(5)
+        g.time_step()
+        g.time_loop(3)
+        assert ("fused" in g.profile_steps(2)[0]) is not two_pass
+        g.time_step()
+        states.append(g.populations())
+        g.close()
+    assert np.isfinite(states[0]).all()
+    assert np.array_equal(*states), f"max {np.abs(states[0] - states[1]).max()}"
+
+
 @pytest.mark.parametrize("kw", [
     dict(ncomp=2), dict(ncomp=3, precision=LB3D_FP32_DEV),
     dict(ncomp=2, boundary=LB3D_BC_LEES_EDWARDS, shear_u=0.04),

@@ -1168,7 +1168,8 @@ __device__ __forceinline__ void bgk_site(const Phys<R> &P, const R (&n)[C][19], 
 // --------------------------------------------------------------------------
 // k_collide: pull, Shan-Chen forces from the aux field, BGK; the second pass
 // of the two-pass step (k_moments then k_collide).
-// NT: bit 0 loads, bit 1 stores the populations with the non-temporal hint
+// NT: bit 0 loads, bit 1 stores the populations with the non-temporal hint; bit
+// 2 pulls before the forces
 template <typename R, bool Dev, int C, bool LE, int BD, bool Rock = false, bool ZH = false, int NT = 0,
           bool PK = false>
 __device__ __forceinline__ void collide_site(const Phys<R> &P, const R *__restrict__ f,
@@ -1198,15 +1199,25 @@ __device__ __forceinline__ void collide_site(const Phys<R> &P, const R *__restri
 #pragma unroll
             for (int c = 0; c < C; c++) n[c][i] = pull_rock<R, C>(f, bits, P, c, i, x, y, z);
     } else {
-        // the force stencil first, then the pulls (a compiler barrier keeps
+        // NT & 4: the pulls first, in flight together with the stencil's loads.
+        // Otherwise the force stencil, then the pulls (a compiler barrier keeps
         // them after it): the populations are not live while the stencil's
         // loads are in flight, which leaves the registers to batch those loads
+        auto pulls = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 19; i++)
+#pragma unroll
+                for (int c = 0; c < C; c++) n[c][i] = pull<R, C, LE, (NT & 1) != 0>(f, face_pc, P, c, i, x, y, z);
+        };
+        if constexpr ((NT & 4) != 0) {
+            pulls();
+            __builtin_amdgcn_sched_barrier(0);
+        }
         sc_forces<R, Dev, C, LE, PK>(P, aux, face_aux, db, x, y, z, s, F);
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int i = 0; i < 19; i++)
-#pragma unroll
-            for (int c = 0; c < C; c++) n[c][i] = pull<R, C, LE, (NT & 1) != 0>(f, face_pc, P, c, i, x, y, z);
+        if constexpr ((NT & 4) == 0) {
+            asm volatile("" ::: "memory");
+            pulls();
+        }
     }
     if constexpr (ZH) {
         if (z == 0 || z == P.nz - 1) {
@@ -1258,7 +1269,13 @@ __global__ __launch_bounds__(256) void k_collide(Phys<R> P, const R *__restrict_
     if (s >= P.ns) return;
     // measured on MI355X (FP32 and FP64): ternary loads and stores (128^3:
     // -6 to -8% per step), binary stores only (256^3 FP64: -2%)
-    constexpr int nt = !NT ? 0 : (C == 3 ? 3 : 2);
+    // Pulls before the forces (bit 2) where it measured faster, per two-pass step:
+    // binary FP32 64^3 22.1 -> 21.5 us, 112^3 133 -> 129, FP64 48^3 20.3 -> 18.9,
+    // 80^3 92 -> 89; ternary FP64 56^3 64 -> 61, 64^3 90 -> 83.  Ternary FP32
+    // (112^3 261 -> 270 us) and lattices beyond the memory-side cache (ternary
+    // FP64 128^3 731 -> 752) have more from the registers that the forces have
+    // to themselves.
+    constexpr int nt = !NT ? (C == 2 || !Dev ? 4 : 0) : (C == 3 ? 3 : 2);
     collide_site<R, Dev, C, LE, BD, Rock, ZH, nt>(P, f, face_pc, aux, face_aux, db, fout, s, rock, edge_pc);
 }
 

@@ -14,6 +14,7 @@ void step_buffers_fp64(const lb3d_params &p, const DevBufs &b, hipStream_t s)
     L.xg = q.xg;
     if (q.fused && L.fused(b, q.tx, q.ty, q.lz, q.stage, s)) return;
     L.moments(b, s);
+    if (L.dipole_collide(b, s)) return;
     L.dipole(b, s);
     L.collide(b, s);
 }

@@ -60,8 +60,9 @@ struct Events {
 };
 
 const char *const KNAMES[] = {"le_faces_pc", "moments",
-                              "le_faces_aux",  "dipole",      "collide", "fused"};
-enum { K_LE6 = 0, K_MOM, K_LE8, K_DIP, K_COL, K_FUS, K_COUNT };
+                              "le_faces_aux",  "dipole",      "collide", "fused",
+                              "dipole_collide"};
+enum { K_LE6 = 0, K_MOM, K_LE8, K_DIP, K_COL, K_FUS, K_DC, K_COUNT };
 
 const char *const STAGE_NAMES[3] = {"regs", "lds", "reload"};
 
@@ -781,7 +782,7 @@ static int launch_collision(lb3d_ctx *c)
     if (c->plan.fused) {
         if (!c->L->fused(c->b, c->plan.tx, c->plan.ty, c->plan.lz, c->plan.stage, c->stream))
             return fail(LB3D_EINVAL, "the one-pass plan has no kernel for this lattice");
-    } else {
+    } else if (!c->L->dipole_collide(c->b, c->stream)) {
         c->L->dipole(c->b, c->stream);
         c->L->collide(c->b, c->stream);
     }
@@ -1433,6 +1434,11 @@ int lb3d_gpu_profile_steps(lb3d_ctx *c, int32_t nsteps, int32_t max_kernels, con
                 return fail(LB3D_EINVAL, "the one-pass plan has no kernel for this lattice");
             HIP_TRY(rec(st, K_FUS, false));
             mark(K_FUS);
+        } else if (c->L->small()) {
+            HIP_TRY(rec(st, K_DC, true));
+            c->L->dipole_collide(c->b, c->stream);
+            HIP_TRY(rec(st, K_DC, false));
+            mark(K_DC);
         } else {
             if (c->p.ncomp == 3) {
                 HIP_TRY(rec(st, K_DIP, true));

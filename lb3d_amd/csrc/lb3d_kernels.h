@@ -696,12 +696,11 @@ __device__ __forceinline__ void dipole_core(const Phys<R> &P, R hs0, R hs1, R hs
     out[2] = P.omega_d * e2 + P.one_m_omega_d * sd2;
 }
 
+// The relaxed dipole of site s = (x, y, z).
 template <typename R, bool Dev, bool PK = false>
-__device__ __forceinline__ void dipole_site(const Phys<R> &P, const R *__restrict__ aux,
-                                            R *__restrict__ db, uint32_t s)
+__device__ __forceinline__ void dipole_new(const Phys<R> &P, const R *__restrict__ aux, int x, int y, int z,
+                                           uint32_t s, R (&out)[3])
 {
-    int x, y, z;
-    site_xyz(s, P.nx, P.ny, x, y, z);
     const V4<R> *vec = (const V4<R> *)(aux + aux3_vec_off(P.ns));
     // the 18 neighbours' (rho_b - rho_r, da): one vector load each, at a
     // 32-bit byte offset from the field's base (16 ns bytes < 4 GiB for any
@@ -711,7 +710,6 @@ __device__ __forceinline__ void dipole_site(const Phys<R> &P, const R *__restric
     for (int i = 0; i < 18; i++)
         nb[i] = ld_plane(vec, sidx(wrap1(x + CX[i], P.nx), wrap1(y + CY[i], P.ny), wrap1(z + CZ[i], P.nz), P.nx, P.ny));
     const V4<R> own = ld_plane(vec, s);
-    R out[3];
     dipole_core<R, Dev>(
         P, own.b, own.c, own.d, PK ? ld_plane((const V4<R> *)aux, s).d : ld_plane(plane_of(aux, 5u, P.ns), s),
         [&](int i) __attribute__((always_inline)) { return nb[i].a; },
@@ -719,6 +717,16 @@ __device__ __forceinline__ void dipole_site(const Phys<R> &P, const R *__restric
             return a == 0 ? nb[i].b : (a == 1 ? nb[i].c : nb[i].d);
         },
         out);
+}
+
+template <typename R, bool Dev, bool PK = false>
+__device__ __forceinline__ void dipole_site(const Phys<R> &P, const R *__restrict__ aux,
+                                            R *__restrict__ db, uint32_t s)
+{
+    int x, y, z;
+    site_xyz(s, P.nx, P.ny, x, y, z);
+    R out[3];
+    dipole_new<R, Dev, PK>(P, aux, x, y, z, s, out);
     st_plane(db, s, out[0]);
     st_plane(db + (size_t)P.ns, s, out[1]);
     st_plane(db + (size_t)2 * P.ns, s, out[2]);
@@ -1277,6 +1285,65 @@ __global__ __launch_bounds__(256) void k_collide(Phys<R> P, const R *__restrict_
     // to themselves.
     constexpr int nt = !NT ? (C == 2 || !Dev ? 4 : 0) : (C == 3 ? 3 : 2);
     collide_site<R, Dev, C, LE, BD, Rock, ZH, nt>(P, f, face_pc, aux, face_aux, db, fout, s, rock, edge_pc);
+}
+
+// --------------------------------------------------------------------------
+// k_dipole_collide: the dipole relaxation and the collision of a ternary
+// lattice of few sites in one launch.  There each kernel is a launch and a
+// chain of latencies with most CUs idle, so the work-group relaxes the dipoles
+// of its DC_X x DC_Y x DC_Z sites and of the halo around them (240 for 64
+// sites, one a thread), keeps them and their psi in LDS, and has the
+// populations in flight while it sums the forces from there.
+constexpr int DC_X = 8, DC_Y = 4, DC_Z = 2, DC_THREADS = 256;
+template <typename R, bool Dev, int BD>
+__global__ __launch_bounds__(DC_THREADS) void k_dipole_collide(Phys<R> P, const R *__restrict__ f,
+                                                               const R *__restrict__ aux, R *__restrict__ db,
+                                                               R *__restrict__ fout, uint32_t tx, uint32_t ty)
+{
+    constexpr int HX = DC_X + 2, HY = DC_Y + 2, HZ = DC_Z + 2, NH = HX * HY * HZ;
+    static_assert(NH <= DC_THREADS && DC_X * DC_Y * DC_Z <= DC_THREADS);
+    __shared__ R sdb[3][NH], spsi[3][NH];
+    const int t = threadIdx.x;
+    const int x0 = (int)(blockIdx.x % tx) * DC_X, y0 = (int)(blockIdx.x / tx % ty) * DC_Y,
+              z0 = (int)(blockIdx.x / (tx * ty)) * DC_Z;
+    if (t < NH) {
+        const int hx = t % HX, hy = t / HX % HY, hz = t / (HX * HY);
+        // beyond the first halo site of a tile that the lattice does not fill, any site will do
+        auto wrapped = [](int v, int n) { return v < 0 ? n - 1 : (v >= n ? 0 : v); };
+        const int x = wrapped(x0 + hx - 1, P.nx), y = wrapped(y0 + hy - 1, P.ny), z = wrapped(z0 + hz - 1, P.nz);
+        const bool own = hx > 0 && hx <= DC_X && hy > 0 && hy <= DC_Y && hz > 0 && hz <= DC_Z &&
+                         x0 + hx <= P.nx && y0 + hy <= P.ny && z0 + hz <= P.nz;
+        const uint32_t s = sidx(x, y, z, P.nx, P.ny);
+        R out[3];
+        dipole_new<R, Dev>(P, aux, x, y, z, s, out);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            sdb[k][t] = out[k];
+            spsi[k][t] = ld_plane(plane_of(aux, (uint32_t)k, P.ns), s);
+            if (own) st_plane(db + (size_t)k * P.ns, s, out[k]);
+        }
+    }
+    const int sx = t % DC_X, sy = t / DC_X % DC_Y, sz = t / (DC_X * DC_Y);
+    const int x = x0 + sx, y = y0 + sy, z = z0 + sz;
+    const bool site = sz < DC_Z && x < P.nx && y < P.ny && z < P.nz;
+    R n[3][19];
+    if (site) {
+#pragma unroll
+        for (int i = 0; i < 19; i++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) n[c][i] = pull<R, 3, false>(f, nullptr, P, c, i, x, y, z);
+    }
+    __syncthreads();
+    if (!site) return;
+    const int h = ((sz + 1) * HY + sy + 1) * HX + sx + 1;
+    const R dbx[3] = {sdb[0][h], sdb[1][h], sdb[2][h]}, ps_own[3] = {spsi[0][h], spsi[1][h], spsi[2][h]};
+    R F[3][3];
+    sc_forces3<R, Dev>(
+        P, dbx, ps_own,
+        [&](int i, int c) __attribute__((always_inline)) { return spsi[c][h + (CZ[i] * HY + CY[i]) * HX + CX[i]]; },
+        [&](int i, int a) __attribute__((always_inline)) { return sdb[a][h + (CZ[i] * HY + CY[i]) * HX + CX[i]]; },
+        F);
+    bgk_site<R, Dev, 3, BD>(P, n, F, x, y, z, sidx(x, y, z, P.nx, P.ny), fout);
 }
 
 // --------------------------------------------------------------------------

@@ -68,6 +68,10 @@ class Launcher {
     uint32_t xg = 0;
     bool walls = false;  // the lattice has rock sites (the one-pass plans are then unavailable)
     virtual void moments(const DevBufs &b, hipStream_t s) = 0;
+    // dipole and collide in one launch, for lattices of few sites (small());
+    // false: not done
+    virtual bool small() const = 0;
+    virtual bool dipole_collide(const DevBufs &b, hipStream_t s) = 0;
     virtual void dipole(const DevBufs &b, hipStream_t s) = 0;
     virtual void collide(const DevBufs &b, hipStream_t s) = 0;  // f[cur] -> f[1-cur]
     // Lees-Edwards x-halo planes, pre- (post = false) or post-advection, from

@@ -237,3 +237,29 @@ def test_long_batch_runs_replay_a_graph_bitwise():
             b.set_groups(0)  # drops the plan's graph: b stays on single launches
     for k in range(2):
         assert np.array_equal(a.populations(k), b.populations(k))
+
+
+@pytest.mark.parametrize("precision,dims", [
+    (p, d) for p, most in ((LB3D_FP64, 5000), (LB3D_FP32_DEV, 10000))
+    for d in [(2, 1, 1), (8, 4, 2), (9, 5, 3), (7, 3, 1), (17, 13, 11), (3, 40, 41), (625, 8, 1), (25, 20, 20)]
+    if d[0] * d[1] * d[2] <= most])
+@pytest.mark.parametrize("bdist", [0, 2, 1])
+def test_small_ternary_lattice_in_two_launches_equals_three_kernels_bitwise(precision, dims, bdist):
+    """A small ternary lattice relaxes dipoles and populations in one launch,
+    by tiles of 8 x 4 x 2 sites that overhang it; the batch's lattice by
+    lattice plan runs the kernels one by one."""
+    kw = dict(ncomp=3, precision=precision, bdist=bdist, g_br=0.08, g_bs=-0.006, g_ss=-0.003)
+    b = Batch([dims], **kw)
+    b.set_plan(1)
+    b.init_noise(0, 3, amp=(0.05, 0.05, 0.05))
+    b.time_loop(7)
+    g = Lattice(*dims, **kw)
+    g.init_noise(3, amp=(0.05, 0.05, 0.05))
+    g.bc_init()
+    g.time_loop(5)
+    g.time_step()
+    names = list(g.profile_steps(1)[0])
+    assert names == ["moments", "dipole_collide"]
+    got = g.populations()
+    assert np.isfinite(got).all()
+    np.testing.assert_array_equal(got, b.populations(0))

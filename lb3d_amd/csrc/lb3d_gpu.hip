@@ -237,8 +237,8 @@ void io_users(int change)
 //         128^3 386 / 300, 256^3 3170 / 2390.
 // So the lines lie at 0.6 and 0.4 million sites.  Lees-Edwards, whose one-pass
 // plan streams the edge columns once more for the post-advection halo planes:
-//   FP32  96^3 89 / 95, 110x88x112 126 / 130, 256x64x64 112 / 107, 89x135x140
-//         212 / 201, 128^3 222 / 200, 107x246x103 347 / 283, 192^3 689 / 601;
+//   FP32  100^3 109 / 116, 256x64x64 101 / 103, 134x90x104 140 / 153, 89x135x140
+//         216 / 193, 128^3 224 / 191, 160^3 424 / 389, 192^3 690 / 599;
 //   FP64  140x41x93 126 / 122, 60x84x111 134 / 128, 96^3 187 / 181, 256x64x64
 //         223 / 194, 128^3 421 / 358, 160^3 840 / 775:
 // 1.5 and 0.5 million sites.
@@ -251,7 +251,8 @@ void io_users(int change)
 // 32x16 65, 90x100x77: 90x5 47 us, 30x17 58).  FP64 planes do not fit the L2
 // with their halos, so there the halo sites count too (256^3: 64x8 2.39 ms,
 // 128x4 2.49, 256x2 2.62; 200^3: 100x5 1.24 ms, 50x10 1.31); and with
-// Lees-Edwards (256x64x64 FP32: 64x8 95 us, 128x4 103, 256x2 106).
+// Lees-Edwards (256x64x64 FP32: 64x8 95 us, 128x4 103, 256x2 106; not below
+// 48 columns there: 134x90x104 in 34x15 took 1.17 of the two-pass step).
 //
 // z-chunk: the work-groups run in rounds of 256 (one per CU), each lz + 2
 // planes long; the fewest planes in a row win (200^3 FP32: 240 work-groups of
@@ -282,7 +283,7 @@ Plan default_plan(const lb3d_params &p)
     double best = 0.0;
     for (int kx = 1; kx <= p.nx; kx++) {
         const int tx = (p.nx + kx - 1) / kx;
-        if (tx < 16 && kx > 1) break;
+        if (tx < (le && !fp64 ? 48 : 16) && kx > 1) break;
         int ty = T / tx < p.ny ? T / tx : p.ny;
         if (ty > fused2_sites(T) / (tx + 2) - 2) ty = fused2_sites(T) / (tx + 2) - 2;
         if (ty < 1) continue;
@@ -747,6 +748,7 @@ int lb3d_gpu_bc_apply(lb3d_ctx *c, int32_t stage, int32_t nt)
     } else if (stage == 8) {
         if (c->state != AFTER_ADV) return fail(LB3D_ESTATE, "bc_apply(8) must follow advection");
         if (c->le) {
+            ensure_edges(c);  // (the plan may have changed within the step)
             c->L->le_faces(c->b, true, c->plan.fused, c->stream);
             HIP_TRY(hipGetLastError());
         }

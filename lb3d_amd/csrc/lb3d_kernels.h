@@ -368,18 +368,32 @@ __device__ __forceinline__ void zou_he_planes(const Phys<R> &P, R (&n)[19], int 
     if (z == P.nz - 1) zou_he_site<R, Dev>(n, P.zh_flux[c], P.zh_type, false, P.rho0[c]);
 }
 
-// Lees-Edwards edge columns: the populations of the x = nx-1 (col 0) and
-// x = 0 (col 1) sites in a compact site-major layout
-// edge[((z*ny + y)*2 + col)*38 + c*19 + i].  A site's 38 values share two
-// or three cache lines, so the one lane of a row that writes them touches
-// those lines only, and the halo-plane kernels read them by whole sites (in
-// the lattice layout each of them lies on its own cache line).  The columns
-// alternate, so that all a wave writes is near one address.
-constexpr uint32_t EDGE_SITES = 2 * 38;  // values of both columns at one (y, z)
+// Lees-Edwards edge columns: for each (y, z), the 38 populations c*19 + i of
+// the x = nx-1 (col 0) and of the x = 0 (col 1) site, and the 10 of the site
+// next to each that move into it (c*5 + the direction's rank among those of
+// its c_x; the one-pass plan's post-advection halo planes stream them).  A
+// site's values share two or three cache lines, so the one lane of a row that
+// writes them touches those lines only, and the halo-plane kernels read them
+// by whole sites (in the lattice layout each lies on its own cache line).
+// All of a (y, z) is together, so that all a wave writes is near one address.
+constexpr uint32_t EDGE_IN = 2 * 38, EDGE_SITES = EDGE_IN + 2 * 10;  // values of a (y, z)
 template <typename T>
 __device__ __forceinline__ T *edge_site(T *edge, int col, uint32_t q)
 {
     return edge + (q * EDGE_SITES + (uint32_t)col * 38u);
+}
+// the place of an incoming population, c_x(i) != 0, after the 38s: column 0's
+// come with c_x = 1, column 1's with c_x = -1.  The FP32 one-pass plan keeps
+// them (EDGES_IN): its halo planes' streaming takes 12.8 us at 128^3 instead of
+// 23, its step 193 instead of 201.  In FP64 the selects cost the kernel its
+// registers (256x64x64 166 -> 194 us), so the lattice is read.
+template <typename R>
+constexpr bool EDGES_IN = sizeof(R) == 4;
+constexpr uint32_t edge_in_at(int c, int i)
+{
+    uint32_t rank = 0;
+    for (int k = 0; k < i; k++) rank += CX[k] == CX[i] ? 1u : 0u;
+    return EDGE_IN + (CX[i] > 0 ? 0u : 10u) + (uint32_t)c * 5u + rank;
 }
 
 // Stores population (c, i) of an edge-column site from the register that
@@ -388,13 +402,17 @@ __device__ __forceinline__ T *edge_site(T *edge, int col, uint32_t q)
 // exec mask, each of the 38 was a branch in the middle of the relaxation, and
 // the FP32 one-pass step of 128^3 took 185 us instead of 171 (256x64x64 94 /
 // 88; FP64 128^3 327 / 320).
-template <typename R>
+// In: the incoming populations too, from the sites next to the edge columns,
+// in the same stores.
+template <typename R, bool In>
 struct EdgeSink {
     __amdgpu_buffer_rsrc_t rsrc;
-    uint32_t off;
+    uint32_t off[In ? 3 : 1];  // In: by c_x + 1; of the lane's column, of its (y, z) alone, or outside
+    bool in;                   // the site is next to an edge column
     __device__ __forceinline__ void operator()(int c, int i, R v) const
     {
-        const uint32_t o = off + (uint32_t)(c * 19 + i) * (uint32_t)sizeof(R);
+        uint32_t o = off[In ? CX[i] + 1 : 0] + (uint32_t)(c * 19 + i) * (uint32_t)sizeof(R);
+        if (In && CX[i] != 0) o = in ? off[In ? CX[i] + 1 : 0] + edge_in_at(c, i) * (uint32_t)sizeof(R) : o;
         if constexpr (sizeof(R) == 4) {
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, o, 0, 0);
         } else {
@@ -405,16 +423,26 @@ struct EdgeSink {
 };
 // The site (x, y, z) of this lane; the lanes of a wave are in order of q, at
 // most 63 apart (each row has a lane at least).
-template <typename R>
-__device__ __forceinline__ EdgeSink<R> edge_sink(R *edge, const Phys<R> &P, int x, int y, int z)
+template <bool In, typename R>
+__device__ __forceinline__ EdgeSink<R, In> edge_sink(R *edge, const Phys<R> &P, int x, int y, int z)
 {
-    constexpr uint32_t BYTES = 64 * EDGE_SITES * (uint32_t)sizeof(R);
+    constexpr uint32_t RS = (uint32_t)sizeof(R), BYTES = 64 * EDGE_SITES * RS;
     const uint32_t q = (uint32_t)z * (uint32_t)P.ny + (uint32_t)y;
     const uint32_t q0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)q);
-    const uint32_t off = ((q - q0) * EDGE_SITES + (x == 0 ? 38u : 0u)) * (uint32_t)sizeof(R);
-    // nx >= 2: a site is in at most one column
-    return EdgeSink<R>{__builtin_amdgcn_make_buffer_rsrc(edge_site(edge, 0, q0), 0, (int)BYTES, 0x00027000),
-                       x == 0 || x == P.nx - 1 ? off : BYTES};
+    const uint32_t row = (q - q0) * EDGE_SITES * RS;
+    const bool edge_col = x == 0 || x == P.nx - 1;  // nx >= 2: one of them
+    EdgeSink<R, In> e;
+    e.rsrc = __builtin_amdgcn_make_buffer_rsrc(edge_site(edge, 0, q0), 0, (int)BYTES, 0x00027000);
+    e.in = !edge_col;
+    e.off[0] = edge_col ? row + (x == 0 ? 38u * RS : 0u) : BYTES;
+    if constexpr (In) {
+        e.off[1] = e.off[2] = e.off[0];
+        if (!edge_col) {
+            e.off[0] = x == 1 ? row : BYTES;
+            e.off[2] = x == P.nx - 2 ? row : BYTES;
+        }
+    }
+    return e;
 }
 
 template <typename R, bool Dev, int C, bool LE, bool Rock = false, bool ZH = false, bool Flat = false>
@@ -561,6 +589,9 @@ __global__ __launch_bounds__(256) void k_le_gather_edges(Phys<R> P, const R *__r
     const int y = (int)(q % (uint32_t)P.ny), z = (int)(q / (uint32_t)P.ny);
     const int x = col == 0 ? P.nx - 1 : 0;
     edge_site(edge_pc, (int)col, q)[ci] = f[ci * P.ns + sidx(x, y, z, P.nx, P.ny)];
+    const int c = (int)ci / 19, i = (int)ci % 19;
+    if (P.nx > 2 && CX[i] == (col == 0 ? 1 : -1))
+        edge_site(edge_pc, 0, q)[edge_in_at(c, i)] = f[ci * P.ns + sidx(x - CX[i], y, z, P.nx, P.ny)];
 }
 
 // --------------------------------------------------------------------------
@@ -1251,7 +1282,7 @@ __device__ __forceinline__ void collide_site(const Phys<R> &P, const R *__restri
         }
     }
     if constexpr (LE && C == 2)  // the edge columns' post-collision populations
-        bgk_site<R, Dev, C, BD, (NT & 2) != 0>(P, n, F, x, y, z, s, fout, edge_sink(edge_pc, P, x, y, z));
+        bgk_site<R, Dev, C, BD, (NT & 2) != 0>(P, n, F, x, y, z, s, fout, edge_sink<false>(edge_pc, P, x, y, z));
     else
         bgk_site<R, Dev, C, BD, (NT & 2) != 0>(P, n, F, x, y, z, s, fout);
 }
@@ -1649,7 +1680,7 @@ __global__ __launch_bounds__(T) void k_fused2(Phys<R> P, const R *__restrict__ f
                     bgk_site<R, Dev, 2, 2>(P, cur, F, x, y, k, sk, fout, sink);
             };
             if constexpr (LE)  // the edge columns' post-collision populations
-                relax(edge_sink(edge_pc, P, x, y, k));
+                relax(edge_sink<EDGES_IN<R>>(edge_pc, P, x, y, k));
             else
                 relax(NoSink());
         }
@@ -1908,7 +1939,7 @@ __global__ __launch_bounds__(TX *TY) void k_fused3(
 // Streamed population (c, i) of an edge-column site (x = nx-1 for Low, x = 0
 // otherwise; y, z), as pull gives it: from the post-collision edge columns
 // where the source lies in the same column, the halo plane face_pc where it
-// lies outside, the lattice for the column next to it.
+// lies outside, the incoming ones or the lattice for the column next to it.
 template <typename R, bool Low>
 __device__ __forceinline__ R le_streamed(const Phys<R> &P, const R *__restrict__ f, const R *__restrict__ face_pc,
                                          const R *__restrict__ edge, int c, int i, int y, int z)
@@ -1917,6 +1948,9 @@ __device__ __forceinline__ R le_streamed(const Phys<R> &P, const R *__restrict__
     const uint32_t plane = (uint32_t)P.ny * (uint32_t)P.nz, q = (uint32_t)zs * (uint32_t)P.ny + (uint32_t)ys;
     if (CX[i] == 0) return edge_site(edge, Low ? 0 : 1, q)[c * 19 + i];
     if (CX[i] == (Low ? -1 : 1)) return face_pc[((uint32_t)((Low ? 2 : 0) + c) * 19u + (uint32_t)i) * plane + q];
+    // (with two columns, each is the other's neighbour)
+    if constexpr (EDGES_IN<R>)
+        return edge_site(edge, 0, q)[P.nx > 2 ? edge_in_at(c, i) : (Low ? 38u : 0u) + (uint32_t)(c * 19 + i)];
     return f[((uint32_t)c * 19u + (uint32_t)i) * P.ns + sidx(Low ? P.nx - 2 : 1, ys, zs, P.nx, P.ny)];
 }
 

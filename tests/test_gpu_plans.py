@@ -310,6 +310,7 @@ def test_untuned_one_pass_plan_equals_two_pass_bitwise(precision, dims):
     (LB3D_FP64, (97, 83, 75)),
     (LB3D_FP64, (333, 1511, 1)),        # one plane: every z offset wraps onto it
     (LB3D_FP32_DEV, (256, 80, 75)),
+    (LB3D_FP32_DEV, (2, 1301, 601)),    # each column is the other's neighbour
     (LB3D_FP32_DEV, (3, 1001, 501)),    # the columns next to the edges coincide
 ])
 def test_untuned_lees_edwards_one_pass_plan_equals_two_pass_bitwise(precision, dims):

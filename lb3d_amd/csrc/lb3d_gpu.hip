@@ -237,11 +237,13 @@ void io_users(int change)
 //         128^3 386 / 300, 256^3 3170 / 2390.
 // So the lines lie at 0.6 and 0.4 million sites.  Lees-Edwards, whose one-pass
 // plan streams the edge columns once more for the post-advection halo planes:
-//   FP32  100^3 109 / 116, 256x64x64 101 / 103, 134x90x104 140 / 153, 89x135x140
-//         216 / 193, 128^3 224 / 191, 160^3 424 / 389, 192^3 690 / 599;
+//   FP32  96^3 91 / 93, 256x64x64 109 / 102, 96x100x110 127 / 118, 128x128x64
+//         112 / 108, 128x128x80 138 / 133, 89x135x140 216 / 193, 128^3 224 / 191,
+//         160^3 424 / 389, 192^3 690 / 599 (the two passes' figures are up to 9%
+//         lower or higher from one allocation of the lattice to the next);
 //   FP64  140x41x93 126 / 122, 60x84x111 134 / 128, 96^3 187 / 181, 256x64x64
 //         223 / 194, 128^3 421 / 358, 160^3 840 / 775:
-// 1.5 and 0.5 million sites.
+// 1 and 0.5 million sites.
 //
 // Tile: 512 threads (one work-group fills a CU's registers), the shape that
 // leaves the fewest threads idle over the whole plane.  A tile narrower than
@@ -278,7 +280,7 @@ Plan default_plan(const lb3d_params &p)
     const int64_t sites = (int64_t)p.nx * p.ny * p.nz;
     const bool le = p.boundary == LB3D_BC_LEES_EDWARDS;
     if (p.ncomp != 2 || p.bdist != 2 || p.inv_fluid != 0 || !(le || p.boundary == LB3D_BC_PERIODIC)) return q;
-    if (sites < (le ? (fp64 ? 500000 : 1500000) : (fp64 ? 400000 : 600000))) return q;
+    if (sites < (le ? (fp64 ? 500000 : 1000000) : (fp64 ? 400000 : 600000))) return q;
     const int T = 512, CUS = 256;
     double best = 0.0;
     for (int kx = 1; kx <= p.nx; kx++) {

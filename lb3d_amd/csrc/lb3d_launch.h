@@ -294,7 +294,13 @@ class LauncherT : public Launcher {
     }
     unsigned blocks() const { return (P.ns + BLOCK - 1) / BLOCK; }
     // grid of the stepping kernels: whole XCD rounds (xcd_tile order)
-    unsigned tiles() const { return xcd_round(blocks()); }
+    unsigned tiles() const { return xcd_round((P.ns + threads() - 1) / threads()); }
+    // Their work-groups: one wave on lattices that leave CUs idle or uneven
+    // otherwise (32^3 is 128 groups of 256).  Step, groups of 256 -> 64 (us):
+    // binary FP32 16^3 8.4 -> 7.1, 32^3 8.3 -> 7.7, FP64 16^3 11.3 -> 9.2, 32^3
+    // 12.2 -> 10.7, 48^3 18.9 -> 18.0; ternary FP32 24^3 17.5 -> 14.8, FP64 32^3
+    // 23.4 -> 20.7, 48^3 42.1 -> 41.3; ternary FP64 64^3 84 -> 87.
+    unsigned threads() const { return P.ns <= 120000u ? 64u : BLOCK; }
     unsigned diag_blocks() const override { return blocks(); }
     size_t real_bytes() const override { return sizeof(R); }
 
@@ -302,19 +308,19 @@ class LauncherT : public Launcher {
     {
         const R *f = (const R *)b.f[b.cur];
         if (C == 3 && P.zh)
-            k_moments<R, Dev, 3, false, false, true><<<tiles(), BLOCK, 0, s>>>(P, f, nullptr, (const R *)b.db,
+            k_moments<R, Dev, 3, false, false, true><<<tiles(), threads(), 0, s>>>(P, f, nullptr, (const R *)b.db,
                                                                                (R *)b.aux, xg, nullptr);
         else if (C == 3)
-            k_moments<R, Dev, 3, false><<<tiles(), BLOCK, 0, s>>>(P, f, nullptr, (const R *)b.db, (R *)b.aux, xg,
+            k_moments<R, Dev, 3, false><<<tiles(), threads(), 0, s>>>(P, f, nullptr, (const R *)b.db, (R *)b.aux, xg,
                                                                   nullptr);
         else if (le)
-            k_moments<R, Dev, 2, true><<<tiles(), BLOCK, 0, s>>>(P, f, (const R *)b.face_pc, nullptr, (R *)b.aux, xg,
+            k_moments<R, Dev, 2, true><<<tiles(), threads(), 0, s>>>(P, f, (const R *)b.face_pc, nullptr, (R *)b.aux, xg,
                                                                  nullptr, (R *)b.edge_adv);
         else if (b.rock)
-            k_moments<R, Dev, 2, false, true><<<tiles(), BLOCK, 0, s>>>(P, f, nullptr, nullptr, (R *)b.aux, xg,
+            k_moments<R, Dev, 2, false, true><<<tiles(), threads(), 0, s>>>(P, f, nullptr, nullptr, (R *)b.aux, xg,
                                                                         b.rock);
         else
-            k_moments<R, Dev, 2, false><<<tiles(), BLOCK, 0, s>>>(P, f, nullptr, nullptr, (R *)b.aux, xg, nullptr);
+            k_moments<R, Dev, 2, false><<<tiles(), threads(), 0, s>>>(P, f, nullptr, nullptr, (R *)b.aux, xg, nullptr);
     }
     void forces(const DevBufs &b, void *out, hipStream_t s) override
     {
@@ -329,7 +335,7 @@ class LauncherT : public Launcher {
     void dipole(const DevBufs &b, hipStream_t s) override
     {
         // the relaxed field goes to db_alt (the collide reads it there)
-        if (C == 3) k_dipole<R, Dev><<<tiles(), BLOCK, 0, s>>>(P, (const R *)b.aux, (R *)b.db_alt, xg);
+        if (C == 3) k_dipole<R, Dev><<<tiles(), threads(), 0, s>>>(P, (const R *)b.aux, (R *)b.db_alt, xg);
     }
     // Step, three kernels against moments and k_dipole_collide (us): FP32 12^3
     // 17.5 / 13.7, 16^3 15.9 / 13.3, 20^3 17.1 / 15.1, 24^3 16.6 / 16.4, 32^3
@@ -359,23 +365,23 @@ class LauncherT : public Launcher {
         const R *f = (const R *)b.f[b.cur];
         R *fo = (R *)b.f[1 - b.cur];
         if (P.zh && C == 3)
-            k_collide<R, Dev, 3, false, BD, false, true, NT><<<tiles(), BLOCK, 0, s>>>(
+            k_collide<R, Dev, 3, false, BD, false, true, NT><<<tiles(), threads(), 0, s>>>(
                 P, f, nullptr, (const R *)b.aux, nullptr, (const R *)b.db_alt, fo, xg, nullptr);
         else if (P.zh && !le && !b.rock)
-            k_collide<R, Dev, 2, false, BD, false, true, NT><<<tiles(), BLOCK, 0, s>>>(
+            k_collide<R, Dev, 2, false, BD, false, true, NT><<<tiles(), threads(), 0, s>>>(
                 P, f, nullptr, (const R *)b.aux, nullptr, nullptr, fo, xg, nullptr);
         else if (C == 3)
-            k_collide<R, Dev, 3, false, BD, false, false, NT><<<tiles(), BLOCK, 0, s>>>(
+            k_collide<R, Dev, 3, false, BD, false, false, NT><<<tiles(), threads(), 0, s>>>(
                 P, f, nullptr, (const R *)b.aux, nullptr, (const R *)b.db_alt, fo, xg, nullptr);
         else if (le)
-            k_collide<R, Dev, 2, true, BD, false, false, NT><<<tiles(), BLOCK, 0, s>>>(
+            k_collide<R, Dev, 2, true, BD, false, false, NT><<<tiles(), threads(), 0, s>>>(
                 P, f, (const R *)b.face_pc, (const R *)b.aux, (const R *)b.face_aux, nullptr, fo, xg, nullptr,
                 (R *)b.edge_pc, le_commit == LE_STATE_AS_IS ? nullptr : b.le, le_commit);
         else if (b.rock)
-            k_collide<R, Dev, 2, false, BD, true><<<tiles(), BLOCK, 0, s>>>(P, f, nullptr, (const R *)b.aux,
+            k_collide<R, Dev, 2, false, BD, true><<<tiles(), threads(), 0, s>>>(P, f, nullptr, (const R *)b.aux,
                                                                             nullptr, nullptr, fo, xg, b.rock);
         else
-            k_collide<R, Dev, 2, false, BD, false, false, NT><<<tiles(), BLOCK, 0, s>>>(
+            k_collide<R, Dev, 2, false, BD, false, false, NT><<<tiles(), threads(), 0, s>>>(
                 P, f, nullptr, (const R *)b.aux, nullptr, nullptr, fo, xg, nullptr);
     }
     // the non-temporal form once one copy of the populations exceeds the

@@ -337,26 +337,28 @@ class LauncherT : public Launcher {
         // the relaxed field goes to db_alt (the collide reads it there)
         if (C == 3) k_dipole<R, Dev><<<tiles(), threads(), 0, s>>>(P, (const R *)b.aux, (R *)b.db_alt, xg);
     }
-    // Step, three kernels against moments and k_dipole_collide (us): FP32 12^3
-    // 17.5 / 13.7, 16^3 15.9 / 13.3, 20^3 17.1 / 15.1, 24^3 16.6 / 16.4, 32^3
-    // 16.2 / 17.6; FP64 13x9x7 21.2 / 19.9, 16^3 20.4 / 18.4, 20^3 21.7 / 22.7.
-    // The dipoles of the halo are 2.8 times as many as the sites, which pays
-    // while the CUs are idle otherwise.
-    bool small() const override { return C == 3 && !P.zh && P.ns <= (Dev ? 10000u : 5000u); }
+    // FP32 step, three kernels against moments and k_dipole_collide (us): 8^3
+    // 14.3 / 12.3, 12^3 15.0 / 12.8, 16^3 14.8 / 13.4, 20^3 15.2 / 14.2, 22^3 15.6 /
+    // 14.9, 24^3 14.3 / 15.6.  The dipoles of the halo are 2.8 times as many as the
+    // sites, which pays while the CUs are idle otherwise.  In FP64, whose relaxation
+    // takes longer than a launch, it does not (12^3 18.1 / 19.1, 16^3 17.3 / 18.0).
+    bool small() const override { return Dev && C == 3 && !P.zh && P.ns <= 10000u; }
     bool dipole_collide(const DevBufs &b, hipStream_t s) override
     {
         if (!small()) return false;
-        const uint32_t tx = (P.nx + DC_X - 1) / DC_X, ty = (P.ny + DC_Y - 1) / DC_Y, tz = (P.nz + DC_Z - 1) / DC_Z;
-        auto go = [&](auto kernel) {
-            kernel<<<tx * ty * tz, DC_THREADS, 0, s>>>(P, (const R *)b.f[b.cur], (const R *)b.aux, (R *)b.db_alt,
-                                                       (R *)b.f[1 - b.cur], tx, ty);
-        };
-        if (P.bdist == 0)
-            go(k_dipole_collide<R, Dev, 0>);
-        else if (P.bdist == 2)
-            go(k_dipole_collide<R, Dev, 2>);
-        else
-            go(k_dipole_collide<R, Dev, BD_GENERAL>);
+        if constexpr (Dev) {
+            const uint32_t tx = (P.nx + DC_X - 1) / DC_X, ty = (P.ny + DC_Y - 1) / DC_Y, tz = (P.nz + DC_Z - 1) / DC_Z;
+            auto go = [&](auto kernel) {
+                kernel<<<tx * ty * tz, DC_THREADS, 0, s>>>(P, (const R *)b.f[b.cur], (const R *)b.aux, (R *)b.db_alt,
+                                                           (R *)b.f[1 - b.cur], tx, ty);
+            };
+            if (P.bdist == 0)
+                go(k_dipole_collide<R, Dev, 0>);
+            else if (P.bdist == 2)
+                go(k_dipole_collide<R, Dev, 2>);
+            else
+                go(k_dipole_collide<R, Dev, BD_GENERAL>);
+        }
         return true;
     }
     template <int BD, bool NT>

@@ -239,16 +239,14 @@ def test_long_batch_runs_replay_a_graph_bitwise():
         assert np.array_equal(a.populations(k), b.populations(k))
 
 
-@pytest.mark.parametrize("precision,dims", [
-    (p, d) for p, most in ((LB3D_FP64, 5000), (LB3D_FP32_DEV, 10000))
-    for d in [(2, 1, 1), (8, 4, 2), (9, 5, 3), (7, 3, 1), (17, 13, 11), (3, 40, 41), (625, 8, 1), (25, 20, 20)]
-    if d[0] * d[1] * d[2] <= most])
+@pytest.mark.parametrize("dims", [(2, 1, 1), (8, 4, 2), (9, 5, 3), (7, 3, 1), (17, 13, 11), (3, 40, 41),
+                                  (625, 8, 1), (25, 20, 20)])
 @pytest.mark.parametrize("bdist", [0, 2, 1])
-def test_small_ternary_lattice_in_two_launches_equals_three_kernels_bitwise(precision, dims, bdist):
-    """A small ternary lattice relaxes dipoles and populations in one launch,
-    by tiles of 8 x 4 x 2 sites that overhang it; the batch's lattice by
+def test_small_ternary_lattice_in_two_launches_equals_three_kernels_bitwise(dims, bdist):
+    """A small FP32 ternary lattice relaxes dipoles and populations in one
+    launch, by tiles of 8 x 4 x 2 sites that overhang it; the batch's lattice by
     lattice plan runs the kernels one by one."""
-    kw = dict(ncomp=3, precision=precision, bdist=bdist, g_br=0.08, g_bs=-0.006, g_ss=-0.003)
+    kw = dict(ncomp=3, precision=LB3D_FP32_DEV, bdist=bdist, g_br=0.08, g_bs=-0.006, g_ss=-0.003)
     b = Batch([dims], **kw)
     b.set_plan(1)
     b.init_noise(0, 3, amp=(0.05, 0.05, 0.05))

@@ -153,7 +153,7 @@ int lb3d_gpu_run_steps_timed(lb3d_ctx *ctx, int32_t nsteps, double *ms);
 
 /* Autotuner (not a reference routine): times every execution plan of this
  * lattice -- the two-pass kernels and, for binary lattices, the one-pass
- * z-march kernel over its tile shapes and z-chunks, then the XCD chunking of
+ * z-march kernel with a fitted tile and over its tile shapes and z-chunks, then the XCD chunking of
  * the best -- on trial_steps trial steps each, keeps the fastest and writes a
  * text report (may be NULL).  The lattice state is unchanged. */
 int lb3d_gpu_autotune(lb3d_ctx *ctx, int32_t trial_steps, char *report, int32_t report_len);
@@ -248,8 +248,8 @@ int lb3d_gpu_profile_steps(lb3d_ctx *ctx, int32_t nsteps, int32_t max_kernels,
  * One timestep that allocates nothing.  No counterpart in the reference: it
  * is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  A
- * periodic lattice of parameters p advances one step of the two-pass plan
- * from f_in to f_out (the populations in the device layout of p->precision:
+ * periodic lattice of parameters p advances one step, on the plan that a
+ * context of its size runs untuned, from f_in to f_out (the populations in the device layout of p->precision:
  * f[(c*19 + i)*ns + s], FP64 values or FP32 deviations n_i - w_i*rho0_c;
  * s = x + nx*(y + ny*z)); ternary lattices also read the dipole field db_in
  * and write the relaxed field to db_out (db[k*ns + s]).  All four are

@@ -380,7 +380,7 @@ constexpr uint32_t EDGE_IN = 2 * 38, EDGE_SITES = EDGE_IN + 2 * 10;  // values o
 template <typename T>
 __device__ __forceinline__ T *edge_site(T *edge, int col, uint32_t q)
 {
-    return edge + (q * EDGE_SITES + (uint32_t)col * 38u);
+    return edge + (size_t)q * EDGE_SITES + (uint32_t)col * 38u;  // (96 values a site may pass 2^32)
 }
 // the place of an incoming population, c_x(i) != 0, after the 38s: column 0's
 // come with c_x = 1, column 1's with c_x = -1.  The FP32 one-pass plan keeps

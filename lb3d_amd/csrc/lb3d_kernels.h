@@ -1506,7 +1506,11 @@ __global__ __launch_bounds__(T) void k_fused2(Phys<R> P, const R *__restrict__ f
     // against 1.10 ms, 200^3: 0.65 against 0.56 ms).
     constexpr bool BR = sizeof(R) == 4 && !LE;
     const bool need = slot && x <= P.nx && y <= P.ny;
-    const int xw = need && x < P.nx ? x : 0, yw = need && y < P.ny ? y : 0;
+    // (a thread that fills no slot takes column 0: at its own x beyond the
+    // lattice it would read a halo column, at a y that wrapping once need not
+    // bring into the plane)
+    const int xn = need ? x : 0;
+    const int xw = xn < P.nx ? xn : 0, yw = need && y < P.ny ? y : 0;
     // a thread whose psi nobody reads writes it to a spare slot: a branch here
     // would leave its loads unfinished on one path, and the compiler then
     // waits for everything, the stores of the collide too, in every plane
@@ -1589,7 +1593,7 @@ __global__ __launch_bounds__(T) void k_fused2(Phys<R> P, const R *__restrict__ f
             r0 = r0 + v0 * R(GD[i]);
             r1 = r1 + v1 * R(GD[i]);
         }
-        put(rs, mine, x, y, zp, psi_of<Dev>(r0, P.emr0[0]), psi_of<Dev>(r1, P.emr0[1]));
+        put(rs, mine, xn, y, zp, psi_of<Dev>(r0, P.emr0[0]), psi_of<Dev>(r1, P.emr0[1]));
 #pragma unroll
         for (int r = 0; r < NHS; r++)
             if (hv[r]) {

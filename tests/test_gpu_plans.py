@@ -367,3 +367,21 @@ def test_long_runs_replay_a_graph_bitwise(kw):
         for _ in range(99):
             ref.time_step()
         assert np.array_equal(g.populations(), ref.populations()), again
+
+
+@pytest.mark.parametrize("precision", [LB3D_FP64, LB3D_FP32_DEV])
+@pytest.mark.parametrize("dims", [(3, 2, 1), (40, 2, 1), (33, 3, 2), (5, 1, 4)])
+def test_lees_edwards_tiles_taller_than_twice_the_lattice(precision, dims):
+    """Tiles of 2 to 16 rows on lattices of 1 to 3: the threads beyond the
+    lattice, some more than a whole lattice beyond it, fill no slot and read
+    no halo plane."""
+    kw = dict(ncomp=2, precision=precision, g_br=0.09, boundary=LB3D_BC_LEES_EDWARDS, shear_u=0.04)
+    _, ref = pair(*dims, **kw)
+    ref.set_plan(0)
+    ref.time_loop(4)
+    want = ref.populations()
+    for mode, tx, ty in fused_shapes(precision):
+        _, g = pair(*dims, **kw)
+        g.set_plan(mode, tx, ty, dims[2])
+        g.time_loop(4)
+        assert np.array_equal(g.populations(), want), f"mode {mode} {tx}x{ty}"

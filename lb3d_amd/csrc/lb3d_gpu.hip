@@ -37,6 +37,12 @@ int fail(int code, const std::string &msg)
 
 enum StageState { IDLE = 0, AFTER_BC6 = 1, AFTER_ADV = 2, AFTER_BC8 = 3 };
 
+// The moments of the last advection: none since the state was set; in the aux
+// field; or, after the one-pass plans, which keep none, to be rebuilt from the
+// populations that it streamed: f[1-cur] once the step is complete, f[cur]
+// between advection and collision.
+enum MomentState { MOMENTS_NONE = 0, MOMENTS_KEPT, MOMENTS_PREV, MOMENTS_CUR };
+
 // HIP events that are destroyed when the scope ends, also on an early error return
 struct Events {
     std::vector<hipEvent_t> e;
@@ -86,7 +92,7 @@ struct lb3d_ctx {
     int nt = 0;
     int state = IDLE;
     bool le = false;
-    bool aux_valid = false;
+    MomentState moments = MOMENTS_NONE;
     LEState host_le{};
     hipGraphExec_t graph = nullptr;
     int graph_len = 0;     // steps of the captured graph
@@ -97,12 +103,15 @@ struct lb3d_ctx {
     size_t aux_elems = 0;  // elements of the aux field
     Plan plan;
     bool tuned = false;
-    bool aux_from_prev = false;  // aux is recomputable from f[1-cur] (fused binary steps)
     // ternary dipole fields, tied to the population parity: a step reads
     // dbk[cur] (the field of the state) and writes dbk[1-cur] (the relaxed
     // field), so a captured two-step graph finds the live field where it
     // expects it whatever the host did before
     void *dbk[2] = {nullptr, nullptr};
+    // Lees-Edwards halo planes of the populations f[0] and f[1]: those that the
+    // last step streamed through stay what they were while the planes of the
+    // new state are built (rebuild_aux may still need them)
+    void *facek[2] = {nullptr, nullptr};
     // Lees-Edwards: the edge columns b.edge_pc hold f[cur]'s (written by the
     // last kernel of a step, else gathered before the next halo-plane pass)
     bool edges_ok = false;
@@ -118,12 +127,13 @@ static void ensure_edges(lb3d_ctx *c)
     }
 }
 
-// Points b.db / b.db_alt at the dipole fields of the current parity.
+// Points b.db / b.db_alt / b.face_pc at the fields of the current parity.
 static void set_cur(lb3d_ctx *c, int cur)
 {
     c->b.cur = cur;
     c->b.db = c->dbk[cur];
     c->b.db_alt = c->dbk[1 - cur];
+    c->b.face_pc = c->facek[cur];
 }
 
 static void flip(lb3d_ctx *c) { set_cur(c, 1 - c->b.cur); }
@@ -456,15 +466,17 @@ int lb3d_gpu_create(const lb3d_params *p, lb3d_ctx **out)
     if (c->db_bytes && ((e = hipMalloc(&c->dbk[0], c->db_bytes)) != hipSuccess ||
                         (e = hipMalloc(&c->dbk[1], c->db_bytes)) != hipSuccess))
         return cleanup(LB3D_ENOMEM, std::string("hipMalloc db: ") + hipGetErrorString(e));
-    set_cur(c, 0);
     if (c->le) {
         const size_t edges = EDGE_SITES * plane * rs;
         if ((e = hipMalloc(&c->b.edge_pc, edges)) != hipSuccess || (e = hipMalloc(&c->b.edge_adv, edges)) != hipSuccess)
             return cleanup(LB3D_ENOMEM, std::string("hipMalloc LE edge columns: ") + hipGetErrorString(e));
-        if ((e = hipMalloc(&c->b.face_pc, 2 * 2 * 19 * plane * rs)) != hipSuccess ||
-            (e = hipMalloc(&c->b.face_aux, 2 * 4 * plane * rs)) != hipSuccess)
+        for (int k = 0; k < 2; k++)
+            if ((e = hipMalloc(&c->facek[k], 2 * 2 * 19 * plane * rs)) != hipSuccess)
+                return cleanup(LB3D_ENOMEM, std::string("hipMalloc LE planes: ") + hipGetErrorString(e));
+        if ((e = hipMalloc(&c->b.face_aux, 2 * 4 * plane * rs)) != hipSuccess)
             return cleanup(LB3D_ENOMEM, std::string("hipMalloc LE planes: ") + hipGetErrorString(e));
     }
+    set_cur(c, 0);
     if ((e = hipMalloc((void **)&c->b.le, sizeof(LEState))) != hipSuccess ||
         (e = hipMalloc((void **)&c->d_partials, (size_t)c->L->diag_blocks() * NSAN * sizeof(double))) !=
             hipSuccess)
@@ -493,7 +505,8 @@ int lb3d_gpu_destroy(lb3d_ctx *c)
         if (c->dbk[k]) (void)hipFree(c->dbk[k]);
     if (c->b.edge_pc) (void)hipFree(c->b.edge_pc);
     if (c->b.edge_adv) (void)hipFree(c->b.edge_adv);
-    if (c->b.face_pc) (void)hipFree(c->b.face_pc);
+    for (int k = 0; k < 2; k++)
+        if (c->facek[k]) (void)hipFree(c->facek[k]);
     if (c->b.face_aux) (void)hipFree(c->b.face_aux);
     if (c->b.le) (void)hipFree(c->b.le);
     if (c->d_partials) (void)hipFree(c->d_partials);
@@ -575,7 +588,7 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
     uint8_t *mask = nullptr;
     if (walls_ok) {
         mask = (uint8_t *)c->b.aux;
-        c->aux_valid = false;
+        c->moments = MOMENTS_NONE;
     }
     IoLoan io;
     const PopBase pb = pop_base(p);
@@ -603,7 +616,6 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
     HIP_TRY(hipStreamSynchronize(c->stream));
     std::memcpy(&nrock, io->pin[0], sizeof nrock);
     if (nrock && !walls_ok) {
-        c->aux_from_prev = false;  // f[1 - cur] holds the refused records
         if (p.ncomp != 2 || c->le)
             return fail(LB3D_EINVAL, "rock sites (walls) are supported on periodic binary lattices");
         return fail(LB3D_EINVAL, "rock sites (walls) and the Zou-He boundary are not supported together");
@@ -617,8 +629,7 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
     c->nt = nt0;
     c->host_le.nt = nt0;
     c->state = IDLE;
-    c->aux_valid = false;
-    c->aux_from_prev = false;
+    c->moments = MOMENTS_NONE;
     c->edges_ok = false;
     return LB3D_OK;
 }
@@ -636,8 +647,7 @@ int lb3d_gpu_init_noise(lb3d_ctx *c, uint64_t seed, const double rho_mean[3], co
     c->nt = 0;
     c->host_le.nt = 0;
     c->state = IDLE;
-    c->aux_valid = false;
-    c->aux_from_prev = false;
+    c->moments = MOMENTS_NONE;
     c->edges_ok = false;
     return LB3D_OK;
 }
@@ -653,18 +663,20 @@ int lb3d_gpu_get_populations(lb3d_ctx *c, double *out)
 }
 
 // The one-pass plans keep no moments: rebuild those of the last advection
-// from the previous post-collision populations f[1-cur] and the dipole field
-// that step read (db_alt).
+// from the populations that it streamed, with the dipole field that its step
+// read and the Lees-Edwards halo planes of that step.
 static int rebuild_aux(lb3d_ctx *c)
 {
-    if (c->aux_valid || !c->aux_from_prev) return LB3D_OK;
-    DevBufs prev = c->b;
-    prev.cur = 1 - c->b.cur;
-    if (c->p.ncomp == 3) prev.db = c->b.db_alt;
-    c->L->moments(prev, c->stream);
+    if (c->moments != MOMENTS_PREV && c->moments != MOMENTS_CUR) return LB3D_OK;
+    DevBufs src = c->b;
+    if (c->moments == MOMENTS_PREV) {
+        src.cur = 1 - c->b.cur;
+        src.db = c->b.db_alt;
+        src.face_pc = c->facek[src.cur];
+    }
+    c->L->moments(src, c->stream);
     HIP_TRY(hipGetLastError());
-    c->aux_valid = true;
-    c->aux_from_prev = false;
+    c->moments = MOMENTS_KEPT;
     return LB3D_OK;
 }
 
@@ -687,7 +699,7 @@ int lb3d_gpu_download_sites(lb3d_ctx *c, double *N, int32_t h, int32_t sd)
         auto go = [&](auto r) {
             using R = decltype(r);
             k_get_sites<R><<<nb, 256, lds, c->stream>>>(
-                (const R *)c->b.f[c->b.cur], c->aux_valid ? (const R *)c->b.aux : nullptr, (const R *)c->b.db,
+                (const R *)c->b.f[c->b.cur], c->moments == MOMENTS_KEPT ? (const R *)c->b.aux : nullptr, (const R *)c->b.db,
                 c->b.rock, pb, rho0_of(c, 0), rho0_of(c, 1), rho0_of(c, 2), L, (uint32_t)(at / rec), n, (double *)buf);
         };
         is_dev(c) ? go(float()) : go(double());
@@ -773,6 +785,7 @@ int lb3d_gpu_advection(lb3d_ctx *c)
         c->L->moments(c->b, c->stream);
         HIP_TRY(hipGetLastError());
     }
+    if (c->moments != MOMENTS_NONE) c->moments = c->plan.fused ? MOMENTS_CUR : MOMENTS_KEPT;
     c->state = AFTER_ADV;
     return LB3D_OK;
 }
@@ -795,8 +808,7 @@ static int launch_collision(lb3d_ctx *c)
 
 static void mark_stepped(lb3d_ctx *c)
 {
-    c->aux_valid = !c->plan.fused;
-    c->aux_from_prev = c->plan.fused;
+    c->moments = c->plan.fused ? MOMENTS_PREV : MOMENTS_KEPT;
 }
 
 int lb3d_gpu_collision(lb3d_ctx *c)
@@ -1001,8 +1013,7 @@ int lb3d_gpu_autotune(lb3d_ctx *c, int32_t trial_steps, char *report, int32_t re
     // f[1-cur] and db_alt no longer hold the last step's input, so the
     // moments of the last advection cannot be rebuilt from them afterwards;
     // the edge columns are gathered for the trials and are stale after them
-    c->aux_valid = false;
-    c->aux_from_prev = false;
+    c->moments = MOMENTS_NONE;
     if (c->le) {
         c->L->le_gather_edges(c->b, c->stream);
         c->edges_ok = false;
@@ -1158,7 +1169,7 @@ int lb3d_gpu_get_arrows(lb3d_ctx *c, double *out)
     if (c->state != IDLE) return fail(LB3D_ESTATE, "get_arrows needs a completed timestep");
     int rc = rebuild_aux(c);
     if (rc) return rc;
-    if (!c->aux_valid)
+    if (c->moments != MOMENTS_KEPT)
         return fail(LB3D_ESTATE, "get_arrows needs the moments of an advection: run a timestep first");
     const int C = c->p.ncomp, nx = c->p.nx, ny = c->p.ny, nz = c->p.nz;
     const size_t ns = (size_t)nx * ny * nz, rs = c->L->real_bytes();

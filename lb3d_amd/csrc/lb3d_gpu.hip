@@ -762,7 +762,7 @@ int lb3d_gpu_bc_apply(lb3d_ctx *c, int32_t stage, int32_t nt)
     } else if (stage == 8) {
         if (c->state != AFTER_ADV) return fail(LB3D_ESTATE, "bc_apply(8) must follow advection");
         if (c->le) {
-            ensure_edges(c);  // (the plan may have changed within the step)
+            ensure_edges(c);  // (set_plan may have come between, for whose plan they are gathered anew)
             c->L->le_faces(c->b, true, c->plan.fused, c->stream);
             HIP_TRY(hipGetLastError());
         }
@@ -1106,6 +1106,14 @@ int lb3d_gpu_set_plan(lb3d_ctx *c, int32_t fused, int32_t tx, int32_t ty, int32_
         q.tx = tx;
         q.ty = ty;
         q.lz = lz < c->p.nz ? lz : c->p.nz;
+    }
+    // A step under way goes on with the new plan.  The one-pass plans stream
+    // in their collision; the two-pass collision, and the Lees-Edwards planes
+    // before it, read what the moments pass of the advection has written.
+    if (c->plan.fused && !q.fused && (c->state == AFTER_ADV || c->state == AFTER_BC8)) {
+        c->L->moments(c->b, c->stream);
+        HIP_TRY(hipGetLastError());
+        if (c->moments != MOMENTS_NONE) c->moments = MOMENTS_KEPT;
     }
     c->plan = q;
     c->L->xg = q.xg;

@@ -95,3 +95,30 @@ def test_records_within_a_step_leave_the_step_alone(kw, plan):
         g.bc_apply(8, 4)
         g.collision()
         assert np.array_equal(g.populations(), want), f"{what}: {np.abs(g.populations() - want).max()}"
+
+
+@pytest.mark.parametrize("kw,plan", FORMS)
+@pytest.mark.parametrize("precision", [LB3D_FP64, LB3D_FP32_DEV])
+@pytest.mark.parametrize("first", [False, True])
+def test_plan_changes_within_a_step(kw, plan, precision, first):
+    """set_plan between any two calls of a staged step, in either direction and
+    back again, on the first step of a state too: populations and records are
+    those of the two-pass plan."""
+    kw = dict(kw, precision=precision)
+    dims = (20, 9, 12)
+    steps = 0 if first else 3
+    ref = lattice(dims, 0, steps + 2, **kw)
+    want, want_rec = ref.populations(), ref.download_sites()
+    for switch in range(4):
+        for plans in ((plan, 0), (0, plan), (plan, 0, plan), (0, plan, 0)):
+            g = lattice(dims, plans[0], steps, **kw)
+            calls = [lambda: g.bc_apply(6), g.advection, lambda: g.bc_apply(8), g.collision]
+            for k, call in enumerate(calls):
+                if k == switch:
+                    for p in plans[1:]:
+                        g.set_plan(*p) if p else g.set_plan(0)
+                call()
+            g.time_step()
+            got = g.populations()
+            assert np.array_equal(got, want), f"{plans} before call {switch}: {np.abs(got - want).max()}"
+            assert np.array_equal(g.download_sites(), want_rec), f"{plans} before call {switch}: records"

@@ -38,6 +38,7 @@ struct lb3d_batch {
     double *partials = nullptr;
     uint32_t nitems = 0;
     hipStream_t stream = nullptr;
+    int device = 0;  // that the batch was made on
     hipGraphExec_t graph = nullptr;
     int graph_len = 0;       // steps of the captured graph
     int64_t plan_steps = 0;  // steps run on the current plan (a graph is captured after GRAPH_AFTER)
@@ -313,6 +314,7 @@ int lb3d_gpu_batch_create(int32_t nlat, const lb3d_params *params, lb3d_batch **
     }
     lb3d_batch *b = new lb3d_batch();
     io_users(1);
+    (void)hipGetDevice(&b->device);
     b->nlat = nlat;
     b->C = p0.ncomp;
     b->prec = p0.precision;
@@ -424,6 +426,7 @@ int lb3d_gpu_batch_get_populations(lb3d_batch *b, int32_t k, double *out)
 {
     clear_error();
     if (!b || k < 0 || k >= b->nlat || !out) return set_error(LB3D_EINVAL, "bad argument");
+    const OnDevice on(b->device);
     const void *f = view(b, k).f[b->cur];
     BTRY(b->rs == 4 ? fetch_populations<float>(b->stream, b->p[k], f, out)
                     : fetch_populations<double>(b->stream, b->p[k], f, out));

@@ -89,6 +89,7 @@ struct lb3d_ctx {
     Launcher *L = nullptr;
     DevBufs b;
     hipStream_t stream = nullptr;
+    int device = 0;  // that the context was made on
     int nt = 0;
     int state = IDLE;
     bool le = false;
@@ -441,6 +442,7 @@ int lb3d_gpu_create(const lb3d_params *p, lb3d_ctx **out)
     if (rc) return rc;
     lb3d_ctx *c = new lb3d_ctx();
     io_users(1);
+    (void)hipGetDevice(&c->device);
     c->p = *p;
     c->le = p->boundary == LB3D_BC_LEES_EDWARDS;
     c->L = p->precision == LB3D_FP64 ? make_launcher_fp64(*p) : make_launcher_fp32(*p);
@@ -572,6 +574,7 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
 {
     g_err.clear();
     if (!c || !N) return fail(LB3D_EINVAL, "NULL argument");
+    const OnDevice on(c->device);
     const lb3d_params &p = c->p;
     if (sd != (p.ncomp == 3 ? 79 : 49)) return fail(LB3D_EINVAL, "site_doubles must be 79 (ternary) or 49 (binary)");
     if (h < 1) return fail(LB3D_EINVAL, "halo_extent must be >= 1");
@@ -656,6 +659,7 @@ int lb3d_gpu_get_populations(lb3d_ctx *c, double *out)
 {
     g_err.clear();
     if (!c || !out) return fail(LB3D_EINVAL, "NULL argument");
+    const OnDevice on(c->device);
     const void *f = c->b.f[c->b.cur];
     HIP_TRY(is_dev(c) ? fetch_populations<float>(c->stream, c->p, f, out)
                       : fetch_populations<double>(c->stream, c->p, f, out));
@@ -684,6 +688,7 @@ int lb3d_gpu_download_sites(lb3d_ctx *c, double *N, int32_t h, int32_t sd)
 {
     g_err.clear();
     if (!c || !N) return fail(LB3D_EINVAL, "NULL argument");
+    const OnDevice on(c->device);
     const int C = c->p.ncomp;
     if (sd != (C == 3 ? 79 : 49)) return fail(LB3D_EINVAL, "site_doubles must be 79 (ternary) or 49 (binary)");
     if (h < 1) return fail(LB3D_EINVAL, "halo_extent must be >= 1");
@@ -1134,6 +1139,7 @@ int lb3d_gpu_get_density(lb3d_ctx *c, double *out)
 {
     g_err.clear();
     if (!c || !out) return fail(LB3D_EINVAL, "NULL argument");
+    const OnDevice on(c->device);
     const uint32_t ns = (uint32_t)c->p.nx * (uint32_t)c->p.ny * (uint32_t)c->p.nz;
     const PopBase pb = pop_base(c->p);
     const void *f = c->b.f[c->b.cur];
@@ -1150,6 +1156,7 @@ int lb3d_gpu_get_momentum(lb3d_ctx *c, double *out)
 {
     g_err.clear();
     if (!c || !out) return fail(LB3D_EINVAL, "NULL argument");
+    const OnDevice on(c->device);
     const uint32_t ns = (uint32_t)c->p.nx * (uint32_t)c->p.ny * (uint32_t)c->p.nz;
     const PopBase pb = pop_base(c->p);
     const void *f = c->b.f[c->b.cur];

@@ -382,6 +382,27 @@ struct HostIO {
     }
 };
 
+// Makes a context's device current for the length of a call.  Copies on a
+// stream run whatever device is current; the events, buffers and kernels of a
+// transfer have to be those of the stream's device.
+class OnDevice {
+  public:
+    explicit OnDevice(int device)
+    {
+        if (hipGetDevice(&was_) == hipSuccess && was_ != device) moved_ = hipSetDevice(device) == hipSuccess;
+    }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+    ~OnDevice()
+    {
+        if (moved_) (void)hipSetDevice(was_);
+    }
+
+  private:
+    int was_ = -1;
+    bool moved_ = false;
+};
+
 // Transfer buffers are lent for one call and shared by all contexts (pinning
 // them takes about 4 ms, more than a small lattice's whole run between two
 // dumps): IoLoan takes a set of the current device from a pool, or a new one,

@@ -596,21 +596,18 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
     IoLoan io;
     const PopBase pb = pop_base(p);
     const int to = 1 - c->b.cur;
-    const uint32_t nxy = (uint32_t)p.nx * (uint32_t)p.ny;
-    const size_t plane = (size_t)(p.nx + 2 * h) * (size_t)(p.ny + 2 * h) * (size_t)sd;  // doubles
-    // pieces of whole z planes
-    const size_t piece = plane * 8 * (IO_PIECE < plane * 8 ? 1 : IO_PIECE / (plane * 8));
-    const size_t lds = (size_t)REC_SITES * sd * 8;
+    // the records of the z planes that hold sites
+    const size_t plane = (size_t)(p.nx + 2 * h) * (size_t)(p.ny + 2 * h), skip = (size_t)h * plane;
+    const size_t rec = (size_t)sd * 8, lds = (size_t)REC_SITES * rec;
+    const size_t piece = IO_PIECE / (REC_SITES * rec) * (REC_SITES * rec);  // whole blocks of records
     HIP_TRY(io->ensure(1));
     HIP_TRY(hipMemsetAsync(io->count, 0, sizeof(uint32_t), c->stream));
-    HIP_TRY(io->up(c->stream, N + (size_t)h * plane, (size_t)p.nz * plane * 8, piece, [&](size_t at, size_t len, void *buf) {
-        const uint32_t z = (uint32_t)(at / (plane * 8)), n = (uint32_t)(len / (plane * 8)) * nxy;
-        const uint32_t nb = (n + REC_SITES - 1) / REC_SITES;
+    HIP_TRY(io->up(c->stream, N + skip * sd, (size_t)p.nz * plane * rec, piece, [&](size_t at, size_t len, void *buf) {
+        const uint32_t n = (uint32_t)(len / rec), nb = (n + REC_SITES - 1) / REC_SITES;
         auto go = [&](auto r) {
             using R = decltype(r);
-            k_put_sites<R><<<nb, 256, lds, c->stream>>>((const double *)buf, z + (uint32_t)h, L, pb, z * nxy, n,
-                                                        (R *)c->b.f[to], (R *)c->dbk[to],
-                                                        mask, io->count);
+            k_put_sites<R><<<nb, 256, lds, c->stream>>>((const double *)buf, L, pb, (uint32_t)(skip + at / rec), n,
+                                                        (R *)c->b.f[to], (R *)c->dbk[to], mask, io->count);
         };
         is_dev(c) ? go(float()) : go(double());
     }));

@@ -168,34 +168,28 @@ __global__ __launch_bounds__(256) void k_get_sites(const R *__restrict__ f, cons
         out[(size_t)first * (uint32_t)L.sd + q] = rec[q];
 }
 
-// Interior sites [s0, s0 + n) from records of the z planes that in starts
-// with (plane z0 of the halo'd lattice): populations, dipoles and the rock
-// mask (mask may be nullptr); *nrock counts the rock sites.
+// Records [r0, r0 + n) of the lattice (z slowest, halo included), which in
+// starts with: populations, dipoles and the rock mask (mask may be nullptr) of
+// those that are interior sites; *nrock counts the rock sites.
 template <typename R>
-__global__ __launch_bounds__(256) void k_put_sites(const double *__restrict__ in, uint32_t z0, RecLayout L,
-                                                   PopBase b, uint32_t s0, uint32_t n, R *__restrict__ f,
-                                                   R *__restrict__ db, uint8_t *__restrict__ mask,
-                                                   uint32_t *__restrict__ nrock)
+__global__ __launch_bounds__(256) void k_put_sites(const double *__restrict__ in, RecLayout L, PopBase b, uint32_t r0,
+                                                   uint32_t n, R *__restrict__ f, R *__restrict__ db,
+                                                   uint8_t *__restrict__ mask, uint32_t *__restrict__ nrock)
 {
     extern __shared__ double rec[];
-    __shared__ size_t off[REC_SITES];  // first double of each record
     const int j = (int)(threadIdx.x % REC_SITES), g = (int)(threadIdx.x / REC_SITES);
     const uint32_t first = blockIdx.x * REC_SITES;
     const uint32_t m = n - first < (uint32_t)REC_SITES ? n - first : (uint32_t)REC_SITES;
-    const uint32_t s = s0 + first + (uint32_t)j;
-    if (g == 0 && (uint32_t)j < m) {
-        const uint32_t t = s / (uint32_t)L.nx, x = s - t * (uint32_t)L.nx;
-        const uint32_t z = t / (uint32_t)L.ny, y = t - z * (uint32_t)L.ny;
-        const size_t lx = (size_t)(L.nx + 2 * L.h), ly = (size_t)(L.ny + 2 * L.h);
-        off[j] = ((x + L.h) + lx * ((y + L.h) + ly * (size_t)(z + L.h - z0))) * (size_t)L.sd;
-    }
-    __syncthreads();
-    for (uint32_t q = threadIdx.x; q < m * (uint32_t)L.sd; q += 256u) {
-        const uint32_t r = q / (uint32_t)L.sd;
-        rec[q] = in[off[r] + (q - r * (uint32_t)L.sd)];
-    }
+    for (uint32_t q = threadIdx.x; q < m * (uint32_t)L.sd; q += 256u)
+        rec[q] = in[(size_t)first * (uint32_t)L.sd + q];
     __syncthreads();
     if ((uint32_t)j >= m) return;
+    const uint32_t r = r0 + first + (uint32_t)j, h = (uint32_t)L.h;
+    const uint32_t lx = (uint32_t)L.nx + 2u * h, ly = (uint32_t)L.ny + 2u * h;
+    // (a halo coordinate below 0 is a large unsigned one)
+    const uint32_t t = r / lx, x = r - t * lx - h, y = t % ly - h, z = t / ly - h;
+    if (x >= (uint32_t)L.nx || y >= (uint32_t)L.ny || z >= (uint32_t)L.nz) return;
+    const uint32_t s = x + (uint32_t)L.nx * (y + (uint32_t)L.ny * z);
     const double *S = rec + j * L.sd;
     for (int p = g; p < 19 * L.C; p += 4) {
         const int c = p / 19, i = p % 19;
@@ -284,8 +278,7 @@ class CopyCrew {
 
 // Transfers in pieces through two pinned buffers: while one piece crosses
 // PCIe, the one before it is copied to (or from) the caller's memory.  The
-// buffers grow to what is asked of them (pieces of IO_PIECE bytes, or one
-// z plane of records).
+// buffers grow to what is asked of them, at most IO_PIECE bytes each.
 constexpr size_t IO_PIECE = 8u << 20;
 struct HostIO {
     int device = -1;

@@ -214,3 +214,29 @@ def test_transfers_of_several_threads_do_not_mix():
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("precision", [LB3D_FP64, LB3D_FP32_DEV])
+@pytest.mark.parametrize("dims,halo,ncomp", [((150, 149, 3), 1, 2), ((211, 97, 2), 3, 3), ((31, 5, 3000), 2, 2),
+                                              ((40000, 1, 1), 1, 2)])
+def test_uploads_in_several_pieces(precision, dims, halo, ncomp):
+    """Records that cross to the device in pieces, which end anywhere in a row
+    or its halo: populations, dipoles and rock sites as uploaded, whatever the
+    halo records hold."""
+    rng = np.random.default_rng(11)
+    g = Lattice(*dims, ncomp=ncomp, precision=precision)
+    nx, ny, nz = dims
+    N = np.full((nz + 2 * halo, ny + 2 * halo, nx + 2 * halo, g.site_doubles), np.nan)
+    sites = N[halo:-halo, halo:-halo, halo:-halo]
+    sites[...] = rng.random(sites.shape)
+    sites[..., -1] = rng.random((nz, ny, nx)) < 0.3 if ncomp == 2 else 0.0
+    g.upload_sites(N, halo_extent=halo)
+    want = np.stack([np.moveaxis(sites[..., 24 * c:24 * c + 19], -1, 0) for c in range(ncomp)])
+    tol = 0.0 if precision == LB3D_FP64 else 2.0**-24  # the deviations are below 1
+    assert np.abs(g.populations() - want).max() <= tol
+    got = g.download_sites(halo)
+    assert np.isfinite(got).all()
+    got = got[halo:-halo, halo:-halo, halo:-halo]
+    if ncomp == 3:
+        assert np.abs(got[..., 75:78] - sites[..., 75:78]).max() <= tol
+    assert np.array_equal(got[..., -1], sites[..., -1])

@@ -29,3 +29,19 @@ def test_read_backs_and_uploads_run_on_the_contexts_device(so):
         assert d.value == 0
         assert len(log()) > 10
     """)
+
+
+@pytest.mark.parametrize("dims,halo,ncomp", [((300, 300, 2), 1, 2), ((400, 120, 1), 3, 3)])
+def test_transfer_buffers_do_not_grow_with_the_plane(so, dims, halo, ncomp):
+    """A z plane of records larger than a piece: the pinned and device buffers
+    of an upload stay those of a piece."""
+    fakehip.run(so, f"""
+        dims, h, ncomp = {dims}, {halo}, {ncomp}
+        g = Lattice(*dims, ncomp=ncomp)
+        knob("fake_largest_device").value = 0
+        g.upload_sites(np.zeros((dims[2] + 2 * h, dims[1] + 2 * h, dims[0] + 2 * h, g.site_doubles)), halo_extent=h)
+        g.download_sites(h)
+        assert sum("put_sites" in l for l in log()) > 1
+        for k in ("fake_largest_pinned", "fake_largest_device"):
+            assert 0 < knob(k).value <= 8 << 20, (k, knob(k).value)
+    """)

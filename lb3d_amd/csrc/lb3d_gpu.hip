@@ -206,7 +206,7 @@ HostIO *io_lend()
 
 void io_give_back(HostIO *io)
 {
-    if (io->cap <= IO_KEPT_BYTES) {
+    if (!io->pageable) {
         std::lock_guard<std::mutex> lock(g_io_mu);
         if (g_io_users > 0)
             for (HostIO *&q : g_io)
@@ -472,11 +472,11 @@ int lb3d_gpu_create(const lb3d_params *p, lb3d_ctx **out)
         const size_t edges = EDGE_SITES * plane * rs;
         if ((e = hipMalloc(&c->b.edge_pc, edges)) != hipSuccess || (e = hipMalloc(&c->b.edge_adv, edges)) != hipSuccess)
             return cleanup(LB3D_ENOMEM, std::string("hipMalloc LE edge columns: ") + hipGetErrorString(e));
-        for (int k = 0; k < 2; k++)
-            if ((e = hipMalloc(&c->facek[k], 2 * 2 * 19 * plane * rs)) != hipSuccess)
-                return cleanup(LB3D_ENOMEM, std::string("hipMalloc LE planes: ") + hipGetErrorString(e));
-        if ((e = hipMalloc(&c->b.face_aux, 2 * 4 * plane * rs)) != hipSuccess)
+        const size_t faces = 2 * 2 * 19 * plane * rs, step = (faces + 255) / 256 * 256;
+        if ((e = hipMalloc(&c->facek[0], step + faces)) != hipSuccess ||
+            (e = hipMalloc(&c->b.face_aux, 2 * 4 * plane * rs)) != hipSuccess)
             return cleanup(LB3D_ENOMEM, std::string("hipMalloc LE planes: ") + hipGetErrorString(e));
+        c->facek[1] = (char *)c->facek[0] + step;
     }
     set_cur(c, 0);
     if ((e = hipMalloc((void **)&c->b.le, sizeof(LEState))) != hipSuccess ||
@@ -507,8 +507,7 @@ int lb3d_gpu_destroy(lb3d_ctx *c)
         if (c->dbk[k]) (void)hipFree(c->dbk[k]);
     if (c->b.edge_pc) (void)hipFree(c->b.edge_pc);
     if (c->b.edge_adv) (void)hipFree(c->b.edge_adv);
-    for (int k = 0; k < 2; k++)
-        if (c->facek[k]) (void)hipFree(c->facek[k]);
+    if (c->facek[0]) (void)hipFree(c->facek[0]);  // (one allocation)
     if (c->b.face_aux) (void)hipFree(c->b.face_aux);
     if (c->b.le) (void)hipFree(c->b.le);
     if (c->d_partials) (void)hipFree(c->d_partials);
@@ -598,11 +597,10 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
     const int to = 1 - c->b.cur;
     // the records of the z planes that hold sites
     const size_t plane = (size_t)(p.nx + 2 * h) * (size_t)(p.ny + 2 * h), skip = (size_t)h * plane;
-    const size_t rec = (size_t)sd * 8, lds = (size_t)REC_SITES * rec;
-    const size_t piece = IO_PIECE / (REC_SITES * rec) * (REC_SITES * rec);  // whole blocks of records
-    HIP_TRY(io->ensure(1));
+    const size_t rec = (size_t)sd * 8, lds = (size_t)REC_SITES * rec;  // bytes of a record and of a block of them
+    HIP_TRY(io->counter());
     HIP_TRY(hipMemsetAsync(io->count, 0, sizeof(uint32_t), c->stream));
-    HIP_TRY(io->up(c->stream, N + skip * sd, (size_t)p.nz * plane * rec, piece, [&](size_t at, size_t len, void *buf) {
+    HIP_TRY(io->up(c->stream, N + skip * sd, (size_t)p.nz * plane * rec, lds, [&](size_t at, size_t len, void *buf) {
         const uint32_t n = (uint32_t)(len / rec), nb = (n + REC_SITES - 1) / REC_SITES;
         auto go = [&](auto r) {
             using R = decltype(r);
@@ -693,10 +691,9 @@ int lb3d_gpu_download_sites(lb3d_ctx *c, double *N, int32_t h, int32_t sd)
     const RecLayout L = rec_layout(c->p, h, sd);
     const PopBase pb = pop_base(c->p);
     const size_t recs = (size_t)(c->p.nx + 2 * h) * (size_t)(c->p.ny + 2 * h) * (size_t)(c->p.nz + 2 * h);
-    const size_t rec = (size_t)sd * 8, lds = (size_t)REC_SITES * rec;
-    const size_t piece = IO_PIECE / (REC_SITES * rec) * (REC_SITES * rec);  // whole blocks of records
+    const size_t rec = (size_t)sd * 8, lds = (size_t)REC_SITES * rec;  // bytes of a record and of a block of them
     IoLoan io;
-    HIP_TRY(io->down(c->stream, N, recs * rec, piece, [&](size_t at, size_t len, void *buf) -> const void * {
+    HIP_TRY(io->down(c->stream, N, recs * rec, lds, true, [&](size_t at, size_t len, void *buf) -> const void * {
         const uint32_t n = (uint32_t)(len / rec), nb = (n + REC_SITES - 1) / REC_SITES;
         auto go = [&](auto r) {
             using R = decltype(r);

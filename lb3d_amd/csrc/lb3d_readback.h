@@ -15,6 +15,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <thread>
 
@@ -278,45 +279,99 @@ class CopyCrew {
 
 // Transfers in pieces through two pinned buffers: while one piece crosses
 // PCIe, the one before it is copied to (or from) the caller's memory.  The
-// buffers grow to what is asked of them, at most IO_PIECE bytes each.
+// buffers grow to what is asked of them, at most IO_PIECE bytes each.  Where
+// no memory can be pinned they are pageable, and where the device has no room
+// for a piece the pieces are smaller: slower, but nothing that copies straight
+// to the caller's pages could do is refused.
 constexpr size_t IO_PIECE = 8u << 20;
 struct HostIO {
     int device = -1;
     void *pin[2] = {nullptr, nullptr}, *dev[2] = {nullptr, nullptr};
     hipEvent_t ev[2] = {nullptr, nullptr};
     uint32_t *count = nullptr;  // device counter of an upload's rock sites
-    size_t cap = 0;
-    hipError_t ensure(size_t n)
+    size_t host_cap = 0, dev_cap = 0;
+    bool pageable = false;
+    static size_t round_up(size_t n) { return (n + 65535) & ~(size_t)65535; }
+    hipError_t counter()
     {
+        return count ? hipSuccess : hipMalloc((void **)&count, sizeof(uint32_t));
+    }
+    // Host buffers of n bytes.
+    hipError_t host_room(size_t n)
+    {
+        if (n <= host_cap) return hipSuccess;
+        free_host();
+        n = round_up(n);
+        for (void *&q : pin)
+            if (!pageable && hipHostMalloc(&q, n, hipHostMallocPortable) != hipSuccess) {
+                q = nullptr;
+                (void)hipGetLastError();
+                pageable = true;
+            }
+        if (pageable) {
+            if (pin[0]) (void)hipHostFree(pin[0]);
+            for (void *&q : pin) q = std::malloc(n);
+            if (!pin[0] || !pin[1]) {
+                free_host();
+                return hipErrorOutOfMemory;
+            }
+        }
+        host_cap = n;
+        return hipSuccess;
+    }
+    // Device buffers of n bytes, or as many as can be had, at least `least`.
+    hipError_t dev_room(size_t n, size_t least)
+    {
+        if (n <= dev_cap) return hipSuccess;
+        free_dev();
+        for (n = round_up(n);; n = round_up(n / 2)) {
+            hipError_t e = hipMalloc(&dev[0], n);
+            if (e != hipSuccess) dev[0] = nullptr;
+            if (e == hipSuccess && (e = hipMalloc(&dev[1], n)) != hipSuccess) dev[1] = nullptr;
+            if (e == hipSuccess) break;
+            (void)hipGetLastError();
+            free_dev();
+            if (n <= round_up(least)) return e;
+        }
+        dev_cap = n;
+        return hipSuccess;
+    }
+    // The bytes of a piece, whole units, for a transfer of total; room: the
+    // pieces need device memory of their own.
+    hipError_t prepare(size_t total, size_t unit, bool room, size_t *piece)
+    {
+        size_t n = unit < IO_PIECE ? IO_PIECE / unit * unit : unit;
+        const size_t want = total < n ? total : n;
         hipError_t e = hipSuccess;
         for (int j = 0; j < 2 && e == hipSuccess; j++)
             if (!ev[j]) e = hipEventCreateWithFlags(&ev[j], hipEventDisableTiming);
-        if (e == hipSuccess && !count) e = hipMalloc((void **)&count, sizeof(uint32_t));
-        if (e != hipSuccess || n <= cap) return e;
-        free_buffers();
-        n = (n + 65535) & ~(size_t)65535;
-        for (int j = 0; j < 2 && e == hipSuccess; j++) {
-            e = hipHostMalloc(&pin[j], n, hipHostMallocPortable);
-            if (e == hipSuccess) e = hipMalloc(&dev[j], n);
-        }
-        if (e == hipSuccess)
-            cap = n;
-        else
-            free_buffers();
+        if (e == hipSuccess && room) e = dev_room(want, total < unit ? total : unit);
+        if (room && dev_cap < want) n = dev_cap < unit ? unit : dev_cap / unit * unit;
+        if (e == hipSuccess) e = host_room(total < n ? total : n);
+        *piece = n;
         return e;
     }
-    void free_buffers()
+    void free_host()
     {
-        for (int j = 0; j < 2; j++) {
-            if (pin[j]) (void)hipHostFree(pin[j]);
-            if (dev[j]) (void)hipFree(dev[j]);
-            pin[j] = dev[j] = nullptr;
+        for (void *&q : pin) {
+            if (q) pageable ? std::free(q) : (void)hipHostFree(q);
+            q = nullptr;
         }
-        cap = 0;
+        pageable = false;
+        host_cap = 0;
+    }
+    void free_dev()
+    {
+        for (void *&q : dev) {
+            if (q) (void)hipFree(q);
+            q = nullptr;
+        }
+        dev_cap = 0;
     }
     void release()
     {
-        free_buffers();
+        free_host();
+        free_dev();
         for (hipEvent_t &x : ev) {
             if (x) (void)hipEventDestroy(x);
             x = nullptr;
@@ -325,12 +380,13 @@ struct HostIO {
         count = nullptr;
     }
     // dst[0..total) bytes in pieces: go(off, n, buf) returns the device memory
-    // that holds bytes [off, off + n), having launched what fills it (buf is
-    // room for a piece).
+    // that holds bytes [off, off + n), having launched what fills it (buf, with
+    // room: memory for a piece).  Pieces are whole units.
     template <typename Go>
-    hipError_t down(hipStream_t st, void *dst, size_t total, size_t piece, Go go)
+    hipError_t down(hipStream_t st, void *dst, size_t total, size_t unit, bool room, Go go)
     {
-        hipError_t e = ensure(total < piece ? total : piece);
+        size_t piece = 0;
+        hipError_t e = prepare(total, unit, room, &piece);
         if (e != hipSuccess) return e;
         CopyCrew crew(total);
         const size_t n = (total + piece - 1) / piece;
@@ -354,9 +410,10 @@ struct HostIO {
     // what reads piece [off, off + n) from buf.  All work is queued on st when
     // this returns, and src has been read.
     template <typename Go>
-    hipError_t up(hipStream_t st, const void *src, size_t total, size_t piece, Go go)
+    hipError_t up(hipStream_t st, const void *src, size_t total, size_t unit, Go go)
     {
-        hipError_t e = ensure(total < piece ? total : piece);
+        size_t piece = 0;
+        hipError_t e = prepare(total, unit, true, &piece);
         if (e != hipSuccess) return e;
         CopyCrew crew(total);
         size_t k = 0;
@@ -399,11 +456,12 @@ class OnDevice {
 // Transfer buffers are lent for one call and shared by all contexts (pinning
 // them takes about 4 ms, more than a small lattice's whole run between two
 // dumps): IoLoan takes a set of the current device from a pool, or a new one,
-// and gives it back.  The pool keeps at most IO_KEPT sets of at most
-// IO_KEPT_BYTES per buffer and frees them when the last context goes
-// (io_users counts contexts); loans of several threads are different sets.
-// The borrower's work on the set is complete when the loan ends.
-constexpr size_t IO_KEPT = 4, IO_KEPT_BYTES = 32u << 20;
+// and gives it back.  The pool keeps at most IO_KEPT sets, of at most 2 IO_PIECE
+// bytes pinned and as many on the device each (64 MiB and 64 MiB in all), and
+// frees them when the last context goes (io_users counts contexts); sets of
+// pageable memory it does not keep.  Loans of several threads are different
+// sets.  The borrower's work on the set is complete when the loan ends.
+constexpr size_t IO_KEPT = 4;
 HostIO *io_lend();
 void io_give_back(HostIO *io);
 void io_users(int change);
@@ -423,7 +481,7 @@ template <typename Go>
 hipError_t fetch_f64(hipStream_t st, double *dst, uint64_t n, Go go)
 {
     IoLoan io;
-    return io->down(st, dst, n * sizeof(double), IO_PIECE, [&](size_t off, size_t len, void *buf) -> const void * {
+    return io->down(st, dst, n * sizeof(double), 65536, true, [&](size_t off, size_t len, void *buf) -> const void * {
         go((uint32_t)(off / sizeof(double)), (uint32_t)(len / sizeof(double)), (double *)buf);
         return buf;
     });
@@ -437,7 +495,7 @@ hipError_t fetch_populations(hipStream_t st, const lb3d_params &p, const void *f
     const uint64_t n = (uint64_t)p.ncomp * 19u * ns;
     if constexpr (sizeof(R) == 8) {  // as stored
         IoLoan io;
-        return io->down(st, out, n * 8, IO_PIECE,
+        return io->down(st, out, n * 8, 65536, false,
                        [&](size_t off, size_t, void *) -> const void * { return (const char *)f + off; });
     } else {
         const PopBase b = pop_base(p);

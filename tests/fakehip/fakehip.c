@@ -20,7 +20,8 @@ static char *log_buf;
 static size_t log_len, log_cap;
 
 /* knobs and counters for the tests */
-int fake_fail_pinned;                       /* pinned allocations fail */
+int fake_fail_pinned;                       /* 1: pinned allocations fail, 2: every second one */
+size_t fake_device_fill;                    /* device memory starts out as the doubles 0, 1, 2, ... */
 size_t fake_device_limit = (size_t)-1;      /* largest device allocation that succeeds */
 size_t fake_largest_pinned, fake_largest_device, fake_live_pinned;
 
@@ -60,6 +61,8 @@ static int add(void **p, size_t n, int kind)
     mem *m = malloc(sizeof *m);
     m->p = calloc(n ? n : 1, 1);
     m->n = n ? n : 1;
+    if (kind == DEVICE && fake_device_fill)
+        for (size_t k = 0; k < n / 8; k++) ((double *)m->p)[k] = (double)k;
     m->kind = kind;
     m->dev = cur_dev;
     m->next = mems;
@@ -91,7 +94,8 @@ int hipFree(void *p) { return drop(p, DEVICE); }
 int hipHostMalloc(void **p, size_t n, unsigned flags)
 {
     (void)flags;
-    if (fake_fail_pinned) return fail(ENOMEM_);
+    static int calls;
+    if (fake_fail_pinned == 1 || (fake_fail_pinned == 2 && ++calls % 2 == 0)) return fail(ENOMEM_);
     if (n > fake_largest_pinned) fake_largest_pinned = n;
     fake_live_pinned += n;
     return add(p, n, PINNED);

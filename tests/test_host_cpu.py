@@ -45,3 +45,38 @@ def test_transfer_buffers_do_not_grow_with_the_plane(so, dims, halo, ncomp):
         for k in ("fake_largest_pinned", "fake_largest_device"):
             assert 0 < knob(k).value <= 8 << 20, (k, knob(k).value)
     """)
+
+
+def test_transfers_without_pinned_memory(so):
+    """Where nothing can be pinned the transfers go through pageable memory, and
+    through pinned memory again once it can be had."""
+    fakehip.run(so, """
+        g = Lattice(70, 60, 40, ncomp=2)          # 51 MB of populations
+        batch = Batch([(8, 6, 6), (6, 6, 6)], ncomp=3)
+        knob("fake_device_fill").value = 1
+        other = Lattice(70, 60, 40, ncomp=2)
+        want = np.arange(2 * 19 * 40 * 60 * 70, dtype=float).reshape(2, 19, 40, 60, 70)
+        fail = knob("fake_fail_pinned", ctypes.c_int)
+        for fail.value in (1, 2, 0):
+            assert np.array_equal(other.populations(), want)
+            g.density(), g.momentum(), batch.populations(0)
+            g.upload_sites(g.download_sites())
+            assert (knob("fake_live_pinned").value > 0) == (fail.value == 0)
+    """)
+
+
+@pytest.mark.parametrize("limit", [3 << 20, 100 << 10, 65536])
+def test_transfers_on_a_full_device(so, limit):
+    """Conversion pieces shrink to the device memory that is left, and FP64
+    populations, which need none, come without any."""
+    fakehip.run(so, f"""
+        lattices = [Lattice(70, 60, 40, ncomp=2, precision=p) for p in (0, 1)]
+        knob("fake_device_limit").value = {limit}
+        for g in lattices:
+            g.populations(), g.density(), g.momentum()
+            g.upload_sites(g.download_sites())
+        assert sum("get_density" in l for l in log()) >= 2 * (8 * 2 * 40 * 60 * 70) // {limit}
+        del lattices[1:]
+        knob("fake_device_limit").value = 0
+        lattices[0].populations()
+    """)

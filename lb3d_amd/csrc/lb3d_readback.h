@@ -13,12 +13,11 @@
 
 #include <hip/hip_runtime.h>
 
-#include <atomic>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
-#include <thread>
 
+#include "lb3d_copycrew.h"
 #include "lb3d_kernels.h"
 #include "lb3d_solver.h"
 
@@ -205,77 +204,6 @@ __global__ __launch_bounds__(256) void k_put_sites(const double *__restrict__ in
         if (rk) atomicAdd(nrock, 1u);
     }
 }
-
-// Copies between the caller's memory and pinned memory, by the calling thread
-// and, for large transfers, a few helpers that live for the transfer: one
-// thread writes fresh pages at 15 GB/s, a fourth of what PCIe brings.
-class CopyCrew {
-  public:
-    explicit CopyCrew(size_t total)
-    {
-        if (total < (size_t)(16u << 20)) return;
-        const unsigned hw = std::thread::hardware_concurrency();
-        const int want = hw >= 8 ? MAX_HELPERS : (hw >= 4 ? 1 : 0);
-        try {
-            for (; n_ < want; n_++) th_[n_] = std::thread([this, i = n_] { work(i); });
-        } catch (...) {  // no thread to be had: fewer helpers
-        }
-    }
-    CopyCrew(const CopyCrew &) = delete;
-    CopyCrew &operator=(const CopyCrew &) = delete;
-    ~CopyCrew()
-    {
-        stop_.store(true, std::memory_order_release);
-        for (int i = 0; i < n_; i++) th_[i].join();
-    }
-    void copy(void *d, const void *s, size_t n)
-    {
-        if (n_ == 0 || n < (size_t)(1u << 20)) {
-            std::memcpy(d, s, n);
-            return;
-        }
-        d_ = (char *)d;
-        s_ = (const char *)s;
-        bytes_ = n;
-        done_.store(0, std::memory_order_relaxed);
-        parts_ = n_ + 1;
-        job_.fetch_add(1, std::memory_order_release);
-        slice(parts_ - 1);
-        while (done_.load(std::memory_order_acquire) != n_) std::this_thread::yield();
-    }
-
-  private:
-    static constexpr int MAX_HELPERS = 3;
-    void slice(int i) const
-    {
-        // whole pages per helper
-        const size_t per = ((bytes_ + parts_ - 1) / parts_ + 4095) & ~(size_t)4095;
-        const size_t at = per * (size_t)i;
-        if (at < bytes_) std::memcpy(d_ + at, s_ + at, bytes_ - at < per ? bytes_ - at : per);
-    }
-    void work(int i)
-    {
-        unsigned seen = 0;
-        for (;;) {
-            unsigned j;
-            while ((j = job_.load(std::memory_order_acquire)) == seen) {
-                if (stop_.load(std::memory_order_acquire)) return;
-                std::this_thread::yield();
-            }
-            seen = j;
-            slice(i);
-            done_.fetch_add(1, std::memory_order_release);
-        }
-    }
-    std::thread th_[MAX_HELPERS];
-    int n_ = 0, parts_ = 1;
-    char *d_ = nullptr;
-    const char *s_ = nullptr;
-    size_t bytes_ = 0;
-    std::atomic<unsigned> job_{0};
-    std::atomic<int> done_{0};
-    std::atomic<bool> stop_{false};
-};
 
 // Transfers in pieces through two pinned buffers: while one piece crosses
 // PCIe, the one before it is copied to (or from) the caller's memory.  The

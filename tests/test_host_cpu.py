@@ -1,8 +1,13 @@
 """The library's host code (device bookkeeping, transfers, graphs, plans) on the
 CPU, against a stand-in for the HIP runtime (fakehip/fakehip.c)."""
+import os
+import subprocess
+
 import pytest
 
 from tests import fakehip
+
+HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 @pytest.fixture(scope="module")
@@ -80,3 +85,14 @@ def test_transfers_on_a_full_device(so, limit):
         knob("fake_device_limit").value = 0
         lattices[0].populations()
     """)
+
+
+def test_copy_threads_copy_and_rest(tmp_path):
+    """The helper threads of large transfers copy every byte and nothing else,
+    and take no processor time while the caller waits for the device."""
+    exe = str(tmp_path / "copycrew")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-pthread", "-I", os.path.join(HERE, "..", "lb3d_amd", "csrc"),
+                    os.path.join(HERE, "copycrew.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert float(r.stdout) < 0.05  # 0.3 s per helper if they spin

@@ -41,7 +41,7 @@ struct lb3d_batch {
     int device = 0;  // that the batch was made on
     hipGraphExec_t graph = nullptr;
     int graph_len = 0;       // steps of the captured graph
-    int64_t plan_steps = 0;  // steps run on the current plan (a graph is captured after GRAPH_AFTER)
+    int64_t plan_steps = 0;  // steps run on the current plan (see replay_graph)
     int cur = 0, nt = 0;
     unsigned nwg = 2048;     // persistent grid size, a multiple of 8
     uint32_t xg = 0;         // work items per XCD chunk (xcd_tile)
@@ -262,6 +262,11 @@ int build_cm(lb3d_batch *b, int cols, int lz, int threads)
     return LB3D_OK;
 }
 
+bool replays(const lb3d_batch *b, int32_t nsteps)
+{
+    return b->graph || replay_graph(b->plan_steps, nsteps, (uint64_t)b->nitems * BLOCK);
+}
+
 int ensure_graph(lb3d_batch *b)
 {
     if (b->graph) return LB3D_OK;
@@ -440,7 +445,7 @@ int lb3d_gpu_batch_run_steps(lb3d_batch *b, int32_t nsteps)
     if (nsteps == 0) return LB3D_OK;
     if (b->cm_cols && !b->aux_ok) prime_aux(b);
     int left = nsteps;
-    if (b->plan_steps >= GRAPH_AFTER) {
+    if (replays(b, nsteps)) {
         if (int rc = ensure_graph(b)) return rc;
         if (b->cur == 1) {
             enqueue_batch_step(b);
@@ -463,7 +468,7 @@ int lb3d_gpu_batch_run_steps_timed(lb3d_batch *b, int32_t nsteps, double *ms)
     // prepared before the first event: the graph, and the moments the
     // collide-moments plan carries
     int rc = LB3D_OK;
-    if (b->plan_steps >= GRAPH_AFTER && (rc = ensure_graph(b))) return rc;
+    if (replays(b, nsteps) && (rc = ensure_graph(b))) return rc;
     if (b->cm_cols && !b->aux_ok) prime_aux(b);
     hipEvent_t e[2] = {nullptr, nullptr};
     struct Ev {

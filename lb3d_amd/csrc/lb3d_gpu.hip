@@ -97,7 +97,7 @@ struct lb3d_ctx {
     LEState host_le{};
     hipGraphExec_t graph = nullptr;
     int graph_len = 0;     // steps of the captured graph
-    int64_t plan_steps = 0;  // steps run on the current plan (a graph is captured after GRAPH_AFTER)
+    int64_t plan_steps = 0;  // steps run on the current plan (see replay_graph)
     double *d_partials = nullptr;
     uint8_t *rock_dev = nullptr;  // rock mask (lattices with walls)
     size_t f_bytes = 0, aux_bytes = 0, db_bytes = 0;
@@ -873,6 +873,11 @@ static int ensure_graph(lb3d_ctx *c)
     return LB3D_OK;
 }
 
+static bool replays(const lb3d_ctx *c, int32_t nsteps)
+{
+    return c->graph || replay_graph(c->plan_steps, nsteps, (uint64_t)c->p.nx * c->p.ny * c->p.nz);
+}
+
 static int sync_le_counter(lb3d_ctx *c)
 {
     if (!c->le) return LB3D_OK;
@@ -897,7 +902,7 @@ int lb3d_gpu_run_steps(lb3d_ctx *c, int32_t nsteps)
     if (rc) return rc;
     ensure_edges(c);
     int left = nsteps;
-    if (c->plan_steps >= GRAPH_AFTER) {
+    if (replays(c, nsteps)) {
         if ((rc = ensure_graph(c))) return rc;
         if (c->b.cur == 1) {
             if ((rc = enqueue_step(c))) return rc;
@@ -922,7 +927,7 @@ int lb3d_gpu_run_steps_timed(lb3d_ctx *c, int32_t nsteps, double *ms)
     if (c->state != IDLE) return fail(LB3D_ESTATE, "run_steps needs a completed timestep");
     int rc = sync_le_counter(c);
     if (rc) return rc;
-    if (c->plan_steps >= GRAPH_AFTER && (rc = ensure_graph(c))) return rc;
+    if (replays(c, nsteps) && (rc = ensure_graph(c))) return rc;
     Events ev(2);
     HIP_TRY(ev.create());
     hipEvent_t e0 = ev[0], e1 = ev[1];

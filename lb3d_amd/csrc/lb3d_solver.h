@@ -50,9 +50,19 @@ Plan two_pass_plan(const lb3d_params &p);
 // graph launch costs about 4 us more than a kernel launch, a kernel inside it
 // about 0.4 us less, and capturing one 0.4-0.7 ms plus 10 us per kernel.  So
 // a graph holds an even number of steps of at least GRAPH_KERNELS kernels, and
-// is captured once GRAPH_AFTER steps on one plan have shown a long run.
+// is captured once GRAPH_AFTER steps on one plan have shown a long run, or where
+// one call of twice as many steps says so beforehand, if the kernels are about
+// as short as a launch.  That call, plain and with the capture (us a step):
+// 2,048 steps of 16^3 binary FP32 7.7 / 6.5, FP64 7.7 / 7.5, 32^3 FP64 9.46 /
+// 9.49, 16^3 ternary FP64 17.1 / 16.2, 32^3 FP32 14.6 / 14.1, 32^3 Lees-Edwards
+// 20.6 / 20.2; 48^3 binary FP32 10.9 / 11.3, FP64 17.9 / 18.2.
 constexpr int GRAPH_KERNELS = 48;
 constexpr int64_t GRAPH_AFTER = 1024;
+constexpr uint64_t GRAPH_SITES = 40000;
+inline bool replay_graph(int64_t steps_before, int64_t steps, uint64_t sites)
+{
+    return steps_before >= GRAPH_AFTER || (steps >= 2 * GRAPH_AFTER && sites <= GRAPH_SITES);
+}
 inline int graph_steps(int kernels_per_step)
 {
     const int k = (GRAPH_KERNELS + 2 * kernels_per_step - 1) / (2 * kernels_per_step);

@@ -96,3 +96,49 @@ def test_copy_threads_copy_and_rest(tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
     assert float(r.stdout) < 0.05  # 0.3 s per helper if they spin
+
+
+STEPS_DONE = """
+    def steps(kernels):
+        \"\"\"Whole steps in the log, of so many kernels each, and the graphs replayed.\"\"\"
+        plain = graphs = replayed = 0
+        for l in log():
+            plain += l.startswith("launch")
+            if l.startswith("graph"):
+                graphs += 1
+                replayed += int(l.split()[1])
+        assert (plain + replayed) % kernels == 0
+        return (plain + replayed) // kernels, graphs
+"""
+
+
+def test_one_long_call_replays_a_graph(so):
+    """A fresh lattice that is asked for a long run in one call replays a graph
+    in that call where launches count (small lattices), runs as many steps as it
+    was asked for, and captures nothing for a short call."""
+    fakehip.run(so, STEPS_DONE + """
+    def fresh(n, **kw):
+        g = Lattice(n, n, n, **kw)
+        g.init_noise(1); g.bc_init(); log()
+        return g
+    for n, call, replays in ((16, 2047, False), (16, 2048, True), (16, 100001, True), (48, 5000, False)):
+        g = fresh(n, ncomp=2)
+        g.time_loop(call)
+        done, graphs = steps(2)
+        assert done == call and graphs == (call // 24 if replays else 0), (n, call, done, graphs)
+    g = fresh(16, ncomp=2)
+    g.time_loop_timed(4001)
+    assert steps(2)[0] == 4001
+    g.time_loop(51)             # the graph is there: shorter calls replay it too
+    assert steps(2) == (51, 2)
+    g = fresh(64, ncomp=2)
+    g.time_loop(1024)
+    assert steps(2) == (1024, 0)
+    g.time_loop(100)            # a run that has shown to be long, of any size
+    assert steps(2) == (100, 4)
+    b = Batch([(16, 16, 16), (8, 8, 8)], ncomp=3)
+    b.init_noise(0, 1), b.init_noise(1, 2), log()
+    b.time_loop(3000)
+    done, graphs = steps(3)
+    assert done == 3000 and graphs > 0
+    """)

@@ -849,7 +849,8 @@ static int ensure_graph(lb3d_ctx *c)
 {
     if (c->graph) return LB3D_OK;
     // an even number of steps starting from cur = 0 (A -> B -> ... -> A)
-    const int len = graph_steps(c->plan.fused ? (c->le ? 3 : 1) : (c->le ? 4 : c->p.ncomp));
+    const int kernels = c->plan.fused ? (c->le ? 3 : 1) : (c->le ? 4 : (c->L->small() ? 2 : c->p.ncomp));
+    const int len = graph_steps(kernels);
     int saved = c->b.cur;
     set_cur(c, 0);
     hipGraph_t g = nullptr;

@@ -142,3 +142,29 @@ def test_one_long_call_replays_a_graph(so):
     done, graphs = steps(3)
     assert done == 3000 and graphs > 0
     """)
+
+
+def test_graphs_hold_at_least_48_kernels(so):
+    """A captured graph holds an even number of steps of at least 48 kernels in
+    all, and not two steps more than that takes, on every plan."""
+    fakehip.run(so, """
+    LE = dict(boundary=LB3D_BC_LEES_EDWARDS, shear_u=0.02)
+    forms = [(dict(ncomp=2), None, 2), (dict(ncomp=2), (1, 32, 4, 4), 1), (LE, None, 4), (LE, (2, 32, 4, 4), 3),
+             (dict(ncomp=3, precision=LB3D_FP32_DEV), None, 2),       # dipoles and collision in one launch
+             (dict(ncomp=3), None, 3), (dict(ncomp=3), (3, 32, 4, 4), 1)]
+    for kw, plan, kernels in forms:
+        g = Lattice(8, 8, 8, **kw)
+        if plan:
+            g.set_plan(*plan)
+        g.init_noise(1)
+        g.time_loop(1)
+        log()
+        g.time_loop(1)
+        assert len(log()) == kernels, (kw, plan)
+        g.time_loop(1024)
+        g.time_loop(200)
+        sizes = {int(l.split()[1]) for l in log() if l.startswith("graph")}
+        assert len(sizes) == 1
+        size = sizes.pop()
+        assert 48 <= size < 48 + 2 * kernels and size % (2 * kernels) == 0, (kw, plan, size)
+    """)

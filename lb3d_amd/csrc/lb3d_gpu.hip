@@ -284,6 +284,9 @@ Plan two_pass_plan(const lb3d_params &p)
     return q;
 }
 
+// The search visits each tile width and each chunk length once and ends where
+// nothing shorter can cost less (lb3d_gpu_step_noalloc does it in every call: some us
+// at most, 2 ms for a column of 400,000 planes when every number of chunks was tried).
 Plan default_plan(const lb3d_params &p)
 {
     Plan q = two_pass_plan(p);
@@ -294,8 +297,9 @@ Plan default_plan(const lb3d_params &p)
     if (sites < (le ? (fp64 ? 500000 : 1000000) : (fp64 ? 400000 : 600000))) return q;
     const int T = 512, CUS = 256;
     double best = 0.0;
-    for (int kx = 1; kx <= p.nx; kx++) {
-        const int tx = (p.nx + kx - 1) / kx;
+    // (the smallest number of tiles of each width: more of them cost more)
+    for (int kx = (p.nx + T - 1) / T, tx; ; kx = (p.nx + tx - 2) / (tx - 1)) {
+        tx = (p.nx + kx - 1) / kx;
         if (tx < (le && !fp64 ? 48 : 16) && kx > 1) break;
         int ty = T / tx < p.ny ? T / tx : p.ny;
         if (ty > fused2_sites(T) / (tx + 2) - 2) ty = fused2_sites(T) / (tx + 2) - 2;
@@ -315,14 +319,17 @@ Plan default_plan(const lb3d_params &p)
     }
     if (!q.fused) return q;
     const int64_t tiles = (int64_t)((p.nx + q.tx - 1) / q.tx) * ((p.ny + q.ty - 1) / q.ty);
+    const int64_t least = (tiles * p.nz + CUS - 1) / CUS;  // planes in a row without those computed twice
     int64_t planes = 0;
-    for (int kz = 1; kz <= p.nz; kz++) {
-        const int lz = (p.nz + kz - 1) / kz;
-        const int64_t c = (tiles * ((p.nz + lz - 1) / lz) + CUS - 1) / CUS * (lz + 2);
+    for (int kz = 1, lz; ; kz = (p.nz + lz - 2) / (lz - 1)) {
+        lz = (p.nz + kz - 1) / kz;
+        const int64_t rounds = (tiles * ((p.nz + lz - 1) / lz) + CUS - 1) / CUS, c = rounds * (lz + 2);
         if (!planes || c < planes) {
             planes = c;
             q.lz = lz;
         }
+        // shorter chunks take as many rounds at least
+        if (lz == 1 || least + 2 * rounds >= planes) break;
     }
     q.stage = 0;
     q.xg = 32;

@@ -1,10 +1,14 @@
 """The library's host code (device bookkeeping, transfers, graphs, plans) on the
 CPU, against a stand-in for the HIP runtime (fakehip/fakehip.c)."""
+import ctypes
 import os
+import random
 import subprocess
+import timeit
 
 import pytest
 
+from lb3d_amd import gpu
 from tests import fakehip
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -168,3 +172,71 @@ def test_graphs_hold_at_least_48_kernels(so):
         size = sizes.pop()
         assert 48 <= size < 48 + 2 * kernels and size % (2 * kernels) == 0, (kw, plan, size)
     """)
+
+
+class Plan(ctypes.Structure):
+    """lb3d::Plan of csrc/lb3d_solver.h."""
+    _fields_ = [("fused", ctypes.c_bool), ("tx", ctypes.c_int), ("ty", ctypes.c_int), ("lz", ctypes.c_int),
+                ("stage", ctypes.c_int), ("xg", ctypes.c_uint32)]
+
+
+def default_plan(p):
+    f = getattr(gpu.lib(), "_ZN4lb3d12default_planERK11lb3d_params")
+    f.restype, f.argtypes = Plan, [ctypes.POINTER(gpu.Params)]
+    return f(ctypes.byref(p))
+
+
+def searched_plan(nx, ny, nz, fp64, le):
+    """The tile and z-chunk that cost least, over every number of tiles and chunks."""
+    def up(a, b):
+        return (a + b - 1) // b
+    T, best = 512, None
+    for kx in range(1, nx + 1):
+        tx = up(nx, kx)
+        if tx < (48 if le and not fp64 else 16) and kx > 1:
+            break
+        ty = min(T // tx, ny, 1040 // (tx + 2) - 2)
+        if ty < 1:
+            continue
+        ky = up(ny, ty)
+        ty = up(ny, ky)
+        if tx * ty <= T // 2:
+            continue
+        halo = 2.0 * (tx + 2) + 2.0 * ty
+        cost = float(kx) * ky * (T + 0.2 * halo if fp64 or le else T) * (1.04 + 6.0 / tx if kx > 1 else 1.0)
+        if best is None or cost < best[0]:
+            best = (cost, tx, ty)
+    if best is None:
+        return None
+    _, tx, ty = best
+    tiles = up(nx, tx) * up(ny, ty)
+    lz = min((up(tiles * up(nz, lz), 256) * (lz + 2), -lz) for lz in {up(nz, kz) for kz in range(1, nz + 1)})[1]
+    return tx, ty, -lz
+
+
+def test_untuned_plan_is_the_cheapest_of_all():
+    rng = random.Random(5)
+    dims = [(2, 1, 300000), (300000, 2, 1), (1, 1, 1), (513, 900, 3), (512, 512, 4), (256, 64, 64), (90, 100, 77)]
+    dims += [tuple(int(2 ** rng.uniform(1, 11)) for _ in range(3)) for _ in range(200)]
+    fused = 0
+    for nx, ny, nz in dims:
+        nx = max(nx, 2)
+        if not 400000 <= nx * ny * nz <= 100000000:
+            continue
+        for fp64, le, line in ((1, 0, 400000), (0, 0, 600000), (1, 1, 500000), (0, 1, 1000000)):
+            if nx * ny * nz < line:
+                continue
+            q = default_plan(gpu.make_params(nx, ny, nz, precision=0 if fp64 else 1, boundary=le))
+            want = searched_plan(nx, ny, nz, fp64, le)
+            assert ((q.tx, q.ty, q.lz) if q.fused else None) == want, (nx, ny, nz, fp64, le)
+            fused += q.fused
+    assert fused > 100
+
+
+def test_untuned_plan_is_found_at_once():
+    """lb3d_gpu_step_noalloc looks for it in every call, on a lattice of any shape."""
+    for dims in ((270, 1, 400000), (50000000, 1, 1), (3, 30000000, 1), (40, 9, 300000), (640, 7, 24999)):
+        p = gpu.make_params(*dims)
+        default_plan(p)
+        t = min(timeit.repeat(lambda: default_plan(p), number=1, repeat=5))
+        assert t < 5e-4, (dims, t)

@@ -103,6 +103,7 @@ struct lb3d_ctx {
     size_t f_bytes = 0, aux_bytes = 0, db_bytes = 0;
     size_t aux_elems = 0;  // elements of the aux field
     Plan plan;
+    Plan displaced;  // fused: the one-pass plan that walls have taken the place of
     bool tuned = false;
     // ternary dipole fields, tied to the population parity: a step reads
     // dbk[cur] (the field of the state) and writes dbk[1-cur] (the relaxed
@@ -545,7 +546,8 @@ static double rho0_of(const lb3d_ctx *c, int k) { return lb3d::rho0_of(c->p, k);
 static double w_of(int i) { return i < 18 ? 1.0 / 36.0 : 1.0 / 3.0; }
 
 // Walls on (the mask is in rock_dev) or off.  With walls only the two-pass
-// plan exists, so a one-pass plan falls back to it.
+// plan exists, so a one-pass plan falls back to it, and is back once the walls
+// are gone unless another plan has been set since.
 static void set_walls(lb3d_ctx *c, bool on)
 {
     // a captured graph holds the kernels of the old wall state (the mask
@@ -554,9 +556,13 @@ static void set_walls(lb3d_ctx *c, bool on)
     c->L->walls = on;
     c->b.rock = on ? c->rock_dev : nullptr;
     if (on && c->plan.fused) {
+        c->displaced = c->plan;
         c->plan = two_pass_plan(c->p);
-        c->L->xg = c->plan.xg;
+    } else if (!on && c->displaced.fused) {
+        c->plan = c->displaced;
+        c->displaced = Plan();
     }
+    c->L->xg = c->plan.xg;
 }
 
 // Site records.
@@ -1082,6 +1088,7 @@ int lb3d_gpu_autotune(lb3d_ctx *c, int32_t trial_steps, char *report, int32_t re
     }
     g.restore = false;
     c->plan = bestp;
+    c->displaced = Plan();
     c->L->xg = bestp.xg;
     c->tuned = true;
     drop_graph(c);
@@ -1128,6 +1135,7 @@ int lb3d_gpu_set_plan(lb3d_ctx *c, int32_t fused, int32_t tx, int32_t ty, int32_
         if (c->moments != MOMENTS_NONE) c->moments = MOMENTS_KEPT;
     }
     c->plan = q;
+    c->displaced = Plan();
     c->L->xg = q.xg;
     c->edges_ok = false;
     drop_graph(c);

@@ -385,3 +385,39 @@ def test_lees_edwards_tiles_taller_than_twice_the_lattice(precision, dims):
         g.set_plan(mode, tx, ty, dims[2])
         g.time_loop(4)
         assert np.array_equal(g.populations(), want), f"mode {mode} {tx}x{ty}"
+
+
+@pytest.mark.parametrize("dims,plan", [((20, 9, 12), (2, 32, 4, 4)), ((64, 84, 96), None)])
+def test_one_pass_plan_is_back_when_the_walls_are_gone(dims, plan):
+    """Rock sites take a one-pass lattice to the two-pass kernels; a state
+    without them runs the plan that the lattice had, unless another was set
+    while there were walls."""
+    def kernels(g):
+        return list(g.profile_steps(1)[0])
+
+    g = Lattice(*dims, ncomp=2, g_br=0.06)
+    if plan:
+        g.set_plan(*plan)
+    g.init_noise(3, amp=(0.02, 0.02, 0.0))
+    free = g.download_sites()
+    walls = free.copy()
+    walls[:, 0:2, :, -1] = 1.0
+    assert kernels(g) == ["fused"]
+    for again in ("records", "noise", "other walls, records"):
+        g.upload_sites(walls)
+        assert kernels(g) == ["moments", "collide"], again
+        if again.startswith("other"):
+            g.upload_sites(walls[::-1].copy())
+            assert kernels(g) == ["moments", "collide"], again
+        g.upload_sites(free) if "records" in again else g.init_noise(3, amp=(0.02, 0.02, 0.0))
+        assert kernels(g) == ["fused"], again
+    g.time_loop(3)
+    ref = Lattice(*dims, ncomp=2, g_br=0.06)
+    ref.set_plan(0)
+    ref.upload_sites(free)
+    ref.time_loop(4)
+    assert np.array_equal(g.populations(), ref.populations())
+    g.upload_sites(walls)
+    g.set_plan(0)
+    g.upload_sites(free)
+    assert kernels(g) == ["moments", "collide"]

@@ -382,8 +382,7 @@ void clear_error() { g_err.clear(); }
 double rho0_of(const lb3d_params &p, int k) { return p.rho0[k] > 0.0 ? p.rho0[k] : 0.7; }
 
 int aos_to_device_layout(const lb3d_params &p, const double *N, int h, int sd,
-                         std::vector<unsigned char> &f_bytes, std::vector<unsigned char> &db_bytes,
-                         std::vector<uint8_t> *rock, size_t *nrock)
+                         std::vector<unsigned char> &f_bytes, std::vector<unsigned char> &db_bytes)
 {
     const int C = p.ncomp;
     if (sd != (C == 3 ? 79 : 49)) return fail(LB3D_EINVAL, "site_doubles must be 79 (ternary) or 49 (binary)");
@@ -400,18 +399,13 @@ int aos_to_device_layout(const lb3d_params &p, const double *N, int h, int sd,
     double *fd = (double *)f_bytes.data();
     float *dbf = (float *)db_bytes.data();
     double *dbd = (double *)db_bytes.data();
-    size_t nr = 0;
-    if (rock) rock->assign(ns, 0);
     for (int z = 0; z < nz; z++)
         for (int y = 0; y < ny; y++)
             for (int x = 0; x < nx; x++) {
                 const double *S = N + ((size_t)(x + h) + lx * ((size_t)(y + h) + ly * (size_t)(z + h))) * sd;
                 size_t s = (size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * z);
-                if (S[rock_off] != 0.0) {
-                    if (!rock) return fail(LB3D_EINVAL, "rock sites are not supported here (rock_state must be 0)");
-                    (*rock)[s] = 1;
-                    nr++;
-                }
+                if (S[rock_off] != 0.0)
+                    return fail(LB3D_EINVAL, "rock sites are not supported here (rock_state must be 0)");
                 for (int k = 0; k < C; k++)
                     for (int i = 0; i < 19; i++) {
                         double v = S[24 * k + i];
@@ -429,7 +423,6 @@ int aos_to_device_layout(const lb3d_params &p, const double *N, int h, int sd,
                             dbd[k * ns + s] = S[75 + k];
                     }
             }
-    if (nrock) *nrock = nr;
     return LB3D_OK;
 }
 

@@ -171,10 +171,9 @@ int set_error(int code, const char *msg);
 void clear_error();
 // Host conversion of the reference's AoS lattice (lbe_site records) into the
 // device layout of one lattice: populations (FP64, or FP32 deviations from
-// w_i*rho0) and the ternary dipole field.  Returns 0 or an LB3D_E* code.
+// w_i*rho0) and the ternary dipole field; rock sites are refused.  Returns 0 or an LB3D_E* code.
 int aos_to_device_layout(const lb3d_params &p, const double *whole_N, int halo, int site_doubles,
-                         std::vector<unsigned char> &f_bytes, std::vector<unsigned char> &db_bytes,
-                         std::vector<uint8_t> *rock = nullptr, size_t *nrock = nullptr);
+                         std::vector<unsigned char> &f_bytes, std::vector<unsigned char> &db_bytes);
 double rho0_of(const lb3d_params &p, int c);
 
 // Parameters in the kernels' working type.

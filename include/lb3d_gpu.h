@@ -154,7 +154,9 @@ int lb3d_gpu_run_steps_timed(lb3d_ctx *ctx, int32_t nsteps, double *ms);
 /* Autotuner (not a reference routine): times every execution plan of this
  * lattice -- the two-pass kernels and, for binary lattices, the one-pass
  * z-march kernel with a fitted tile and over its tile shapes and z-chunks, then the XCD chunking of
- * the best -- on trial_steps trial steps each, keeps the fastest and writes a
+ * the best -- on trial_steps trial steps each, then the best of each kind and
+ * the untuned plan over real steps on a copy of the state (if there is memory
+ * for one), keeps the untuned plan or the fastest that beats it, and writes a
  * text report (may be NULL).  The lattice state is unchanged. */
 int lb3d_gpu_autotune(lb3d_ctx *ctx, int32_t trial_steps, char *report, int32_t report_len);
 /* Choose the execution plan directly: fused = 0 (two-pass), 1 (one-pass

@@ -39,6 +39,11 @@ struct Plan {
     int stage = 1;      // plane k's populations: 0 registers, 1 LDS, 2 pulled again
     uint32_t xg = 0;    // tiles per XCD chunk (xcd_tile): 1 plain order, 0 one run per XCD
 };
+inline bool same_plan(const Plan &a, const Plan &b)
+{
+    if (a.fused != b.fused || a.xg != b.xg) return false;
+    return !a.fused || (a.tx == b.tx && a.ty == b.ty && a.lz == b.lz && a.stage == b.stage);
+}
 // The plan of a lattice that nobody has tuned, and its two-pass plan.
 Plan default_plan(const lb3d_params &p);
 Plan two_pass_plan(const lb3d_params &p);

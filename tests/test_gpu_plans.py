@@ -421,3 +421,37 @@ def test_one_pass_plan_is_back_when_the_walls_are_gone(dims, plan):
     g.set_plan(0)
     g.upload_sites(free)
     assert kernels(g) == ["moments", "collide"]
+
+
+@pytest.mark.parametrize("dims,kw", [
+    ((24, 16, 12), dict(ncomp=2)), ((24, 16, 12), dict(ncomp=3)), ((96, 80, 80), dict(ncomp=2)),
+    ((70, 9, 6), dict(ncomp=2, boundary=LB3D_BC_LEES_EDWARDS, shear_u=0.05)),
+    ((96, 80, 80), dict(ncomp=2, boundary=LB3D_BC_LEES_EDWARDS, shear_u=0.05)),
+])
+@pytest.mark.parametrize("steps", [2, 3])
+def test_tuner_steps_a_copy_of_the_state(dims, kw, steps):
+    """The tuner times its finalists over real steps: populations, dipoles,
+    Lees-Edwards offset and step counter are afterwards what they were, at
+    either parity; the plan it takes is the untuned one or beat it there."""
+    kw = dict(kw, precision=LB3D_FP64)
+    g = Lattice(*dims, **kw)
+    g.init_noise(3, amp=(0.05, 0.05, 0.05))
+    g.bc_init()
+    g.time_loop(steps)
+    pops, rec, le = g.populations(), g.download_sites(), g.le_state()
+    lines = g.autotune(1).strip().splitlines()
+    assert g.nt == steps and g.le_state() == le
+    assert np.array_equal(g.populations(), pops)
+    if kw["ncomp"] == 3:
+        assert np.array_equal(g.download_sites()[..., 75:78], rec[..., 75:78])
+    finals = [(ln.split("steps: ")[1].rsplit(" ", 2)[0], float(ln.split()[-2])) for ln in lines if "steps: " in ln]
+    plan, ms = lines[-1].split("chosen: ")[1].rsplit(" ", 2)[0], float(lines[-1].split()[-2])
+    assert len(finals) >= 2 and (plan, ms) in finals
+    assert plan == finals[0][0] or ms < finals[0][1]
+    ref = Lattice(*dims, **kw)
+    ref.set_plan(0)
+    ref.init_noise(3, amp=(0.05, 0.05, 0.05))
+    ref.bc_init()
+    ref.time_loop(steps + 4)
+    g.time_loop(4)
+    assert np.array_equal(g.populations(), ref.populations())

@@ -240,3 +240,28 @@ def test_untuned_plan_is_found_at_once():
         default_plan(p)
         t = min(timeit.repeat(lambda: default_plan(p), number=1, repeat=5))
         assert t < 5e-4, (dims, t)
+
+
+@pytest.mark.parametrize("dims,kw,kernel", [
+    ((90, 100, 77), "ncomp=2, precision=1", "k_fused2"), ((16, 12, 10), "ncomp=2", "k_moments"),
+    ((128, 96, 90), "ncomp=2, precision=1, boundary=1", "k_fused2"), ((16, 12, 10), "ncomp=3", "k_moments"),
+])
+def test_tuner_keeps_the_untuned_plan_unless_another_is_faster(so, dims, kw, kernel):
+    """Where every plan takes the same time, as on the stand-in, the tuner leaves
+    the untuned plan, and state, parity and offset; without memory for a copy of
+    the state it goes by the trials."""
+    fakehip.run(so, f"""
+        g = Lattice(*{dims}, {kw})
+        g.init_noise(1)
+        g.time_loop(3)
+        log()
+        rep = g.autotune(2).strip().splitlines()
+        assert rep[-1].startswith("chosen: ") and any(l.startswith("steps: ") for l in rep)
+        log()
+        g.time_loop(1)
+        assert any({kernel!r} in l for l in log()), rep[-1]
+        assert g.nt == 4
+        knob("fake_device_limit").value = 1 << 10
+        assert not any(l.startswith("steps: ") for l in g.autotune(2).splitlines())
+        g.time_loop(1)
+    """)

@@ -1308,9 +1308,13 @@ __device__ __forceinline__ void collide_site(const Phys<R> &P, const R *__restri
         bgk_site<R, Dev, C, BD, (NT & 2) != 0>(P, n, F, x, y, z, s, fout);
 }
 
-// NT: the populations' loads and stores with the non-temporal hint, for
-// lattices whose populations do not fit the memory-side cache (see ld_pop)
-template <typename R, bool Dev, int C, bool LE, int BD, bool Rock = false, bool ZH = false, bool NT = false>
+// Mode: how the populations are pulled and stored.  NON_TEMPORAL, for lattices
+// whose populations do not fit the memory-side cache (see ld_pop); measured on
+// MI355X (FP32 and FP64): ternary loads and stores (128^3: -6 to -8% per step),
+// binary stores only (256^3 FP64: -2%).  PULLS_FIRST: before the forces.  The
+// launcher chooses (LauncherT::pulls_first).
+enum { FORCES_FIRST = 0, PULLS_FIRST = 1, NON_TEMPORAL = 2 };
+template <typename R, bool Dev, int C, bool LE, int BD, bool Rock = false, bool ZH = false, int Mode = FORCES_FIRST>
 __global__ __launch_bounds__(256) void k_collide(Phys<R> P, const R *__restrict__ f,
                                                  const R *__restrict__ face_pc,
                                                  const R *__restrict__ aux,
@@ -1327,15 +1331,7 @@ __global__ __launch_bounds__(256) void k_collide(Phys<R> P, const R *__restrict_
         if (le_commit && blockIdx.x == 0 && threadIdx.x == 0) *le_commit = le_advance(*le_commit, P.nz, le_adv);
     uint32_t s = xcd_tile(blockIdx.x, gridDim.x, xg) * blockDim.x + threadIdx.x;
     if (s >= P.ns) return;
-    // measured on MI355X (FP32 and FP64): ternary loads and stores (128^3:
-    // -6 to -8% per step), binary stores only (256^3 FP64: -2%)
-    // Pulls before the forces (bit 2) where it measured faster, per two-pass step:
-    // binary FP32 64^3 22.1 -> 21.5 us, 112^3 133 -> 129, FP64 48^3 20.3 -> 18.9,
-    // 80^3 92 -> 89; ternary FP64 56^3 64 -> 61, 64^3 90 -> 83.  Ternary FP32
-    // (112^3 261 -> 270 us) and lattices beyond the memory-side cache (ternary
-    // FP64 128^3 731 -> 752) have more from the registers that the forces have
-    // to themselves.
-    constexpr int nt = !NT ? (C == 2 || !Dev ? 4 : 0) : (C == 3 ? 3 : 2);
+    constexpr int nt = Mode == NON_TEMPORAL ? (C == 3 ? 3 : 2) : (Mode == PULLS_FIRST ? 4 : 0);
     collide_site<R, Dev, C, LE, BD, Rock, ZH, nt>(P, f, face_pc, aux, face_aux, db, fout, s, rock, edge_pc);
 }
 

@@ -361,43 +361,78 @@ class LauncherT : public Launcher {
         }
         return true;
     }
-    template <int BD, bool NT>
+    // Whether the collide pulls before the forces, so that its loads are in flight
+    // together; otherwise the forces have the registers to themselves.  Two-pass
+    // steps, forces first against pulls first (us):
+    //   bdist 2: binary FP32 64^3 21.5 / 20.7, 108^3 124 / 121, FP64 48^3 19.7 / 17.8,
+    //     80^3 91.8 / 87.7; ternary FP64 48^3 43.0 / 41.2, 64^3 87.1 / 82.6; Lees-Edwards
+    //     and Zou-He as these or within 1%.  Ternary FP32 112^3 261 / 270, and lattices
+    //     beyond the memory-side cache (ternary FP64 128^3 731 / 752): forces first.
+    //   bdist 0: binary FP64 48^3 21.0 / 19.9, but 56^3 31.6 / 33.3, 72^3 58.2 / 63.2;
+    //     ternary FP64 32^3 23.0 / 22.3, but 48^3 48.5 / 49.8, 72^3 151.9 / 155.8;
+    //     binary FP32 48^3 11.6 / 12.0, 96^3 69.8 / 72.2.
+    //   bdist 1 FP64, whose forces spill: 16^3 84.9 / 77.6, ternary 110 / 102.
+    //   bdist 3 to 6: FP64 56^3 40.7 / 44.4 (4), 52.8 / 54.9 (5), 47.0 / 50.2 (6),
+    //     FP32 96^3 78.9 / 80.8 (4).
+    //   Lees-Edwards with bdist 0 or 4: FP32 32^3 22.8 / 22.2, 88^3 67.3 / 69.2; FP64
+    //     40^3 40.7 / 39.5, 72^3 102.2 / 103.4.
+    bool pulls_first() const
+    {
+        if (C == 3 && Dev) return false;
+        if (P.bdist == 2) return true;
+        if (le) return P.ns <= 120000u;
+        if (Dev) return false;
+        return P.bdist == 1 || (P.bdist == 0 && P.ns <= (C == 2 ? 120000u : 70000u));
+    }
+    // the kernels that this rule can ask for
+    static constexpr bool collide_exists(int c, bool lees, int bd, int mode)
+    {
+        if (mode == PULLS_FIRST) return bd == 2 ? c == 2 || !Dev : lees || !Dev;
+        if (mode == FORCES_FIRST) return bd != 2 || (c == 3 && Dev);
+        return true;
+    }
+    template <int CC, bool LE, int BD, bool ZH, int Mode>
+    void collide_k(const DevBufs &b, hipStream_t s)
+    {
+        if constexpr (collide_exists(CC, LE, BD, Mode))
+            k_collide<R, Dev, CC, LE, BD, false, ZH, Mode><<<tiles(), threads(), 0, s>>>(
+                P, (const R *)b.f[b.cur], LE ? (const R *)b.face_pc : nullptr, (const R *)b.aux,
+                LE ? (const R *)b.face_aux : nullptr, CC == 3 ? (const R *)b.db_alt : nullptr, (R *)b.f[1 - b.cur], xg,
+                nullptr, LE ? (R *)b.edge_pc : nullptr, LE && le_commit != LE_STATE_AS_IS ? b.le : nullptr,
+                LE ? le_commit : 0);
+    }
+    template <int BD, int Mode>
     void collide_bd(const DevBufs &b, hipStream_t s)
     {
-        const R *f = (const R *)b.f[b.cur];
-        R *fo = (R *)b.f[1 - b.cur];
-        if (P.zh && C == 3)
-            k_collide<R, Dev, 3, false, BD, false, true, NT><<<tiles(), threads(), 0, s>>>(
-                P, f, nullptr, (const R *)b.aux, nullptr, (const R *)b.db_alt, fo, xg, nullptr);
-        else if (P.zh && !le && !b.rock)
-            k_collide<R, Dev, 2, false, BD, false, true, NT><<<tiles(), threads(), 0, s>>>(
-                P, f, nullptr, (const R *)b.aux, nullptr, nullptr, fo, xg, nullptr);
+        if (b.rock)
+            k_collide<R, Dev, 2, false, BD, true><<<tiles(), threads(), 0, s>>>(
+                P, (const R *)b.f[b.cur], nullptr, (const R *)b.aux, nullptr, nullptr, (R *)b.f[1 - b.cur], xg, b.rock);
         else if (C == 3)
-            k_collide<R, Dev, 3, false, BD, false, false, NT><<<tiles(), threads(), 0, s>>>(
-                P, f, nullptr, (const R *)b.aux, nullptr, (const R *)b.db_alt, fo, xg, nullptr);
+            P.zh ? collide_k<3, false, BD, true, Mode>(b, s) : collide_k<3, false, BD, false, Mode>(b, s);
         else if (le)
-            k_collide<R, Dev, 2, true, BD, false, false, NT><<<tiles(), threads(), 0, s>>>(
-                P, f, (const R *)b.face_pc, (const R *)b.aux, (const R *)b.face_aux, nullptr, fo, xg, nullptr,
-                (R *)b.edge_pc, le_commit == LE_STATE_AS_IS ? nullptr : b.le, le_commit);
-        else if (b.rock)
-            k_collide<R, Dev, 2, false, BD, true><<<tiles(), threads(), 0, s>>>(P, f, nullptr, (const R *)b.aux,
-                                                                            nullptr, nullptr, fo, xg, b.rock);
+            collide_k<2, true, BD, false, Mode>(b, s);
         else
-            k_collide<R, Dev, 2, false, BD, false, false, NT><<<tiles(), threads(), 0, s>>>(
-                P, f, nullptr, (const R *)b.aux, nullptr, nullptr, fo, xg, nullptr);
+            P.zh ? collide_k<2, false, BD, true, Mode>(b, s) : collide_k<2, false, BD, false, Mode>(b, s);
     }
     // the non-temporal form once one copy of the populations exceeds the
     // memory-side cache
     bool nt() const { return (uint64_t)C * 19u * P.ns * sizeof(R) > MALL_BYTES; }
+    template <int BD>
+    void collide_form(const DevBufs &b, hipStream_t s)
+    {
+        if (nt())
+            collide_bd<BD, NON_TEMPORAL>(b, s);
+        else
+            pulls_first() ? collide_bd<BD, PULLS_FIRST>(b, s) : collide_bd<BD, FORCES_FIRST>(b, s);
+    }
     void collide(const DevBufs &b, hipStream_t s) override
     {
-        const bool n = nt();
         if (P.bdist == 0)
-            n ? collide_bd<0, true>(b, s) : collide_bd<0, false>(b, s);
+            collide_form<0>(b, s);
         else if (P.bdist == 2)
-            n ? collide_bd<2, true>(b, s) : collide_bd<2, false>(b, s);
+            collide_form<2>(b, s);
         else
-            n ? collide_bd<BD_GENERAL, true>(b, s) : collide_bd<BD_GENERAL, false>(b, s);
+            collide_form<BD_GENERAL>(b, s);
     }
     void le_faces(const DevBufs &b, bool post, bool stream, hipStream_t s, int adv) override
     {

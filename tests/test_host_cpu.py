@@ -265,3 +265,41 @@ def test_tuner_keeps_the_untuned_plan_unless_another_is_faster(so, dims, kw, ker
         assert not any(l.startswith("steps: ") for l in g.autotune(2).splitlines())
         g.time_loop(1)
     """)
+
+
+FORCES_FIRST, PULLS_FIRST, NON_TEMPORAL = range(3)
+LE = dict(boundary=gpu.LB3D_BC_LEES_EDWARDS, shear_u=0.02)
+ZH = dict(inv_fluid=12)
+
+
+def test_order_of_the_collides_loads(so):
+    """Whether the two-pass collide pulls before its forces, by component count,
+    precision, equilibrium form, boundary and size."""
+    cases = []
+    for precision in (gpu.LB3D_FP64, gpu.LB3D_FP32_DEV):
+        fp64 = precision == gpu.LB3D_FP64
+        for bdist in range(7):
+            for ncomp, kw in ((2, {}), (2, ZH), (2, LE), (3, {}), (3, ZH)):
+                for n in (24, 41, 48, 56):
+                    if kw is LE and bdist != 2:
+                        first = n < 56
+                    elif bdist == 2:
+                        first = ncomp == 2 or fp64
+                    elif bdist == 1:
+                        first = fp64
+                    else:
+                        first = fp64 and bdist == 0 and (n < 56 if ncomp == 2 else n < 48)
+                    cases.append((n, dict(kw, ncomp=ncomp, bdist=bdist, precision=precision),
+                                  PULLS_FIRST if first else FORCES_FIRST))
+            cases.append((124, dict(ncomp=2, bdist=bdist, precision=precision), NON_TEMPORAL))
+    fakehip.run(so, f"""
+        for n, kw, mode in {cases}:
+            g = Lattice(n, n, n, **kw)
+            g.set_plan(0)
+            log()
+            g.time_loop(1)
+            name = [l.split()[1] for l in log() if "collide" in l]
+            # ..., Rock, Zou-He, mode, then the arguments
+            assert len(name) == 1 and name[0].split("EvNS")[0].endswith(f"Li{{mode}}EE"), (n, kw, name)
+            g.close()
+    """)

@@ -374,13 +374,13 @@ class LauncherT : public Launcher {
     //   bdist 1 FP64, whose forces spill: 16^3 84.9 / 77.6, ternary 110 / 102.
     //   bdist 3 to 6: FP64 56^3 40.7 / 44.4 (4), 52.8 / 54.9 (5), 47.0 / 50.2 (6),
     //     FP32 96^3 78.9 / 80.8 (4).
-    //   Lees-Edwards with bdist 0 or 4: FP32 32^3 22.8 / 22.2, 88^3 67.3 / 69.2; FP64
-    //     40^3 40.7 / 39.5, 72^3 102.2 / 103.4.
+    //   Lees-Edwards with bdist 0 or 4: FP32 32^3 22.8 / 22.2, 64^3 37.9 / 37.2, 88^3
+    //     67.3 / 69.2; FP64 40^3 62.4 / 60.4 (4), 512x64x16 124.7 / 121.9 (0).
     bool pulls_first() const
     {
         if (C == 3 && Dev) return false;
         if (P.bdist == 2) return true;
-        if (le) return P.ns <= 120000u;
+        if (le) return !Dev || P.ns <= 300000u;
         if (Dev) return false;
         return P.bdist == 1 || (P.bdist == 0 && P.ns <= (C == 2 ? 120000u : 70000u));
     }
@@ -388,7 +388,7 @@ class LauncherT : public Launcher {
     static constexpr bool collide_exists(int c, bool lees, int bd, int mode)
     {
         if (mode == PULLS_FIRST) return bd == 2 ? c == 2 || !Dev : lees || !Dev;
-        if (mode == FORCES_FIRST) return bd != 2 || (c == 3 && Dev);
+        if (mode == FORCES_FIRST) return bd == 2 ? c == 3 && Dev : !lees || Dev;
         return true;
     }
     template <int CC, bool LE, int BD, bool ZH, int Mode>

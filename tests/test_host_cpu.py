@@ -280,9 +280,9 @@ def test_order_of_the_collides_loads(so):
         fp64 = precision == gpu.LB3D_FP64
         for bdist in range(7):
             for ncomp, kw in ((2, {}), (2, ZH), (2, LE), (3, {}), (3, ZH)):
-                for n in (24, 41, 48, 56):
+                for n in (24, 41, 48, 56, 72):
                     if kw is LE and bdist != 2:
-                        first = n < 56
+                        first = fp64 or n < 72
                     elif bdist == 2:
                         first = ncomp == 2 or fp64
                     elif bdist == 1:

@@ -8,7 +8,7 @@ default_rng(1)), g_br uniform in [0.06, 0.12], g_bs = -0.006, g_ss = -0.003,
 tau = tau_d = 1, beta = 10, d_0 = 1, bdist 2, densities 0.7 + U(-0.01, 0.01)
 for red and blue, 0.7 surfactant, dipoles uniform on the sphere (noise seed
 1000 + k), FP32 deviation storage, all lattices advanced together by the
-tuner's plan with graph-replayed steps.  The timed region is `--steps` whole
+tuner's plan.  The timed region is `--steps` whole
 steps with every lattice resident in HBM, bracketed by stream
 synchronisation; `value` is its MLUPS (sum of lattice sites x steps / wall
 time).  Beside it: the 48 lattices run one after another on the plain FP64
@@ -888,7 +888,7 @@ def main():
     dom = max(r["phases_ms"], key=r["phases_ms"].get)
     roofline = dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                     frac=round(achieved / HBM_PEAK_GBS, 4), traffic=None,
-                    kernel=(f"one graph-replayed step of the ensemble on the tuner's plan ({r['plan']}): "
+                    kernel=(f"one step of the ensemble on the tuner's plan ({r['plan']}): "
                             f"{', '.join(names.values())}"),
                     algorithmic_bytes_per_launch=B * sites,
                     algorithmic_bytes_note=f"{B} B per site update (3 x 19 FP32 populations and the 3-vector "
@@ -1009,7 +1009,7 @@ def main():
         "config": {"workload": "batched ternary ensemble: 48 periodic D3Q19 lattices, cube edges uniform in "
                                "{16,...,96} (seed 1), g_br uniform in [0.06,0.12], g_bs=-0.006, g_ss=-0.003, "
                                "tau=tau_d=1, beta=10, bdist=2, rho=0.7+-0.01, dipoles on the sphere (seeds 1000+k), "
-                               "FP32 deviation storage, one batch, graph-replayed steps, tuned plan",
+                               "FP32 deviation storage, one batch, tuned plan",
                    "lattices": ens["lattices"], "sites": sites, "edges": ens["edges"], "components": 3,
                    "bytes_per_site": B, "plan": r["plan"]},
         "roofline": roofline,
@@ -1018,8 +1018,8 @@ def main():
         "fp64_plain": dict(fp64s, workload="the same 48 lattices run one after another on the plain FP64 path"),
         "speedup_fp32_batched_vs_fp64_plain": round(r["mlups"] / fp64s["value"], 3),
         "phases_ms": r["phases_ms"],
-        "phases_note": ("HIP events around each launch over 3 steps launched one by one after the timed loop "
-                        "(not graph-replayed); roofline.mean_launch_ms is the timed loop's per-step time"),
+        "phases_note": ("HIP events around each launch over 3 steps after the timed loop, which has none "
+                        "between its launches; roofline.mean_launch_ms is the timed loop's per-step time"),
         "binary_256": binary,
         "lees_edwards_256x64x64": le,
         "accuracy_fp32_vs_fp64": accuracy,

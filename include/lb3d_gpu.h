@@ -143,8 +143,9 @@ int lb3d_gpu_advection(lb3d_ctx *ctx);                           /* code/lb3d_ad
 int lb3d_gpu_collision(lb3d_ctx *ctx);                           /* code/lb3d_collision.F90:41-291 */
 
 /* nsteps whole timesteps nt+1 .. nt+nsteps (the body of lb3d_time_loop,
- * code/lb3d_time_loop.F90:58-92); a long run replays them from a captured HIP
- * graph. */
+ * code/lb3d_time_loop.F90:58-92).  A call that begins after 1024 steps on one
+ * plan replays them from a captured HIP graph, and so does one of at least 2048
+ * steps on a lattice of at most 40,000 sites. */
 int lb3d_gpu_run_steps(lb3d_ctx *ctx, int32_t nsteps);
 /* Timing support (not a reference routine): lb3d_gpu_run_steps between two
  * HIP events recorded on the context's stream; *ms is the elapsed time

@@ -296,10 +296,21 @@ class LauncherT : public Launcher {
     // grid of the stepping kernels: whole XCD rounds (xcd_tile order)
     unsigned tiles() const { return xcd_round((P.ns + threads() - 1) / threads()); }
     // Their work-groups: one wave on lattices that leave CUs idle or uneven
-    // otherwise (32^3 is 128 groups of 256).  Step, groups of 256 -> 64 (us):
-    // binary FP32 16^3 8.4 -> 7.1, 32^3 8.3 -> 7.7, FP64 16^3 11.3 -> 9.2, 32^3
-    // 12.2 -> 10.7, 48^3 18.9 -> 18.0; ternary FP32 24^3 17.5 -> 14.8, FP64 32^3
-    // 23.4 -> 20.7, 48^3 42.1 -> 41.3; ternary FP64 64^3 84 -> 87.
+    // otherwise (32^3 is 128 groups of 256).  Two-pass step,
+    // groups of 256 / of 64 (us), at 16^3, 32^3, 48^3, then 56^3 and 64^3:
+    //   binary FP32       7.4/6.1   7.7/7.2   11.0/10.9   14.7/14.7   20.9/21.0
+    //   binary FP64       9.7/7.3  10.9/9.1   18.6/17.8   29.3/28.8   40.0/39.9
+    //   walls FP32        9.7/8.3  10.0/9.1   13.6/13.7   17.7/17.7   24.5/25.5
+    //   walls FP64       11.4/8.9  12.2/10.4  23.5/23.0   34.0/33.1   46.1/46.8
+    //   Zou-He FP64      10.3/7.7  11.4/9.5   18.9/18.0   30.3/30.1   42.0/41.8
+    //   Lees-Edwards FP32 18.9/18.3 20.4/20.0 24.8/24.8   28.7/28.5   33.8/33.9
+    //   Lees-Edwards FP64 24.3/22.9 27.0/25.7 38.9/37.9   47.7/47.2   58.9/59.3
+    //   ternary FP32     13.2/12.0 15.4/13.9  23.2/22.9   32.0/32.5   42.5/42.7
+    //   ternary FP64     19.5/16.1 23.0/20.4  42.0/41.2   59.9/59.4   82.4/84.1
+    //   ternary Zou-He FP64 19.7/14.9 23.0/19.3 39.1/38.3 55.9/56.7   81.6/82.5
+    // Up to 48^3 the small groups are nowhere slower by more than 1%; from 56^3 on
+    // either may be, by up to 4%.  (Between, at 52^3, they still win: binary FP64
+    // 26.3/23.5, walls 31.4/29.8, ternary FP64 56.3/53.3.)
     unsigned threads() const { return P.ns <= 120000u ? 64u : BLOCK; }
     unsigned diag_blocks() const override { return blocks(); }
     size_t real_bytes() const override { return sizeof(R); }

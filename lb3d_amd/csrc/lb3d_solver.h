@@ -119,7 +119,8 @@ class Launcher {
     virtual size_t real_bytes() const = 0;
 };
 
-// Tile shapes of k_fused2 that are instantiated (TX, TY).
+// Tile shapes (TX, TY) that a plan can be set to: k_fused3 has an instance of
+// each that fits, k_fused2 takes its tile at run time.
 constexpr int FUSED_SHAPES[][2] = {{64, 4}, {32, 8}, {64, 8}, {32, 16}, {128, 4}, {32, 4}, {16, 16},
                                    {128, 2}, {256, 2}};
 constexpr int N_FUSED_SHAPES = sizeof(FUSED_SHAPES) / sizeof(FUSED_SHAPES[0]);

@@ -635,8 +635,8 @@ end module lb3d_sanity_module
 
 !------------------------------------------------------------------------------
 !> lb3d_time_loop (code/lb3d_time_loop.F90:42-97): the same stages per step.
-!> With fast_loop the steps between two I/O or sanity points are replayed
-!> from the library's captured HIP graph instead of stage by stage.
+!> With fast_loop the steps between two I/O or sanity points are one call of
+!> the library instead of stage by stage.
 module lb3d_time_loop_module
   use lb3d_host_config
   use lb3d_host_state

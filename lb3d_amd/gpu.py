@@ -359,7 +359,7 @@ class Lattice:
         self.collision()
 
     def time_loop(self, nsteps):
-        """nsteps timesteps (a long run replays a captured HIP graph)."""
+        """nsteps timesteps (a long run replays a captured HIP graph; see lb3d_gpu_run_steps)."""
         check(lib().lb3d_gpu_run_steps(self._h, int(nsteps)), "run_steps")
 
     def time_loop_timed(self, nsteps):

@@ -22,8 +22,10 @@ using namespace lb3d;
 #define BTRY(expr)                                                                          \
     do {                                                                                    \
         hipError_t e_ = (expr);                                                             \
-        if (e_ != hipSuccess)                                                               \
+        if (e_ != hipSuccess) {                                                             \
+            (void)hipGetLastError(); /* reported here, not by the next call */              \
             return set_error(LB3D_EHIP, (std::string(#expr) + ": " + hipGetErrorString(e_)).c_str()); \
+        }                                                                                   \
     } while (0)
 
 struct lb3d_batch {

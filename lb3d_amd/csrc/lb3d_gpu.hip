@@ -32,8 +32,10 @@ int fail(int code, const std::string &msg)
 #define HIP_TRY(expr)                                                                     \
     do {                                                                                  \
         hipError_t e_ = (expr);                                                           \
-        if (e_ != hipSuccess)                                                             \
+        if (e_ != hipSuccess) {                                                           \
+            (void)hipGetLastError(); /* reported here, not by the next call */            \
             return fail(LB3D_EHIP, std::string(#expr) + ": " + hipGetErrorString(e_));   \
+        }                                                                                 \
     } while (0)
 
 enum StageState { IDLE = 0, AFTER_BC6 = 1, AFTER_ADV = 2, AFTER_BC8 = 3 };

@@ -320,6 +320,7 @@ struct HostIO {
         const size_t n = (total + piece - 1) / piece;
         auto len = [&](size_t k) { return total - k * piece < piece ? total - k * piece : piece; };
         auto start = [&](size_t k) {
+            (void)hipGetLastError();  // (an error that an earlier call left is not go's)
             const void *src = go(k * piece, len(k), dev[k & 1]);
             hipError_t r = hipGetLastError();
             if (r == hipSuccess) r = hipMemcpyAsync(pin[k & 1], src, len(k), hipMemcpyDeviceToHost, st);
@@ -352,8 +353,10 @@ struct HostIO {
             crew.copy(pin[k & 1], (const char *)src + off, n);
             e = hipMemcpyAsync(dev[k & 1], pin[k & 1], n, hipMemcpyHostToDevice, st);
             if (e == hipSuccess) e = hipEventRecord(ev[k & 1], st);
-            if (e == hipSuccess) go(off, n, dev[k & 1]);
-            if (e == hipSuccess) e = hipGetLastError();
+            if (e != hipSuccess) break;
+            (void)hipGetLastError();
+            go(off, n, dev[k & 1]);
+            e = hipGetLastError();
         }
         if (e != hipSuccess) (void)hipStreamSynchronize(st);
         return e;

@@ -303,3 +303,17 @@ def test_order_of_the_collides_loads(so):
             assert len(name) == 1 and name[0].split("EvNS")[0].endswith(f"Li{{mode}}EE"), (n, kw, name)
             g.close()
     """)
+
+
+def test_a_pending_error_of_the_caller_does_not_fail_transfers(so):
+    """An error that an earlier call of the program left behind in the runtime
+    is not the transfer's."""
+    fakehip.run(so, """
+        for precision in (0, 1):
+            g = Lattice(12, 10, 8, ncomp=2, precision=precision)
+            batch = Batch([(8, 6, 6)], ncomp=2, precision=precision)
+            for call in (g.populations, g.density, g.momentum, g.download_sites, lambda: batch.populations(0),
+                         lambda: g.upload_sites(np.zeros((10, 12, 14, 49)))):
+                assert fake.hipSetDevice(7) != 0
+                call()
+    """)

@@ -596,11 +596,20 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
     const RecLayout L = rec_layout(p, h, sd);
     // the mask goes to the aux field, which holds nothing after an upload, and
     // from there to its own memory if there are rock sites
-    uint8_t *mask = nullptr;
-    if (walls_ok) {
-        mask = (uint8_t *)c->b.aux;
-        c->moments = MOMENTS_NONE;
-    }
+    uint8_t *mask = walls_ok ? (uint8_t *)c->b.aux : nullptr;
+    // where the upload fails after that, the moments of the last advection are
+    // gone, and a two-pass step under way gets its own again
+    struct Lost {
+        lb3d_ctx *c;
+        bool armed = false;
+        ~Lost()
+        {
+            if (!armed) return;
+            const bool under_way = !c->plan.fused && (c->state == AFTER_ADV || c->state == AFTER_BC8);
+            if (under_way) c->L->moments(c->b, c->stream);
+            c->moments = under_way && c->moments != MOMENTS_NONE ? MOMENTS_KEPT : MOMENTS_NONE;
+        }
+    } lost{c};
     IoLoan io;
     const PopBase pb = pop_base(p);
     const int to = 1 - c->b.cur;
@@ -611,6 +620,7 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
     HIP_TRY(hipMemsetAsync(io->count, 0, sizeof(uint32_t), c->stream));
     HIP_TRY(io->up(c->stream, N + skip * sd, (size_t)p.nz * plane * rec, lds, [&](size_t at, size_t len, void *buf) {
         const uint32_t n = (uint32_t)(len / rec), nb = (n + REC_SITES - 1) / REC_SITES;
+        lost.armed = walls_ok;
         auto go = [&](auto r) {
             using R = decltype(r);
             k_put_sites<R><<<nb, 256, lds, c->stream>>>((const double *)buf, L, pb, (uint32_t)(skip + at / rec), n,
@@ -619,8 +629,9 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
         is_dev(c) ? go(float()) : go(double());
     }));
     uint32_t nrock = 0;
-    HIP_TRY(hipMemcpyAsync(io->pin[0], io->count, sizeof nrock, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    const hipError_t counted = hipMemcpyAsync(io->pin[0], io->count, sizeof nrock, hipMemcpyDeviceToHost, c->stream);
+    HIP_TRY(hipStreamSynchronize(c->stream));  // (the loan ends with its buffers at rest)
+    HIP_TRY(counted);
     std::memcpy(&nrock, io->pin[0], sizeof nrock);
     if (nrock && !walls_ok) {
         if (p.ncomp != 2 || c->le)
@@ -631,6 +642,7 @@ int lb3d_gpu_upload_sites(lb3d_ctx *c, const double *N, int32_t h, int32_t sd, i
         if (!c->rock_dev) HIP_TRY(hipMalloc((void **)&c->rock_dev, L.ns));
         HIP_TRY(hipMemcpyAsync(c->rock_dev, mask, L.ns, hipMemcpyDeviceToDevice, c->stream));
     }
+    lost.armed = false;
     set_walls(c, nrock != 0);
     set_cur(c, to);
     c->nt = nt0;

@@ -20,6 +20,7 @@ static char *log_buf;
 static size_t log_len, log_cap;
 
 /* knobs and counters for the tests */
+int fake_fail_copy;                         /* the n-th copy from now on fails (0: none) */
 int fake_fail_pinned;                       /* 1: pinned allocations fail, 2: every second one */
 size_t fake_device_fill;                    /* device memory starts out as the doubles 0, 1, 2, ... */
 size_t fake_device_limit = (size_t)-1;      /* largest device allocation that succeeds */
@@ -143,6 +144,7 @@ static int on(const void *p, stream *s)
 int hipMemcpyAsync(void *d, const void *src, size_t n, int kind, stream *s)
 {
     (void)kind;
+    if (fake_fail_copy && --fake_fail_copy == 0) return fail(EINVALID);
     if (!on(d, s) || !on(src, s)) return fail(EINVALID);
     if (s && s->capturing) return fail(EINVALID);
     memmove(d, src, n);

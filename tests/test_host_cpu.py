@@ -317,3 +317,38 @@ def test_a_pending_error_of_the_caller_does_not_fail_transfers(so):
                 assert fake.hipSetDevice(7) != 0
                 call()
     """)
+
+
+@pytest.mark.parametrize("copy", [1, 2])
+def test_failed_upload_leaves_the_step_alone(so, copy):
+    """An upload that fails on its first or its last copy: before anything was
+    written the moments of the last advection are still there; after it a
+    two-pass step under way gets its moments again."""
+    fakehip.run(so, f"""
+        N = np.zeros((10, 12, 14, 49))
+        fail = knob("fake_fail_copy", ctypes.c_int)
+        for plan, calls in (((0,), 2), ((2, 32, 4, 4), 2), ((2, 32, 4, 4), 0)):
+            g = Lattice(12, 10, 8, ncomp=2)
+            g.set_plan(*plan)
+            g.init_noise(1)
+            g.time_loop(1)
+            if calls:
+                g.bc_apply(6, 2), g.advection()
+            log()
+            fail.value = {copy}
+            try:
+                g.upload_sites(N)
+            except LB3DError as e:
+                assert e.code == 2
+            else:
+                raise AssertionError("no error")
+            names = "".join(log())
+            assert ("put_sites" in names) == ({copy} == 2)
+            again = {copy} == 2 and plan == (0,)
+            assert ("k_moments" in names) == again, (plan, calls, names)
+            g.download_sites()
+            rebuilt = {copy} == 1 and plan != (0,)
+            assert any("k_moments" in l for l in log()) == rebuilt, (plan, calls)
+            if calls:
+                g.bc_apply(8, 2), g.collision()
+    """)

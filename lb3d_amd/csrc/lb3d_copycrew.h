@@ -15,9 +15,9 @@ namespace lb3d {
 // Copies between the caller's memory and pinned memory, by the calling thread
 // and, for large transfers, a few helpers that live for the transfer: one
 // thread writes fresh pages at 15 GB/s, a fourth of what PCIe brings.  A helper
-// without work looks for it for SPIN, somewhat longer than a piece of 8 MiB
-// takes to cross PCIe (0.15 ms), so that between two pieces it is there at
-// once; then it is parked, and leaves its processor alone while the caller
+// without work looks for it for SPIN, longer than a piece of 8 MiB takes to be
+// converted and to cross PCIe (0.2 ms), so that it is there at once for the
+// first piece and between two; then it is parked, and leaves its processor alone while the caller
 // waits for the device.
 class CopyCrew {
   public:
@@ -64,7 +64,7 @@ class CopyCrew {
 
   private:
     static constexpr int MAX_HELPERS = 3;
-    static constexpr std::chrono::microseconds SPIN{200};
+    static constexpr std::chrono::microseconds SPIN{500};
     void slice(int i) const
     {
         // whole pages per helper

